@@ -144,6 +144,63 @@ __device__ __forceinline__ uint64_t mul_mod52(uint64_t a, uint64_t b, const DevM
     mac52(acc, split26(a), b);
     return reduce52(acc, m);
 }
+
+// Products by constants modulo primes just below a power of two: q = 2^b - delta,
+// delta < 2^29 (every prime of a context is the largest free one of its bit size that
+// is 1 mod 2N, so delta is a small multiple of 2N). A constant w < q travels as
+// w = h0 2^s + l0 and 2^32 w mod q = h1 2^s + l1 with s = b - 30, so h < 2^30.
+// For x = xh 2^32 + xl (signed 64-bit, any value),
+//   x w = H 2^s + L (mod q),  H = xl h0 + xh h1,  L = xl l0 + xh l1,
+// and 2^(s + 32) = 2^(b + 2) = 4 delta (mod q), so
+//   x w = (H mod 2^32) 2^s + L + floor(H / 2^32) 4 delta (mod q):
+// six 32 x 32 -> 64-bit multiply-adds, no quotient and no carry handling (a Shoup
+// product with its 64-bit high part takes about twice the issue slots: every
+// multiply-add, 64-bit add and shift issues in 4 cycles per wave here).
+struct FoldMod {
+    uint32_t pw;    // 2^s
+    int32_t d4, d;  // 4 delta, delta
+    uint32_t sh;    // b - 32
+    uint32_t mask;  // 2^(b - 32) - 1
+    uint32_t s;     // b - 30
+    uint64_t off;   // the smallest multiple of q that is at least 2^63
+};
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // (h0, l0, h1, l1)
+
+// |result| <= 2.5 2^(b+2) + 6 2^30 delta for any signed x.
+__device__ __forceinline__ uint64_t fold_mul(uint64_t x, u32x4 w, const FoldMod &f) {
+    const uint32_t xl = (uint32_t)x;
+    const int32_t xh = (int32_t)(x >> 32);
+    const uint64_t H = (uint64_t)((int64_t)xh * (int32_t)w.z) + (uint64_t)xl * w.x;
+    const uint64_t L = (uint64_t)((int64_t)xh * (int32_t)w.w) + (uint64_t)xl * w.y;
+    const uint64_t r = (uint64_t)(uint32_t)H * f.pw + L;
+    return (uint64_t)((int64_t)(int32_t)(H >> 32) * f.d4) + r;
+}
+
+// x mod 2^b + floor(x / 2^b) delta: congruent to a signed x and within
+// (-2^(63-b) delta, 2^b + 2^(63-b) delta).
+__device__ __forceinline__ uint64_t fold_tight(uint64_t x, const FoldMod &f) {
+    const int32_t xh = (int32_t)(x >> 32);
+    const uint64_t lo = ((uint64_t)((uint32_t)xh & f.mask) << 32) | (uint32_t)x;
+    return (uint64_t)((int64_t)(xh >> f.sh) * f.d) + lo;
+}
+
+// Canonical residue of a signed x, |x| <= 2^63 - q: the offset makes it unsigned, and one
+// fold leaves it below 2^b + 2^(64-b) delta < 2q.
+__device__ __forceinline__ uint64_t fold_canon(uint64_t x, uint64_t q, const FoldMod &f) {
+    const uint64_t y = x + f.off;
+    const uint32_t yh = (uint32_t)(y >> 32);
+    const uint64_t lo = ((uint64_t)(yh & f.mask) << 32) | (uint32_t)y;
+    return csub((uint64_t)(yh >> f.sh) * (uint32_t)f.d + lo, q);
+}
+
+// The split form of a constant w < q given its Shoup companion.
+__device__ __forceinline__ u32x4 fold_split(uint64_t w, uint64_t ws, uint64_t q, const FoldMod &f) {
+    const uint64_t w1 = mul_shoup(uint64_t(1) << 32, w, ws, q);
+    const uint32_t m = f.pw - 1;
+    return u32x4{(uint32_t)(w >> f.s), (uint32_t)w & m, (uint32_t)(w1 >> f.s), (uint32_t)w1 & m};
+}
+
 // [v]_q of an integral double v with |v| < 2^128; negative v maps to q - (|v| mod q),
 // which is q itself when |v| is a multiple of q (callers reduce when they need [0, q)).
 __device__ __forceinline__ uint64_t residue_of_rounded(double v, const DevMod &m) {

@@ -108,6 +108,39 @@ uint64_t min_root_2n(uint64_t q, uint64_t two_n) {
     return best;
 }
 
+// The split form of prime q (FoldMod), and in *bound the largest |fold_mul|; false when
+// q has none: 36 to 58 bits, delta below 2^29, and one fold of an unsigned 64-bit word
+// leaves it below 2q.
+bool fold_form(uint64_t q, FoldMod *f, uint64_t *bound) {
+    int b = 0;
+    while (b < 64 && (q >> b)) b++;
+    if (b < 36 || b > 58) return false;
+    const uint64_t delta = (uint64_t(1) << b) - q;
+    if (delta >= (uint64_t(1) << 29) || (((hu128)delta << (64 - b)) + 2 * delta) >> b) return false;
+    f->s = (uint32_t)(b - 30);
+    f->pw = 1u << f->s;
+    f->d = (int32_t)delta;
+    f->d4 = (int32_t)(4 * delta);
+    f->sh = (uint32_t)(b - 32);
+    f->mask = (1u << f->sh) - 1;
+    f->off = ((uint64_t(1) << 63) + q - 1) / q * q;
+    *bound = (uint64_t(10) << b) + (delta << 32) + (delta << 31);  // 2.5 2^(b+2) + 6 2^30 delta
+    return true;
+}
+
+// Split forms of a twiddle table: row p of `out` from row p of `tw` (one thread per
+// twiddle; primes without a split form, pw = 0, are skipped).
+__global__ void k_split_twiddles(const uint64_t *__restrict__ tw, const DevMod *__restrict__ mods,
+                                 const FoldMod *__restrict__ fold, u32x4 *__restrict__ out, size_t N) {
+    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    const uint32_t p = blockIdx.y;
+    const FoldMod f = fold[p];
+    if (i >= N || f.pw == 0) return;
+    const uint64_t w = tw[(size_t)p * N + i], w1 = mul_mod(w, uint64_t(1) << 32, mods[p]);
+    const uint32_t m = f.pw - 1;
+    out[(size_t)p * N + i] = u32x4{(uint32_t)(w >> f.s), (uint32_t)w & m, (uint32_t)(w1 >> f.s), (uint32_t)w1 & m};
+}
+
 template <class T>
 void upload(DevBuf &b, const std::vector<T> &v) {
     b.alloc(std::max<size_t>(v.size() * sizeof(T), 8));
@@ -372,6 +405,19 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
     upload(c->itw_s, itws);
     upload(c->ninv, ninv);
     upload(c->ninv_s, ninvs);
+    std::vector<FoldMod> fold(QP, FoldMod{});
+    c->fold_bound.assign(QP, 0);
+    bool any_fold = false;
+    for (size_t p = 0; p < QP; p++) any_fold = fold_form(c->q[p], &fold[p], &c->fold_bound[p]) || any_fold;
+    upload(c->d_fold, fold);
+    if (any_fold) {
+        c->tw_f.alloc(QP * N * sizeof(u32x4));
+        c->itw_f.alloc(QP * N * sizeof(u32x4));
+        const dim3 grid((unsigned)((N + 255) / 256), (unsigned)QP);
+        k_split_twiddles<<<grid, 256>>>(c->tw.as<uint64_t>(), c->mods(), c->d_fold.as<FoldMod>(), c->tw_f.as<u32x4>(), N);
+        k_split_twiddles<<<grid, 256>>>(c->itw.as<uint64_t>(), c->mods(), c->d_fold.as<FoldMod>(), c->itw_f.as<u32x4>(), N);
+        SHM_HIP(hipGetLastError());
+    }
 
     // ModDown constants (rns.cu:95-128, 187-190): P mod q_i, P^-1 mod q_i,
     // (P/p_j)^-1 mod p_j, (P/p_j) mod q_i.

@@ -144,6 +144,11 @@ struct Context {
     DevBuf tw, tw_s;        // [QP][N]
     DevBuf itw, itw_s;      // [QP][N]
     DevBuf ninv, ninv_s;    // [QP]
+    // split forms of the twiddles for primes just below a power of two (FoldMod):
+    // u32x4[QP][N], and FoldMod[QP]; fold_bound[p] is the largest |fold_mul| of prime
+    // p, 0 when it has no split form
+    DevBuf tw_f, itw_f, d_fold;
+    std::vector<uint64_t> fold_bound;
     DevBuf pinv, pinv_s;    // P^-1 mod q_i, i < nQ
     DevBuf pmod, pmod_s;    // P mod q_i, i < nQ
     DevBuf phat_inv, phat_inv_s;  // [nP] (P/p_j)^-1 mod p_j

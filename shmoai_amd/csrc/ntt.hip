@@ -15,11 +15,15 @@
 // units). A sub-transform whose first-stage group id is G uses twiddle
 // tw[(G << u) + i'] at its local stage u for local group i'.
 //
-// Lazy ranges (Harvey): forward keeps [0, 4q) between stages, inverse [0, 2q);
-// primes are < 2^61 so nothing wraps. When every prime of a launch is below
-// 2^64 / (5 + 4 log N) (about 2^57.9) the forward stages skip the per-butterfly
-// reduction of a altogether and take a cheaper quotient in the twiddle product
-// (values stay below (4 + 4 log N) q). Outputs are canonical residues.
+// Butterfly arithmetic, by the primes of a launch (launch_ntt):
+//   - primes with a split form (FoldMod, arith.h), i.e. all of 36 to 58 bits just below a
+//     power of two: signed unreduced words, nine issue slots a butterfly. The tile pass of
+//     64 x 24 limbs at N = 2^16 issues 734 VALU instructions per wave instead of 1325 (the
+//     unreduced Shoup form): 548 -> 393 us forward, 646 -> 393 us inverse;
+//   - otherwise, forward and below 2^64 / (5 + 4 log N) (about 2^57.9): unreduced Shoup
+//     butterflies with a cheaper quotient (values below (4 + 4 log N) q);
+//   - otherwise Harvey's lazy ranges: [0, 4q) forward, [0, 2q) inverse (primes < 2^61).
+// Outputs are canonical residues, the same words in every form.
 #include <algorithm>
 
 #include <mutex>
@@ -67,21 +71,48 @@ __device__ __forceinline__ const __attribute__((address_space(1))) V *global_ptr
     return (const __attribute__((address_space(1))) V *)p;
 }
 
-// Per-prime constant as the butterflies see it.
-struct IntK {
-    uint64_t q;
-};
-
 // Twiddle and constant tables of one launch (forward or inverse set).
 struct NttTables {
     const DevMod *mods;
     const uint64_t *tw, *tws;   // twiddles and their Shoup quotients
     const uint64_t *ninv, *ninv_s;
+    const u32x4 *twf;           // split twiddles and prime constants (primes with a split form)
+    const FoldMod *fold;
 };
 
+// Butterfly arithmetic of a launch, chosen by its primes (launch_ntt):
+//   HARVEY : any prime below 2^61; forward keeps [0, 4q), inverse [0, 2q).
+//   LAZY   : forward, (5 + 4 log N) q < 2^64; a stays unreduced (below).
+//   FOLD   : every prime has a split form (FoldMod) and log N fold_mul results fit a
+//            signed word; words are signed and unreduced.
+enum { HARVEY = 0, LAZY = 1, FOLD = 2 };
+
+// One prime's tables in the form its butterflies read them.
+struct HarveyK {
+    const uint64_t *__restrict__ tw, *__restrict__ tws;
+    uint64_t q;
+};
+struct LazyK {
+    const uint64_t *__restrict__ tw, *__restrict__ tws;
+    uint64_t q;
+};
+struct FoldK {
+    const u32x4 *__restrict__ tw;
+    FoldMod f;
+};
+
+template <int A>
+__device__ __forceinline__ auto arith_of(const NttTables &tb, uint32_t prime, size_t N) {
+    if constexpr (A == FOLD)
+        return FoldK{tb.twf + (size_t)prime * N, tb.fold[prime]};
+    else if constexpr (A == LAZY)
+        return LazyK{tb.tw + (size_t)prime * N, tb.tws + (size_t)prime * N, tb.mods[prime].q};
+    else
+        return HarveyK{tb.tw + (size_t)prime * N, tb.tws + (size_t)prime * N, tb.mods[prime].q};
+}
+
 template <int R>
-__device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const uint64_t *__restrict__ tw,
-                                        const uint64_t *__restrict__ tws, IntK k) {
+__device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const HarveyK &k) {
     const uint64_t q = k.q, q2 = q << 1;
 #pragma unroll
     for (int u = 0; u < R; u++) {
@@ -90,7 +121,7 @@ __device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const uint64_t 
         for (int l = 0; l < (1 << R); l++) {
             if ((l & h) == 0) {
                 const uint32_t ti = (G << u) + (uint32_t)(l >> (R - u));
-                const uint64_t w = tw[ti], ws = tws[ti];
+                const uint64_t w = k.tw[ti], ws = k.tws[ti];
                 uint64_t a = x[l];
                 a = a >= q2 ? a - q2 : a;
                 const uint64_t t = mul_shoup_lazy(x[l + h], w, ws, q);
@@ -106,13 +137,8 @@ __device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const uint64_t 
 // a + 4q, so log N stages from inputs below 4q end below (4 + 4 log N) q, which fits
 // 64 bits for the primes the launcher allows here. Saves the compare-select-subtract
 // of every butterfly and part of the quotient's multiplies; the final pass reduces once.
-struct IntKLazy {
-    uint64_t q;
-};
-
 template <int R>
-__device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const uint64_t *__restrict__ tw,
-                                        const uint64_t *__restrict__ tws, IntKLazy k) {
+__device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const LazyK &k) {
     const uint64_t q = k.q, q4 = q << 2;
 #pragma unroll
     for (int u = 0; u < R; u++) {
@@ -122,7 +148,7 @@ __device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const uint64_t 
             if ((l & h) == 0) {
                 const uint32_t ti = (G << u) + (uint32_t)(l >> (R - u));
                 const uint64_t a = x[l];
-                const uint64_t t = mul_shoup_lazy4(x[l + h], tw[ti], tws[ti], q);
+                const uint64_t t = mul_shoup_lazy4(x[l + h], k.tw[ti], k.tws[ti], q);
                 x[l] = a + t;
                 x[l + h] = a + q4 - t;
             }
@@ -130,18 +156,28 @@ __device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const uint64_t 
     }
 }
 
+// Signed forward butterflies (a + t, a - t) with t = fold_mul(x, w), |t| <= R: log N
+// stages add at most log N R to the input's bound, which the launcher checks against
+// 2^63. Nine multiply-add or 64-bit add slots a butterfly where the Shoup form issued 26.
 template <int R>
-__device__ __forceinline__ void gs_unit(uint64_t *x, uint32_t G, const uint64_t *__restrict__ tw,
-                                        const uint64_t *__restrict__ tws, IntK k);
-template <int R>
-__device__ __forceinline__ void gs_unit(uint64_t *x, uint32_t G, const uint64_t *__restrict__ tw,
-                                        const uint64_t *__restrict__ tws, IntKLazy k) {
-    gs_unit<R>(x, G, tw, tws, IntK{k.q});  // the inverse keeps its reductions
+__device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const FoldK &k) {
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+        const int h = 1 << (R - 1 - u);
+#pragma unroll
+        for (int l = 0; l < (1 << R); l++) {
+            if ((l & h) == 0) {
+                const uint64_t a = x[l];
+                const uint64_t t = fold_mul(x[l + h], k.tw[(G << u) + (uint32_t)(l >> (R - u))], k.f);
+                x[l] = a + t;
+                x[l + h] = a - t;
+            }
+        }
+    }
 }
 
 template <int R>
-__device__ __forceinline__ void gs_unit(uint64_t *x, uint32_t G, const uint64_t *__restrict__ tw,
-                                        const uint64_t *__restrict__ tws, IntK k) {
+__device__ __forceinline__ void gs_unit(uint64_t *x, uint32_t G, const HarveyK &k) {
     const uint64_t q = k.q, q2 = q << 1;
 #pragma unroll
     for (int u = R - 1; u >= 0; u--) {
@@ -150,12 +186,31 @@ __device__ __forceinline__ void gs_unit(uint64_t *x, uint32_t G, const uint64_t 
         for (int l = 0; l < (1 << R); l++) {
             if ((l & h) == 0) {
                 const uint32_t ti = (G << u) + (uint32_t)(l >> (R - u));
-                const uint64_t w = tw[ti], ws = tws[ti];
+                const uint64_t w = k.tw[ti], ws = k.tws[ti];
                 const uint64_t a = x[l], b = x[l + h];
                 uint64_t s = a + b;
                 s = s >= q2 ? s - q2 : s;
                 x[l] = s;
                 x[l + h] = mul_shoup_lazy(a + q2 - b, w, ws, q);
+            }
+        }
+    }
+}
+
+// Signed inverse butterflies (a + b, (a - b) w). A unit's inputs are within the bound R of
+// fold_mul, sums double per stage (2^(R-1) R before the last product: below 2^63 is
+// checked by the launcher), and the sums of the unit's last stage are folded to b bits.
+template <int R>
+__device__ __forceinline__ void gs_unit(uint64_t *x, uint32_t G, const FoldK &k) {
+#pragma unroll
+    for (int u = R - 1; u >= 0; u--) {
+        const int h = 1 << (R - 1 - u);
+#pragma unroll
+        for (int l = 0; l < (1 << R); l++) {
+            if ((l & h) == 0) {
+                const uint64_t a = x[l], b = x[l + h];
+                x[l] = u == 0 ? fold_tight(a + b, k.f) : a + b;
+                x[l + h] = fold_mul(a - b, k.tw[(G << u) + (uint32_t)(l >> (R - u))], k.f);
             }
         }
     }
@@ -190,9 +245,9 @@ __host__ __device__ constexpr int round_start(int logt, int r, int maxr) {
 // One round over the LDS tile: SUBS independent sub-transforms of size 2^LOGT
 // (row stride TP words). Sub-transform `sub` has first-stage group id
 // gbase(sub) at local stage 0.
-template <int LOGT, int R, bool FWD, int NT, typename E, typename K>
-__device__ __forceinline__ void lds_round(E *lds, int s0, uint32_t gmul, uint32_t gadd_step, uint32_t gadd0,
-                                          const E *__restrict__ tw, const E *__restrict__ tws, K k) {
+template <int LOGT, int R, bool FWD, int NT, typename K>
+__device__ __forceinline__ void lds_round(uint64_t *lds, int s0, uint32_t gmul, uint32_t gadd_step, uint32_t gadd0,
+                                          const K &k) {
     constexpr int T = 1 << LOGT;
     constexpr int SUBS = kTile / T;
     constexpr int TP = row_stride<T>();
@@ -209,15 +264,15 @@ __device__ __forceinline__ void lds_round(E *lds, int s0, uint32_t gmul, uint32_
         // one sub-transform of at least 64 units: the 64 lanes of a wave share kk,
         // so G is wave-uniform and the twiddles come through scalar loads
         if (SUBS == 1 && ups >= 64) G = __builtin_amdgcn_readfirstlane(G);
-        E *row = lds + sub * TP;
+        uint64_t *row = lds + sub * TP;
         const int i0 = kk * T0 + o;
-        E x[1 << R];
+        uint64_t x[1 << R];
 #pragma unroll
         for (int l = 0; l < (1 << R); l++) x[l] = row[swz<T>(i0 + l * ups)];
-        if (FWD)
-            ct_unit<R>(x, G, tw, tws, k);
+        if constexpr (FWD)
+            ct_unit<R>(x, G, k);
         else
-            gs_unit<R>(x, G, tw, tws, k);
+            gs_unit<R>(x, G, k);
 #pragma unroll
         for (int l = 0; l < (1 << R); l++) row[swz<T>(i0 + l * ups)] = x[l];
     }
@@ -228,21 +283,21 @@ struct NoHook {
 };
 
 // before_last runs (forward only) just before the last round
-template <int LOGT, bool FWD, int NT, typename E, typename K, typename H = NoHook>
-__device__ __forceinline__ void run_rounds(E *lds, uint32_t gmul, uint32_t gadd_step, uint32_t gadd0, const E *tw,
-                                           const E *tws, K k, H before_last = H{}) {
+template <int LOGT, bool FWD, int NT, typename K, typename H = NoHook>
+__device__ __forceinline__ void run_rounds(uint64_t *lds, uint32_t gmul, uint32_t gadd_step, uint32_t gadd0,
+                                           const K &k, H before_last = H{}) {
     constexpr int MAXR = NT >= 512 ? 3 : 4;
     constexpr int NR = n_rounds(LOGT, MAXR);
-    if (FWD) {
+    if constexpr (FWD) {
 #pragma unroll
         for (int r = 0; r < NR; r++) {
             const int R = round_len(LOGT, r, MAXR), s0 = round_start(LOGT, r, MAXR);
             if (r == NR - 1) before_last();
             switch (R) {
-                case 4: lds_round<LOGT, 4, true, NT>(lds, s0, gmul, gadd_step, gadd0, tw, tws, k); break;
-                case 3: lds_round<LOGT, 3, true, NT>(lds, s0, gmul, gadd_step, gadd0, tw, tws, k); break;
-                case 2: lds_round<LOGT, 2, true, NT>(lds, s0, gmul, gadd_step, gadd0, tw, tws, k); break;
-                default: lds_round<LOGT, 1, true, NT>(lds, s0, gmul, gadd_step, gadd0, tw, tws, k); break;
+                case 4: lds_round<LOGT, 4, true, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
+                case 3: lds_round<LOGT, 3, true, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
+                case 2: lds_round<LOGT, 2, true, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
+                default: lds_round<LOGT, 1, true, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
             }
             __syncthreads();
         }
@@ -251,10 +306,10 @@ __device__ __forceinline__ void run_rounds(E *lds, uint32_t gmul, uint32_t gadd_
         for (int r = NR - 1; r >= 0; r--) {
             const int R = round_len(LOGT, r, MAXR), s0 = round_start(LOGT, r, MAXR);
             switch (R) {
-                case 4: lds_round<LOGT, 4, false, NT>(lds, s0, gmul, gadd_step, gadd0, tw, tws, k); break;
-                case 3: lds_round<LOGT, 3, false, NT>(lds, s0, gmul, gadd_step, gadd0, tw, tws, k); break;
-                case 2: lds_round<LOGT, 2, false, NT>(lds, s0, gmul, gadd_step, gadd0, tw, tws, k); break;
-                default: lds_round<LOGT, 1, false, NT>(lds, s0, gmul, gadd_step, gadd0, tw, tws, k); break;
+                case 4: lds_round<LOGT, 4, false, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
+                case 3: lds_round<LOGT, 3, false, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
+                case 2: lds_round<LOGT, 2, false, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
+                default: lds_round<LOGT, 1, false, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
             }
             __syncthreads();
         }
@@ -308,7 +363,7 @@ struct NttIO {
 // !FWD: inverse stages logN1-1..0, then x N^-1, output canonical.
 // At most 80 VGPRs (6 waves per SIMD): the inverse form would otherwise take 99. The
 // encoder's form keeps its registers (it would spill).
-template <int LOGT, bool FWD, int IO, bool LAZY>
+template <int LOGT, bool FWD, int IO, int A>
 __global__ __launch_bounds__(kThreads, IO == IO_ENCODE ? 1 : 6) void k_ntt_cols(uint64_t *__restrict__ data, LimbMap mp, NttTables tb,
                                                        int logN, NttIO io) {
     constexpr int T = 1 << LOGT;
@@ -330,6 +385,10 @@ __global__ __launch_bounds__(kThreads, IO == IO_ENCODE ? 1 : 6) void k_ntt_cols(
 #pragma unroll
             for (int r = 0; r < T; r++) {
                 const uint64_t v = src[r * N2];
+                if (A == FOLD) {  // signed words need no reduction
+                    x[r] = io.center && v > io.center ? v - (2 * io.center + 1) : v;
+                    continue;
+                }
                 uint64_t y = reduce64(v, m);
                 if (io.center && v > io.center) y = sub_mod(y, reduce64(2 * io.center + 1, m), m.q);
                 x[r] = y;
@@ -349,20 +408,24 @@ __global__ __launch_bounds__(kThreads, IO == IO_ENCODE ? 1 : 6) void k_ntt_cols(
 #pragma unroll
             for (int r = 0; r < T; r++) x[r] = base[r * N2];
         }
-        const uint64_t *tw = tb.tw + (size_t)prime * N, *tws = tb.tws + (size_t)prime * N;
-        if (FWD) {
-            if (LAZY)
-                ct_unit<LOGT>(x, 1u, tw, tws, IntKLazy{q});
-            else
-                ct_unit<LOGT>(x, 1u, tw, tws, IntK{q});
+        const auto ar = arith_of<A>(tb, prime, N);
+        if constexpr (FWD) {
+            ct_unit<LOGT>(x, 1u, ar);
             // streaming store: the tile pass reads these words back long after
 #pragma unroll
             for (int r = 0; r < T; r++) __builtin_nontemporal_store(x[r], &base[r * N2]);
         } else {
-            gs_unit<LOGT>(x, 1u, tw, tws, IntK{q});
+            gs_unit<LOGT>(x, 1u, ar);
             const uint64_t ni = tb.ninv[prime], nis = tb.ninv_s[prime];
+            if constexpr (A == FOLD) {
+                const u32x4 nf = fold_split(ni, nis, q, ar.f);
 #pragma unroll
-            for (int r = 0; r < T; r++) __builtin_nontemporal_store(mul_shoup(x[r], ni, nis, q), &base[r * N2]);
+                for (int r = 0; r < T; r++)
+                    __builtin_nontemporal_store(fold_canon(fold_mul(x[r], nf, ar.f), q, ar.f), &base[r * N2]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < T; r++) __builtin_nontemporal_store(mul_shoup(x[r], ni, nis, q), &base[r * N2]);
+            }
         }
     }
 }
@@ -375,7 +438,7 @@ __global__ __launch_bounds__(kThreads, IO == IO_ENCODE ? 1 : 6) void k_ntt_cols(
 // O = (limb * tiles + tile) * n_polys + poly: the polynomials that share one
 // prime and tile (hence one twiddle slice) run back to back on the same L2.
 // 512-thread blocks ask for 6 waves per SIMD (80 VGPRs), three 32 KB tiles per CU.
-template <int LOGT, bool FWD, int IO, bool LAZY, int NT = kThreads>
+template <int LOGT, bool FWD, int IO, int A, int NT = kThreads>
 __global__ __launch_bounds__(NT, NT >= 512 ? 6 : 1) void k_ntt_blocks(uint64_t *__restrict__ data, LimbMap mp, NttTables tb,
                                                          int logN, NttIO io, uint32_t n_polys, uint32_t per_xcd) {
     constexpr int T = 1 << LOGT;
@@ -473,15 +536,13 @@ __global__ __launch_bounds__(NT, NT >= 512 ? 6 : 1) void k_ntt_blocks(uint64_t *
         }
     };
     __syncthreads();
-    if (LAZY)
-        run_rounds<LOGT, FWD, NT>(lds, N1, 1u, (uint32_t)(t0 / T), tb.tw + (size_t)prime * N,
-                                  tb.tws + (size_t)prime * N, IntKLazy{q}, load_acc);
-    else
-        run_rounds<LOGT, FWD, NT>(lds, N1, 1u, (uint32_t)(t0 / T), tb.tw + (size_t)prime * N,
-                                  tb.tws + (size_t)prime * N, IntK{q}, load_acc);
-    // canonical residue of a forward output: below 4q, or below (4 + 4 log N) q when lazy
+    const auto ar = arith_of<A>(tb, prime, N);
+    run_rounds<LOGT, FWD, NT>(lds, N1, 1u, (uint32_t)(t0 / T), ar, load_acc);
+    // canonical residue of a forward output: below 4q, below (4 + 4 log N) q when lazy,
+    // signed when folded
     auto canon = [&](uint64_t v) -> uint64_t {
-        if (LAZY) return reduce64(v, tb.mods[prime]);
+        if constexpr (A == FOLD) return fold_canon(v, q, ar.f);
+        if (A == LAZY) return reduce64(v, tb.mods[prime]);
         v = v >= q2 ? v - q2 : v;
         return v >= q ? v - q : v;
     };
@@ -491,8 +552,11 @@ __global__ __launch_bounds__(NT, NT >= 512 ? 6 : 1) void k_ntt_blocks(uint64_t *
         // is taken as acc + (4 + 4 logN) q - v, which the Shoup product accepts as it is
         const uint64_t kq = (uint64_t)(4 + 4 * logN) * q;
         const bool addto = io.out_packed && poly < 64 && ((io.acc_mask >> poly) & 1);
+        u32x4 qf = {0, 0, 0, 0};
+        if constexpr (A == FOLD) qf = fold_split(qi, qis, q, ar.f);
         auto result = [&](uint64_t acc, uint64_t raw) -> uint64_t {
-            return LAZY ? mul_shoup(acc + kq - raw, qi, qis, q) : mul_shoup(sub_mod(acc, canon(raw), q), qi, qis, q);
+            if constexpr (A == FOLD) return fold_canon(fold_mul(acc - raw, qf, ar.f), q, ar.f);
+            return A == LAZY ? mul_shoup(acc + kq - raw, qi, qis, q) : mul_shoup(sub_mod(acc, canon(raw), q), qi, qis, q);
         };
         auto addend = [&](int i) -> uint64_t {
             return *global_ptr(io.add_src.p[poly] + (size_t)k * N + io.add_perm[t0 + i]);
@@ -580,47 +644,64 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
                  FWD ? c.tw.as<uint64_t>() : c.itw.as<uint64_t>(),
                  FWD ? c.tw_s.as<uint64_t>() : c.itw_s.as<uint64_t>(),
                  c.ninv.as<uint64_t>(),
-                 c.ninv_s.as<uint64_t>()};
-    // unreduced forward butterflies when (5 + 4 log N) q < 2^64 for every prime of the
-    // launch: values below (4 + 4 log N) q, plus one q of the fused epilogue's operand
-    bool lazy = FWD;
-    const uint64_t lazy_max = ~uint64_t(0) / (uint64_t)(5 + 4 * c.logN);
-    for (uint32_t j = 0; j < mp.n_active && lazy; j++) {
-        uint32_t k = mp.lo + j;
-        if (k >= mp.skip_lo) k += mp.skip_width;
-        const uint32_t prime = k < mp.Ql ? mp.first_prime + k : mp.nQ + (k - mp.Ql);
-        lazy = c.q.at(prime) < lazy_max;
-    }
+                 c.ninv_s.as<uint64_t>(),
+                 FWD ? c.tw_f.as<u32x4>() : c.itw_f.as<u32x4>(),
+                 c.d_fold.as<FoldMod>()};
     // tile passes in 512-thread blocks of radix-8 rounds (the default): the lazy forward
     // passes and the inverse ones; the forward passes of primes above the lazy bound keep
     // 256-thread radix-16 rounds (their fused form would spill at 80 registers)
     const bool tile512 = ks_tuning().ntt_tile_threads == 512;
+    // Split products when every prime of the launch has them and the signed words cannot
+    // overflow: forward, input (below 4q, or a residue of another prime of the context)
+    // plus log N products plus the fused epilogue's operand; inverse, the sums of one unit.
+    // Otherwise forward butterflies leave a unreduced when (5 + 4 log N) q < 2^64 for every
+    // prime: values below (4 + 4 log N) q, plus one q of the fused epilogue's operand.
+    bool lazy = FWD, fold = true;
+    const uint64_t lazy_max = ~uint64_t(0) / (uint64_t)(5 + 4 * c.logN);
+    const uint64_t q_any = *std::max_element(c.q.begin(), c.q.end());
+    for (uint32_t j = 0; j < mp.n_active && (lazy || fold); j++) {
+        uint32_t k = mp.lo + j;
+        if (k >= mp.skip_lo) k += mp.skip_width;
+        const uint32_t prime = k < mp.Ql ? mp.first_prime + k : mp.nQ + (k - mp.Ql);
+        const uint64_t q = c.q.at(prime), r = c.fold_bound.at(prime);
+        lazy = lazy && q < lazy_max;
+        const uint64_t in = IOA == IO_REDUCE ? std::max(q_any, 4 * q) : 4 * q;
+        const uint64_t top = (uint64_t(1) << 63) - 1 - 2 * q;
+        fold = fold && r != 0 && (FWD ? in < top && r <= (top - in) / (uint64_t)c.logN
+                                       : r < (uint64_t(1) << (63 - std::max(log1, tile512 ? 3 : 4))));
+    }
+    const int arith = fold ? FOLD : lazy ? LAZY : HARVEY;
     // the tile pass reads its input in 16-byte pairs of words
     bool aligned = ((uintptr_t)data & 15) == 0 && mp.poly_stride % 2 == 0;
     if (IOB == IO_GATHER)
         for (uint32_t p = 0; p < n_polys; p++) aligned = aligned && ((uintptr_t)io.acc_p.p[p] & 15) == 0;
     if (!aligned) throw InvalidArgument("NTT operands must be 16-byte aligned");
-#define SHM_COLS(L)                                                                                    \
-    case L:                                                                                            \
-        if (lazy)                                                                                      \
-            k_ntt_cols<L, FWD, IOA, true><<<grid_cols, kThreads, 0, s>>>(data, mp, tb, logN, io);      \
-        else                                                                                           \
-            k_ntt_cols<L, FWD, IOA, false><<<grid_cols, kThreads, 0, s>>>(data, mp, tb, logN, io);     \
+#define SHM_COLS_A(L, A) k_ntt_cols<L, FWD, IOA, A><<<grid_cols, kThreads, 0, s>>>(data, mp, tb, logN, io)
+#define SHM_BLKS_A(L, A, NT) \
+    k_ntt_blocks<L, FWD, IOB, A, NT><<<grid_blk, NT, 0, s>>>(data, mp, tb, logN, io, n_polys, per_xcd)
+#define SHM_COLS(L)                                 \
+    case L:                                         \
+        if (arith == FOLD)                          \
+            SHM_COLS_A(L, FOLD);                    \
+        else if (arith == LAZY)                     \
+            SHM_COLS_A(L, (FWD ? LAZY : HARVEY));   \
+        else                                        \
+            SHM_COLS_A(L, HARVEY);                  \
         break;
-#define SHM_BLKS(L)                                                                                          \
-    case L:                                                                                                  \
-        if (lazy && tile512)                                                                                 \
-            k_ntt_blocks<L, FWD, IOB, true, 512><<<grid_blk, 512, 0, s>>>(data, mp, tb, logN, io, n_polys,   \
-                                                                          per_xcd);                          \
-        else if (lazy)                                                                                       \
-            k_ntt_blocks<L, FWD, IOB, true><<<grid_blk, kThreads, 0, s>>>(data, mp, tb, logN, io, n_polys,    \
-                                                                          per_xcd);                          \
-        else if (!FWD && tile512)                                                                            \
-            k_ntt_blocks<L, FWD, IOB, false, 512><<<grid_blk, 512, 0, s>>>(data, mp, tb, logN, io, n_polys,  \
-                                                                           per_xcd);                         \
-        else                                                                                                 \
-            k_ntt_blocks<L, FWD, IOB, false><<<grid_blk, kThreads, 0, s>>>(data, mp, tb, logN, io, n_polys,   \
-                                                                           per_xcd);                         \
+#define SHM_BLKS(L)                                 \
+    case L:                                         \
+        if (arith == FOLD && tile512)               \
+            SHM_BLKS_A(L, FOLD, 512);               \
+        else if (arith == FOLD)                     \
+            SHM_BLKS_A(L, FOLD, 256);               \
+        else if (arith == LAZY && tile512)          \
+            SHM_BLKS_A(L, (FWD ? LAZY : HARVEY), 512); \
+        else if (arith == LAZY)                     \
+            SHM_BLKS_A(L, (FWD ? LAZY : HARVEY), 256); \
+        else if (!FWD && tile512)                   \
+            SHM_BLKS_A(L, HARVEY, (FWD ? 256 : 512)); \
+        else                                        \
+            SHM_BLKS_A(L, HARVEY, 256);             \
         break;
     auto cols = [&]() {
         switch (log1) {
@@ -641,6 +722,8 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
     };
 #undef SHM_COLS
 #undef SHM_BLKS
+#undef SHM_COLS_A
+#undef SHM_BLKS_A
     if (FWD) {
         cols();
         const bool timed = IOB == IO_RESCALE && g_rescale_tile_ev[0] && g_rescale_tile_ev[1];
