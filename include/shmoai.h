@@ -580,8 +580,8 @@ int shm_keyswitch_counters_reset(void);
  * default) for the autotuned choice; "matmul_overlap" (0, the default, or 1) runs the INT8
  * ct-pt matmul's contraction and rescale one after the other, or overlaps the contraction
  * (row_W <= 256, in limb windows) with the rescale on a second stream of the context;
- * "ntt_tile_threads" (512, the default, or 256) runs the NTT tile passes in 512-thread
- * blocks of radix-8 rounds or 256-thread blocks of radix-16 rounds (the same words).
+ * "ntt_tile_threads" (512, the default, or 256) runs the NTT row pass in blocks of 512 or
+ * 256 threads (the same words).
  * Process-wide. */
 int shm_set_tuning(const char *name, int32_t value);
 int shm_get_tuning(const char *name, int32_t *value);

@@ -162,6 +162,7 @@ struct FoldMod {
     uint32_t sh;    // b - 32
     uint32_t mask;  // 2^(b - 32) - 1
     uint32_t s;     // b - 30
+    uint32_t twice; // one fold of a 64-bit word can leave it at 2q or more
     uint64_t off;   // the smallest multiple of q that is at least 2^63
 };
 
@@ -186,12 +187,17 @@ __device__ __forceinline__ uint64_t fold_tight(uint64_t x, const FoldMod &f) {
 }
 
 // Canonical residue of a signed x, |x| <= 2^63 - q: the offset makes it unsigned, and one
-// fold leaves it below 2^b + 2^(64-b) delta < 2q.
+// fold (two where f.twice) leaves it below 2q.
+template <bool TWICE>
 __device__ __forceinline__ uint64_t fold_canon(uint64_t x, uint64_t q, const FoldMod &f) {
-    const uint64_t y = x + f.off;
-    const uint32_t yh = (uint32_t)(y >> 32);
-    const uint64_t lo = ((uint64_t)(yh & f.mask) << 32) | (uint32_t)y;
-    return csub((uint64_t)(yh >> f.sh) * (uint32_t)f.d + lo, q);
+    auto fold = [&](uint64_t y) {
+        const uint32_t yh = (uint32_t)(y >> 32);
+        const uint64_t lo = ((uint64_t)(yh & f.mask) << 32) | (uint32_t)y;
+        return (uint64_t)(yh >> f.sh) * (uint32_t)f.d + lo;
+    };
+    uint64_t y = fold(x + f.off);
+    if (TWICE) y = fold(y);
+    return csub(y, q);
 }
 
 // The split form of a constant w < q given its Shoup companion.

@@ -108,15 +108,21 @@ uint64_t min_root_2n(uint64_t q, uint64_t two_n) {
     return best;
 }
 
-// The split form of prime q (FoldMod), and in *bound the largest |fold_mul|; false when
-// q has none: 36 to 58 bits, delta below 2^29, and one fold of an unsigned 64-bit word
-// leaves it below 2q.
+// The split form of prime q (FoldMod), and in *bound the largest |fold_mul|; false when q
+// has none: 36 to 58 bits, four products and an input of 2^61 fit a signed word (bound <=
+// 1.25 2^60, which leaves delta below 2^28), and two folds of an unsigned 64-bit word
+// leave it below 2q.
 bool fold_form(uint64_t q, FoldMod *f, uint64_t *bound) {
     int b = 0;
     while (b < 64 && (q >> b)) b++;
     if (b < 36 || b > 58) return false;
     const uint64_t delta = (uint64_t(1) << b) - q;
-    if (delta >= (uint64_t(1) << 29) || (((hu128)delta << (64 - b)) + 2 * delta) >> b) return false;
+    const hu128 r = ((hu128)10 << b) + ((hu128)delta << 32) + ((hu128)delta << 31);  // 2.5 2^(b+2) + 6 2^30 delta
+    if (r > ((hu128)5 << 58)) return false;
+    // one fold: below 2^b + 2^(64-b) delta; a second: below 2^b + (that >> b) delta
+    const hu128 once = ((hu128)1 << b) + ((hu128)delta << (64 - b));
+    if (((once >> b) + 2) * delta >> b) return false;
+    f->twice = once >= 2 * (hu128)q;
     f->s = (uint32_t)(b - 30);
     f->pw = 1u << f->s;
     f->d = (int32_t)delta;
@@ -124,21 +130,8 @@ bool fold_form(uint64_t q, FoldMod *f, uint64_t *bound) {
     f->sh = (uint32_t)(b - 32);
     f->mask = (1u << f->sh) - 1;
     f->off = ((uint64_t(1) << 63) + q - 1) / q * q;
-    *bound = (uint64_t(10) << b) + (delta << 32) + (delta << 31);  // 2.5 2^(b+2) + 6 2^30 delta
+    *bound = (uint64_t)r;
     return true;
-}
-
-// Split forms of a twiddle table: row p of `out` from row p of `tw` (one thread per
-// twiddle; primes without a split form, pw = 0, are skipped).
-__global__ void k_split_twiddles(const uint64_t *__restrict__ tw, const DevMod *__restrict__ mods,
-                                 const FoldMod *__restrict__ fold, u32x4 *__restrict__ out, size_t N) {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    const uint32_t p = blockIdx.y;
-    const FoldMod f = fold[p];
-    if (i >= N || f.pw == 0) return;
-    const uint64_t w = tw[(size_t)p * N + i], w1 = mul_mod(w, uint64_t(1) << 32, mods[p]);
-    const uint32_t m = f.pw - 1;
-    out[(size_t)p * N + i] = u32x4{(uint32_t)(w >> f.s), (uint32_t)w & m, (uint32_t)(w1 >> f.s), (uint32_t)w1 & m};
 }
 
 template <class T>
@@ -368,7 +361,7 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
     const size_t N = c->N, QP = c->q.size();
 
     std::vector<DevMod> mods(QP);
-    std::vector<uint64_t> tw(QP * N), tws(QP * N), itw(QP * N), itws(QP * N), ninv(QP), ninvs(QP);
+    std::vector<uint64_t> tw(QP * N), itw(QP * N), ninv(QP), ninvs(QP);
     c->psi.resize(QP);
     for (size_t p = 0; p < QP; p++) {
         const uint64_t q = c->q[p];
@@ -384,10 +377,6 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
             pw = h_mulmod(pw, psi, q);
             ipw = h_mulmod(ipw, ipsi, q);
         }
-        for (size_t i = 0; i < N; i++) {
-            tws[p * N + i] = h_shoup(tw[p * N + i], q);
-            itws[p * N + i] = h_shoup(itw[p * N + i], q);
-        }
         ninv[p] = h_inv(N, q);
         ninvs[p] = h_shoup(ninv[p], q);
     }
@@ -399,24 +388,20 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
     }
     upload(c->iota, io);
     upload(c->iota_s, ios);
-    upload(c->tw, tw);
-    upload(c->tw_s, tws);
-    upload(c->itw, itw);
-    upload(c->itw_s, itws);
     upload(c->ninv, ninv);
     upload(c->ninv_s, ninvs);
     std::vector<FoldMod> fold(QP, FoldMod{});
     c->fold_bound.assign(QP, 0);
-    bool any_fold = false;
-    for (size_t p = 0; p < QP; p++) any_fold = fold_form(c->q[p], &fold[p], &c->fold_bound[p]) || any_fold;
+    for (size_t p = 0; p < QP; p++)
+        if (!fold_form(c->q[p], &fold[p], &c->fold_bound[p])) fold[p] = FoldMod{};
+    for (const FoldMod &f : fold) c->fold_twice.push_back(f.twice != 0);
     upload(c->d_fold, fold);
-    if (any_fold) {
-        c->tw_f.alloc(QP * N * sizeof(u32x4));
-        c->itw_f.alloc(QP * N * sizeof(u32x4));
-        const dim3 grid((unsigned)((N + 255) / 256), (unsigned)QP);
-        k_split_twiddles<<<grid, 256>>>(c->tw.as<uint64_t>(), c->mods(), c->d_fold.as<FoldMod>(), c->tw_f.as<u32x4>(), N);
-        k_split_twiddles<<<grid, 256>>>(c->itw.as<uint64_t>(), c->mods(), c->d_fold.as<FoldMod>(), c->itw_f.as<u32x4>(), N);
-        SHM_HIP(hipGetLastError());
+    {
+        DevBuf t;
+        upload(t, tw);
+        ntt_make_tables(*c, t.as<uint64_t>(), c->tw_col, c->tw_row);
+        upload(t, itw);
+        ntt_make_tables(*c, t.as<uint64_t>(), c->itw_col, c->itw_row);
     }
 
     // ModDown constants (rns.cu:95-128, 187-190): P mod q_i, P^-1 mod q_i,

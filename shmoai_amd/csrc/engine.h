@@ -141,14 +141,15 @@ struct Context {
 
     // device tables
     DevBuf d_mod;           // DevMod[QP]
-    DevBuf tw, tw_s;        // [QP][N]
-    DevBuf itw, itw_s;      // [QP][N]
-    DevBuf ninv, ninv_s;    // [QP]
-    // split forms of the twiddles for primes just below a power of two (FoldMod):
-    // u32x4[QP][N], and FoldMod[QP]; fold_bound[p] is the largest |fold_mul| of prime
-    // p, 0 when it has no split form
-    DevBuf tw_f, itw_f, d_fold;
+    // NTT twiddles (forward, inverse) as 16-byte entries, split forms for primes just below
+    // a power of two and Shoup pairs for others: the column stages' u32x4[QP][kNttCols] and
+    // the row stages' u32x4[QP][N] in lane order (ntt.hip); FoldMod[QP] (pw = 0: none), and
+    // fold_bound[p], the largest |fold_mul| of prime p (0: no split form); fold_twice[p]: one
+    // fold of a 64-bit word can leave it at 2q or more
+    DevBuf tw_col, tw_row, itw_col, itw_row, d_fold;
     std::vector<uint64_t> fold_bound;
+    std::vector<uint8_t> fold_twice;
+    DevBuf ninv, ninv_s;    // [QP]
     DevBuf pinv, pinv_s;    // P^-1 mod q_i, i < nQ
     DevBuf pmod, pmod_s;    // P mod q_i, i < nQ
     DevBuf phat_inv, phat_inv_s;  // [nP] (P/p_j)^-1 mod p_j
@@ -243,6 +244,10 @@ struct GaloisKeys {
 // (device array) or by a contiguous range starting at first_prime.
 void ntt_forward(const Context &c, uint64_t *data, size_t n_polys, size_t n_limbs, size_t first_prime,
                  hipStream_t s);
+// Twiddle entries in the order the transforms read them, from twiddles tw[QP][N] in
+// bit-reversed order (tw[m + i] belongs to group i of the stage with m groups).
+constexpr int kNttCols = 256;  // column entries kept per prime (N / 512 are used)
+void ntt_make_tables(const Context &c, const uint64_t *tw, DevBuf &col, DevBuf &row);
 // Events recorded around the tile pass of every fused-rescale NTT launched while
 // set (nullptr to stop); used to time the matmul's rescale.
 void set_rescale_tile_events(hipEvent_t start, hipEvent_t stop);
@@ -268,8 +273,8 @@ struct KsTuning {
     // the context's second stream (1) or runs them one after the other (0, the default:
     // both kernels fill the GPU, and the overlapped form measured 7% slower)
     int matmul_overlap = 0;
-    // threads per block of the NTT tile passes: 512 (radix-8 rounds, more waves per
-    // 32 KB tile; the default) or 256 (radix-16 rounds); the results are the same words
+    // threads per block of the NTT row pass, 512 or 256 (one wave per row either way; the
+    // same words and, within 2%, the same times)
     int ntt_tile_threads = 512;
 };
 KsTuning &ks_tuning();

@@ -6,24 +6,31 @@
 //   evaluation at psi^(2 brv(j) + 1) in slot j, fully reduced to [0, q).
 //   inverse Gentleman-Sande with itw[brv(k)] = psi^-k, then x N^-1.
 //
-// Decomposition: N = N1 * N2 with N2 = min(4096, N / 16). The first log N1
-// stages (4 or 5) only pair elements whose indices differ by multiples of N2,
-// so each "column" {c + N2 r} is an independent N1-point transform: phase A
-// gives one column to each thread and runs it in registers. The last log N2
-// stages act on contiguous blocks of N2 elements (phase B): a 4096-word tile
-// is staged in LDS, then rounds of up to 4 stages run in registers (radix-16
-// units). A sub-transform whose first-stage group id is G uses twiddle
-// tw[(G << u) + i'] at its local stage u for local group i'.
+// Decomposition: N = N1 * 512. The first log N1 = log N - 9 stages (3 to 8) pair words
+// whose indices differ by multiples of 512 (column pass): up to 5 stages a thread holds a
+// whole column in registers; 6 to 8 stages take two rounds of register units with one
+// exchange through LDS. The last 9 stages act on 512 contiguous words (row pass): one wave
+// runs a row in three rounds of radix-8 units, 8 words per lane, and exchanges between
+// rounds through LDS words of its own, so the row pass has no block barrier at all. An
+// earlier split of 4 + 12 stages staged 4096-word tiles through LDS with five barriers, and
+// its tile pass held 734 of a word group's 890 vector instructions; with 7 + 9 stages both
+// passes stay below the memory's time (64 x 24 limbs at N = 2^16, forward: column pass 267
+// -> 294 us, tile / row pass 393 -> 326 us; each moves 1.61 GB).
 //
-// Butterfly arithmetic, by the primes of a launch (launch_ntt):
-//   - primes with a split form (FoldMod, arith.h), i.e. all of 36 to 58 bits just below a
-//     power of two: signed unreduced words, nine issue slots a butterfly. The tile pass of
-//     64 x 24 limbs at N = 2^16 issues 734 VALU instructions per wave instead of 1325 (the
-//     unreduced Shoup form): 548 -> 393 us forward, 646 -> 393 us inverse;
-//   - otherwise, forward and below 2^64 / (5 + 4 log N) (about 2^57.9): unreduced Shoup
-//     butterflies with a cheaper quotient (values below (4 + 4 log N) q);
+// Twiddles are 16-byte entries: the split form of a prime just below a power of two
+// (FoldMod, arith.h) or (w, floor(w 2^64 / q)) of any other. A row's 511 entries lie in the
+// order its lanes read them, [round 1: 7][round 2: 7][8][round 3: 7][64], so that every
+// load of a wave is one contiguous run (round 3 read from a table in stage order
+// spreads a load over up to 64 cache lines).
+//
+// Butterfly arithmetic, by prime:
+//   - split form: signed unreduced words, (a + t, a - t) with |t| <= R = fold_bound, nine
+//     issue slots a butterfly (a Shoup butterfly takes about 26);
 //   - otherwise Harvey's lazy ranges: [0, 4q) forward, [0, 2q) inverse (primes < 2^61).
-// Outputs are canonical residues, the same words in every form.
+// A launch whose primes all have split forms and whose log N products fit a signed word
+// runs kernels of that form alone (FAST); any other launch runs kernels that pick the form
+// per limb and fold split-form words every second stage (GENERAL). Outputs are canonical
+// residues, the same words in every form.
 #include <algorithm>
 
 #include <mutex>
@@ -55,7 +62,8 @@ __device__ __forceinline__ void limb_of(const LimbMap &m, uint32_t z, uint32_t &
 
 namespace {
 
-constexpr int kTile = 4096;
+constexpr int kRow = 512;       // words of a row: the last 9 stages
+constexpr int kRowLds = 576;    // LDS words of a row: one of padding per 8 (row_slot)
 constexpr int kThreads = 256;
 
 typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
@@ -74,245 +82,119 @@ __device__ __forceinline__ const __attribute__((address_space(1))) V *global_ptr
 // Twiddle and constant tables of one launch (forward or inverse set).
 struct NttTables {
     const DevMod *mods;
-    const uint64_t *tw, *tws;   // twiddles and their Shoup quotients
+    const FoldMod *fold;              // pw = 0: the prime has no split form
+    const u32x4 *col;                 // [QP][kNttCols]: twiddles 1 .. N1 - 1 of the column stages
+    const u32x4 *row;                 // [QP][N / 512][512]: each row's twiddles in lane order
     const uint64_t *ninv, *ninv_s;
-    const u32x4 *twf;           // split twiddles and prime constants (primes with a split form)
-    const FoldMod *fold;
 };
 
-// Butterfly arithmetic of a launch, chosen by its primes (launch_ntt):
-//   HARVEY : any prime below 2^61; forward keeps [0, 4q), inverse [0, 2q).
-//   LAZY   : forward, (5 + 4 log N) q < 2^64; a stays unreduced (below).
-//   FOLD   : every prime has a split form (FoldMod) and log N fold_mul results fit a
-//            signed word; words are signed and unreduced.
-enum { HARVEY = 0, LAZY = 1, FOLD = 2 };
-
-// One prime's tables in the form its butterflies read them.
+// Arithmetic of one prime. fwd / inv: one stage's butterflies on a unit of 2^R words, tw(e)
+// being the entry of group i at unit stage u, e = 2^u - 1 + i.
 struct HarveyK {
-    const uint64_t *__restrict__ tw, *__restrict__ tws;
     uint64_t q;
+    __device__ HarveyK(const NttTables &tb, uint32_t prime) : q(tb.mods[prime].q) {}
+    static __device__ __forceinline__ uint64_t lo(u32x4 w) { return ((uint64_t)w.y << 32) | w.x; }
+    static __device__ __forceinline__ uint64_t hi(u32x4 w) { return ((uint64_t)w.w << 32) | w.z; }
+    __device__ __forceinline__ void fwd(uint64_t &a, uint64_t &b, u32x4 w) const {
+        const uint64_t q2 = q << 1, s = a >= q2 ? a - q2 : a;
+        const uint64_t t = mul_shoup_lazy(b, lo(w), hi(w), q);
+        a = s + t;
+        b = s + q2 - t;
+    }
+    __device__ __forceinline__ void inv(uint64_t &a, uint64_t &b, u32x4 w) const {
+        const uint64_t q2 = q << 1, d = a + q2 - b, s = a + b;
+        a = s >= q2 ? s - q2 : s;
+        b = mul_shoup_lazy(d, lo(w), hi(w), q);
+    }
+    template <int R>
+    __device__ __forceinline__ void after_fwd(uint64_t *, int) const {}
+    template <int R>
+    __device__ __forceinline__ void after_inv(uint64_t *, int) const {}
+    // canonical residue of a forward word, and of x w (Shoup pair w, ws)
+    __device__ __forceinline__ uint64_t canon(uint64_t v) const {
+        v = v >= (q << 1) ? v - (q << 1) : v;
+        return v >= q ? v - q : v;
+    }
+    struct Const {
+        uint64_t w, ws;
+    };
+    __device__ __forceinline__ Const constant(uint64_t w, uint64_t ws) const { return {w, ws}; }
+    __device__ __forceinline__ uint64_t mul(uint64_t x, Const c) const { return mul_shoup(x, c.w, c.ws, q); }
+    __device__ __forceinline__ uint64_t sub_mul(uint64_t acc, uint64_t v, Const c) const {
+        return mul_shoup(sub_mod(acc, canon(v), q), c.w, c.ws, q);
+    }
+    __device__ __forceinline__ uint64_t load_residue(uint64_t v, uint64_t center, const DevMod &m) const {
+        uint64_t y = reduce64(v, m);
+        if (center && v > center) y = sub_mod(y, reduce64(2 * center + 1, m), q);
+        return y;
+    }
+    __device__ __forceinline__ uint64_t load_rounded(double v, const DevMod &m) const { return residue_of_rounded(v, m); }
 };
-struct LazyK {
-    const uint64_t *__restrict__ tw, *__restrict__ tws;
-    uint64_t q;
-};
+
+// SAFE folds a unit's words every second stage, so only a few products ever add up (for
+// primes further below the power of two, and for limbs of GENERAL launches); otherwise the
+// launcher has checked that log N of them fit.
+template <bool SAFE>
 struct FoldK {
-    const u32x4 *__restrict__ tw;
+    uint64_t q;
     FoldMod f;
+    __device__ FoldK(const NttTables &tb, uint32_t prime) : q(tb.mods[prime].q), f(tb.fold[prime]) {}
+    __device__ __forceinline__ void fwd(uint64_t &a, uint64_t &b, u32x4 w) const {
+        const uint64_t t = fold_mul(b, w, f), s = a;
+        a = s + t;
+        b = s - t;
+    }
+    __device__ __forceinline__ void inv(uint64_t &a, uint64_t &b, u32x4 w) const {
+        const uint64_t d = a - b;
+        a = a + b;
+        b = fold_mul(d, w, f);
+    }
+    template <int R>
+    __device__ __forceinline__ void after_fwd(uint64_t *x, int u) const {
+        if (SAFE && ((u & 1) || u == R - 1))
+#pragma unroll
+            for (int l = 0; l < (1 << R); l++) x[l] = fold_tight(x[l], f);
+    }
+    // sums double per stage: those of a unit's last stage (l < 2^(R-1)) come back to b bits
+    template <int R>
+    __device__ __forceinline__ void after_inv(uint64_t *x, int u) const {
+#pragma unroll
+        for (int l = 0; l < (1 << R); l++)
+            if (u == 0 ? l < (1 << (R - 1)) : SAFE && (((R - 1 - u) & 1) != 0)) x[l] = fold_tight(x[l], f);
+    }
+    __device__ __forceinline__ uint64_t canon(uint64_t v) const { return fold_canon<SAFE>(v, q, f); }
+    typedef u32x4 Const;
+    __device__ __forceinline__ Const constant(uint64_t w, uint64_t ws) const { return fold_split(w, ws, q, f); }
+    __device__ __forceinline__ uint64_t mul(uint64_t x, Const c) const { return fold_canon<SAFE>(fold_mul(x, c, f), q, f); }
+    __device__ __forceinline__ uint64_t sub_mul(uint64_t acc, uint64_t v, Const c) const { return mul(acc - v, c); }
+    // signed words need no reduction
+    __device__ __forceinline__ uint64_t load_residue(uint64_t v, uint64_t center, const DevMod &) const {
+        return center && v > center ? v - (2 * center + 1) : v;
+    }
+    __device__ __forceinline__ uint64_t load_rounded(double v, const DevMod &m) const { return residue_of_rounded(v, m); }
 };
 
-template <int A>
-__device__ __forceinline__ auto arith_of(const NttTables &tb, uint32_t prime, size_t N) {
-    if constexpr (A == FOLD)
-        return FoldK{tb.twf + (size_t)prime * N, tb.fold[prime]};
-    else if constexpr (A == LAZY)
-        return LazyK{tb.tw + (size_t)prime * N, tb.tws + (size_t)prime * N, tb.mods[prime].q};
-    else
-        return HarveyK{tb.tw + (size_t)prime * N, tb.tws + (size_t)prime * N, tb.mods[prime].q};
-}
-
-template <int R>
-__device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const HarveyK &k) {
-    const uint64_t q = k.q, q2 = q << 1;
+template <int R, typename K, typename TW>
+__device__ __forceinline__ void ct_unit(uint64_t *x, const K &k, TW tw) {
 #pragma unroll
     for (int u = 0; u < R; u++) {
         const int h = 1 << (R - 1 - u);
 #pragma unroll
-        for (int l = 0; l < (1 << R); l++) {
-            if ((l & h) == 0) {
-                const uint32_t ti = (G << u) + (uint32_t)(l >> (R - u));
-                const uint64_t w = k.tw[ti], ws = k.tws[ti];
-                uint64_t a = x[l];
-                a = a >= q2 ? a - q2 : a;
-                const uint64_t t = mul_shoup_lazy(x[l + h], w, ws, q);
-                x[l] = a + t;
-                x[l + h] = a + q2 - t;
-            }
-        }
+        for (int l = 0; l < (1 << R); l++)
+            if ((l & h) == 0) k.fwd(x[l], x[l + h], tw((1 << u) - 1 + (l >> (R - u))));
+        k.template after_fwd<R>(x, u);
     }
 }
 
-// Forward butterflies that leave a unreduced: with t = x w mod q in [0, 4q) (the
-// quotient estimate of mul_shoup_lazy4, at most 2 short), both outputs stay below
-// a + 4q, so log N stages from inputs below 4q end below (4 + 4 log N) q, which fits
-// 64 bits for the primes the launcher allows here. Saves the compare-select-subtract
-// of every butterfly and part of the quotient's multiplies; the final pass reduces once.
-template <int R>
-__device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const LazyK &k) {
-    const uint64_t q = k.q, q4 = q << 2;
-#pragma unroll
-    for (int u = 0; u < R; u++) {
-        const int h = 1 << (R - 1 - u);
-#pragma unroll
-        for (int l = 0; l < (1 << R); l++) {
-            if ((l & h) == 0) {
-                const uint32_t ti = (G << u) + (uint32_t)(l >> (R - u));
-                const uint64_t a = x[l];
-                const uint64_t t = mul_shoup_lazy4(x[l + h], k.tw[ti], k.tws[ti], q);
-                x[l] = a + t;
-                x[l + h] = a + q4 - t;
-            }
-        }
-    }
-}
-
-// Signed forward butterflies (a + t, a - t) with t = fold_mul(x, w), |t| <= R: log N
-// stages add at most log N R to the input's bound, which the launcher checks against
-// 2^63. Nine multiply-add or 64-bit add slots a butterfly where the Shoup form issued 26.
-template <int R>
-__device__ __forceinline__ void ct_unit(uint64_t *x, uint32_t G, const FoldK &k) {
-#pragma unroll
-    for (int u = 0; u < R; u++) {
-        const int h = 1 << (R - 1 - u);
-#pragma unroll
-        for (int l = 0; l < (1 << R); l++) {
-            if ((l & h) == 0) {
-                const uint64_t a = x[l];
-                const uint64_t t = fold_mul(x[l + h], k.tw[(G << u) + (uint32_t)(l >> (R - u))], k.f);
-                x[l] = a + t;
-                x[l + h] = a - t;
-            }
-        }
-    }
-}
-
-template <int R>
-__device__ __forceinline__ void gs_unit(uint64_t *x, uint32_t G, const HarveyK &k) {
-    const uint64_t q = k.q, q2 = q << 1;
+template <int R, typename K, typename TW>
+__device__ __forceinline__ void gs_unit(uint64_t *x, const K &k, TW tw) {
 #pragma unroll
     for (int u = R - 1; u >= 0; u--) {
         const int h = 1 << (R - 1 - u);
 #pragma unroll
-        for (int l = 0; l < (1 << R); l++) {
-            if ((l & h) == 0) {
-                const uint32_t ti = (G << u) + (uint32_t)(l >> (R - u));
-                const uint64_t w = k.tw[ti], ws = k.tws[ti];
-                const uint64_t a = x[l], b = x[l + h];
-                uint64_t s = a + b;
-                s = s >= q2 ? s - q2 : s;
-                x[l] = s;
-                x[l + h] = mul_shoup_lazy(a + q2 - b, w, ws, q);
-            }
-        }
-    }
-}
-
-// Signed inverse butterflies (a + b, (a - b) w). A unit's inputs are within the bound R of
-// fold_mul, sums double per stage (2^(R-1) R before the last product: below 2^63 is
-// checked by the launcher), and the sums of the unit's last stage are folded to b bits.
-template <int R>
-__device__ __forceinline__ void gs_unit(uint64_t *x, uint32_t G, const FoldK &k) {
-#pragma unroll
-    for (int u = R - 1; u >= 0; u--) {
-        const int h = 1 << (R - 1 - u);
-#pragma unroll
-        for (int l = 0; l < (1 << R); l++) {
-            if ((l & h) == 0) {
-                const uint64_t a = x[l], b = x[l + h];
-                x[l] = u == 0 ? fold_tight(a + b, k.f) : a + b;
-                x[l + h] = fold_mul(a - b, k.tw[(G << u) + (uint32_t)(l >> (R - u))], k.f);
-            }
-        }
-    }
-}
-
-// LDS layout of a tile: rows of T words. Several rows (T < 4096) get one word
-// of padding each so lanes walking down a column hit distinct banks; within a
-// row of at least 256 words the low 4 index bits are XOR-ed with bits 4..7, so
-// the last round (lanes 16 words apart) is spread over the banks too.
-template <int T>
-__host__ __device__ constexpr int row_stride() {
-    return T >= kTile ? T : T + 1;
-}
-template <int T>
-__device__ __forceinline__ int swz(int r) {
-    return T >= 256 ? (r ^ ((r >> 4) & 15)) : r;
-}
-
-// Round split of LOGT stages into chunks of at most MAXR (4: radix-16 units of
-// 256-thread blocks; 3: radix-8 units of 512-thread blocks).
-__host__ __device__ constexpr int n_rounds(int logt, int maxr) { return (logt + maxr - 1) / maxr; }
-__host__ __device__ constexpr int round_len(int logt, int r, int maxr) {
-    // distribute as evenly as possible, larger rounds first
-    return logt / n_rounds(logt, maxr) + (r < logt % n_rounds(logt, maxr) ? 1 : 0);
-}
-__host__ __device__ constexpr int round_start(int logt, int r, int maxr) {
-    int s = 0;
-    for (int i = 0; i < r; i++) s += round_len(logt, i, maxr);
-    return s;
-}
-
-// One round over the LDS tile: SUBS independent sub-transforms of size 2^LOGT
-// (row stride TP words). Sub-transform `sub` has first-stage group id
-// gbase(sub) at local stage 0.
-template <int LOGT, int R, bool FWD, int NT, typename K>
-__device__ __forceinline__ void lds_round(uint64_t *lds, int s0, uint32_t gmul, uint32_t gadd_step, uint32_t gadd0,
-                                          const K &k) {
-    constexpr int T = 1 << LOGT;
-    constexpr int SUBS = kTile / T;
-    constexpr int TP = row_stride<T>();
-    const int T0 = T >> s0;          // size of the sub-transforms at this round
-    const int ups = T0 >> R;         // units per sub-transform
-    const int units = (T >> R) * SUBS;
-    for (int w = threadIdx.x; w < units; w += NT) {
-        const int sub = w % SUBS;
-        const int w2 = w / SUBS;
-        const int kk = w2 / ups;
-        const int o = w2 - kk * ups;
-        // group id of the whole phase for this sub-transform, shifted by s0
-        uint32_t G = ((gmul + gadd0 + gadd_step * (uint32_t)sub) << s0) + (uint32_t)kk;
-        // one sub-transform of at least 64 units: the 64 lanes of a wave share kk,
-        // so G is wave-uniform and the twiddles come through scalar loads
-        if (SUBS == 1 && ups >= 64) G = __builtin_amdgcn_readfirstlane(G);
-        uint64_t *row = lds + sub * TP;
-        const int i0 = kk * T0 + o;
-        uint64_t x[1 << R];
-#pragma unroll
-        for (int l = 0; l < (1 << R); l++) x[l] = row[swz<T>(i0 + l * ups)];
-        if constexpr (FWD)
-            ct_unit<R>(x, G, k);
-        else
-            gs_unit<R>(x, G, k);
-#pragma unroll
-        for (int l = 0; l < (1 << R); l++) row[swz<T>(i0 + l * ups)] = x[l];
-    }
-}
-
-struct NoHook {
-    __device__ void operator()() const {}
-};
-
-// before_last runs (forward only) just before the last round
-template <int LOGT, bool FWD, int NT, typename K, typename H = NoHook>
-__device__ __forceinline__ void run_rounds(uint64_t *lds, uint32_t gmul, uint32_t gadd_step, uint32_t gadd0,
-                                           const K &k, H before_last = H{}) {
-    constexpr int MAXR = NT >= 512 ? 3 : 4;
-    constexpr int NR = n_rounds(LOGT, MAXR);
-    if constexpr (FWD) {
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const int R = round_len(LOGT, r, MAXR), s0 = round_start(LOGT, r, MAXR);
-            if (r == NR - 1) before_last();
-            switch (R) {
-                case 4: lds_round<LOGT, 4, true, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
-                case 3: lds_round<LOGT, 3, true, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
-                case 2: lds_round<LOGT, 2, true, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
-                default: lds_round<LOGT, 1, true, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
-            }
-            __syncthreads();
-        }
-    } else {
-#pragma unroll
-        for (int r = NR - 1; r >= 0; r--) {
-            const int R = round_len(LOGT, r, MAXR), s0 = round_start(LOGT, r, MAXR);
-            switch (R) {
-                case 4: lds_round<LOGT, 4, false, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
-                case 3: lds_round<LOGT, 3, false, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
-                case 2: lds_round<LOGT, 2, false, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
-                default: lds_round<LOGT, 1, false, NT>(lds, s0, gmul, gadd_step, gadd0, k); break;
-            }
-            __syncthreads();
-        }
+        for (int l = 0; l < (1 << R); l++)
+            if ((l & h) == 0) k.inv(x[l], x[l + h], tw((1 << u) - 1 + (l >> (R - u))));
+        k.template after_inv<R>(x, u);
     }
 }
 
@@ -356,252 +238,329 @@ struct NttIO {
     const double2 *fft;       // IO_ENCODE: [n_polys][N/2]
 };
 
-// Phase A (columns, first log N1 stages, log N1 <= 5). Each thread owns one
-// column {c + N2 r} and runs all its stages in registers: no LDS, no barrier;
-// the 256 threads of a block read and write 256 consecutive words per row.
-// FWD: forward stages 0..logN1-1 (output stays lazy).
-// !FWD: inverse stages logN1-1..0, then x N^-1, output canonical.
-// At most 80 VGPRs (6 waves per SIMD): the inverse form would otherwise take 99. The
-// encoder's form keeps its registers (it would spill).
-template <int LOGT, bool FWD, int IO, int A>
-__global__ __launch_bounds__(kThreads, IO == IO_ENCODE ? 1 : 6) void k_ntt_cols(uint64_t *__restrict__ data, LimbMap mp, NttTables tb,
-                                                       int logN, NttIO io) {
-    constexpr int T = 1 << LOGT;
-    const size_t N = size_t(1) << logN;
-    const size_t N2 = N >> LOGT;
-    const uint32_t groups = (uint32_t)(N2 / kThreads);
-    const uint32_t z = blockIdx.x / groups;
-    const size_t c = (size_t)(blockIdx.x % groups) * kThreads + threadIdx.x;
-    uint32_t poly, k, prime;
-    limb_of(mp, z, poly, k, prime);
-    uint64_t *base = data + poly * mp.poly_stride + (size_t)k * N + c;
-    // every column's group id at stage 0 is 1 (phase A starts at s = 0)
-    {
-        const uint64_t q = tb.mods[prime].q;
-        uint64_t x[T];
+// Column pass, log N1 = RA + RB stages. A block takes C columns (consecutive words of a
+// row of 512) with all their N1 words. Round 1 (RA stages) runs on register units of words
+// 2^RB rows apart, its twiddles the same for every column (scalar loads); with RB > 0 the
+// block then exchanges through LDS once and round 2 (RB stages) runs on 2^RB adjacent rows.
+// 32 columns (16 for RB = 4) keep each access a run of 256 (128) bytes and the block at 16
+// to 32 KB of LDS, five or more blocks a CU. Memory bounds the pass: 1.61 GB in 294 us (5.5
+// TB/s); 64 columns and 512 threads measured 287 us forward and 324 us inverse against 294
+// and 305 us.
+constexpr int col_width(int ra, int rb) { return rb == 0 ? kThreads : kThreads >> rb; }
+
+template <int RA, int RB, bool FWD, int IO, typename K>
+__device__ __forceinline__ void col_pass(const K &k, uint64_t *lds, uint64_t *base, const u32x4 *__restrict__ col,
+                                         uint32_t c0, const NttTables &tb, uint32_t prime, uint32_t poly, size_t N,
+                                         const NttIO &io) {
+    constexpr int C = col_width(RA, RB);
+    constexpr int UNITS = RB == 0 ? 1 : (C << RA) / kThreads;  // round-2 units per thread
+    const uint32_t cl = threadIdx.x % C, c = c0 + cl;
+    const uint32_t r0 = RB == 0 ? 0 : threadIdx.x / C;         // round 1: rows r0 + l 2^RB
+    auto tw1 = [&](int e) { return col[e + 1]; };
+    uint64_t x[1 << RA];
+    // round 2 on unit m: rows g 2^RB + l, g = threadIdx / C + m 256 / C
+    auto round2 = [&](auto body) {
+        if constexpr (RB > 0) {
+#pragma unroll
+            for (int m = 0; m < UNITS; m++) {
+                const uint32_t g = threadIdx.x / C + m * (kThreads / C);
+                auto tw2 = [&](int e) {
+                    const int u = e >= 7 ? 3 : e >= 3 ? 2 : e >= 1 ? 1 : 0;
+                    return col[(((1u << RA) + g) << u) + (uint32_t)(e - ((1 << u) - 1))];
+                };
+                body(g, tw2);
+            }
+        }
+    };
+    if constexpr (FWD) {
         if (IO == IO_REDUCE) {
             const DevMod m = tb.mods[prime];
             const uint64_t *src = io.src + (size_t)poly * N + c;
 #pragma unroll
-            for (int r = 0; r < T; r++) {
-                const uint64_t v = src[r * N2];
-                if (A == FOLD) {  // signed words need no reduction
-                    x[r] = io.center && v > io.center ? v - (2 * io.center + 1) : v;
-                    continue;
-                }
-                uint64_t y = reduce64(v, m);
-                if (io.center && v > io.center) y = sub_mod(y, reduce64(2 * io.center + 1, m), m.q);
-                x[r] = y;
-            }
+            for (int l = 0; l < (1 << RA); l++)
+                x[l] = k.load_residue(src[(size_t)(r0 + (l << RB)) * kRow], io.center, m);
         } else if (IO == IO_ENCODE) {
             const DevMod m = tb.mods[prime];
             const double2 *fb = io.fft + (size_t)poly * (N / 2) + c;
-            // rows r < T/2 lie below N/2 (real parts), row r + T/2 is the
-            // imaginary part of the same entry
+            // rows below N1/2 are real parts; row r + N1/2 is the imaginary part of the same entry
 #pragma unroll
-            for (int r = 0; r < T / 2; r++) {
-                const double2 v = fb[r * N2];
-                x[r] = residue_of_rounded(round(v.x), m);
-                x[r + T / 2] = residue_of_rounded(round(v.y), m);
+            for (int l = 0; l < (1 << RA) / 2; l++) {
+                const double2 v = fb[(size_t)(r0 + (l << RB)) * kRow];
+                x[l] = k.load_rounded(round(v.x), m);
+                x[l + (1 << RA) / 2] = k.load_rounded(round(v.y), m);
             }
         } else {
 #pragma unroll
-            for (int r = 0; r < T; r++) x[r] = base[r * N2];
+            for (int l = 0; l < (1 << RA); l++) x[l] = base[(size_t)(r0 + (l << RB)) * kRow + c];
         }
-        const auto ar = arith_of<A>(tb, prime, N);
-        if constexpr (FWD) {
-            ct_unit<LOGT>(x, 1u, ar);
-            // streaming store: the tile pass reads these words back long after
+        ct_unit<RA>(x, k, tw1);
+        if constexpr (RB == 0) {
 #pragma unroll
-            for (int r = 0; r < T; r++) __builtin_nontemporal_store(x[r], &base[r * N2]);
+            for (int l = 0; l < (1 << RA); l++) __builtin_nontemporal_store(x[l], &base[(size_t)l * kRow + c]);
         } else {
-            gs_unit<LOGT>(x, 1u, ar);
-            const uint64_t ni = tb.ninv[prime], nis = tb.ninv_s[prime];
-            if constexpr (A == FOLD) {
-                const u32x4 nf = fold_split(ni, nis, q, ar.f);
 #pragma unroll
-                for (int r = 0; r < T; r++)
-                    __builtin_nontemporal_store(fold_canon(fold_mul(x[r], nf, ar.f), q, ar.f), &base[r * N2]);
-            } else {
+            for (int l = 0; l < (1 << RA); l++) lds[(r0 + (l << RB)) * C + cl] = x[l];
+            __syncthreads();
+            round2([&](uint32_t g, auto tw2) {
+                uint64_t y[1 << RB];
 #pragma unroll
-                for (int r = 0; r < T; r++) __builtin_nontemporal_store(mul_shoup(x[r], ni, nis, q), &base[r * N2]);
-            }
+                for (int l = 0; l < (1 << RB); l++) y[l] = lds[((g << RB) + l) * C + cl];
+                ct_unit<RB>(y, k, tw2);
+                // streaming store: the row pass reads these words back long after
+#pragma unroll
+                for (int l = 0; l < (1 << RB); l++)
+                    __builtin_nontemporal_store(y[l], &base[(size_t)((g << RB) + l) * kRow + c]);
+            });
         }
+    } else {
+        if constexpr (RB == 0) {
+#pragma unroll
+            for (int l = 0; l < (1 << RA); l++) x[l] = base[(size_t)l * kRow + c];
+        } else {
+            round2([&](uint32_t g, auto tw2) {
+                uint64_t y[1 << RB];
+#pragma unroll
+                for (int l = 0; l < (1 << RB); l++) y[l] = base[(size_t)((g << RB) + l) * kRow + c];
+                gs_unit<RB>(y, k, tw2);
+#pragma unroll
+                for (int l = 0; l < (1 << RB); l++) lds[((g << RB) + l) * C + cl] = y[l];
+            });
+            __syncthreads();
+#pragma unroll
+            for (int l = 0; l < (1 << RA); l++) x[l] = lds[(r0 + (l << RB)) * C + cl];
+        }
+        gs_unit<RA>(x, k, tw1);
+        const auto ni = k.constant(tb.ninv[prime], tb.ninv_s[prime]);
+#pragma unroll
+        for (int l = 0; l < (1 << RA); l++)
+            __builtin_nontemporal_store(k.mul(x[l], ni), &base[(size_t)(r0 + (l << RB)) * kRow + c]);
     }
 }
 
-// Phase B (contiguous blocks of N2, last log N2 stages). LOGT = log N2.
-// FWD: input lazy, output canonical. !FWD: input canonical (< 2q accepted),
-// output lazy.
-// Work order: workgroups are dispatched to the 8 XCDs round-robin, so block b
-// runs on XCD b % 8. Each XCD takes a contiguous range of the work index
-// O = (limb * tiles + tile) * n_polys + poly: the polynomials that share one
-// prime and tile (hence one twiddle slice) run back to back on the same L2.
-// 512-thread blocks ask for 6 waves per SIMD (80 VGPRs), three 32 KB tiles per CU.
-template <int LOGT, bool FWD, int IO, int A, int NT = kThreads>
-__global__ __launch_bounds__(NT, NT >= 512 ? 6 : 1) void k_ntt_blocks(uint64_t *__restrict__ data, LimbMap mp, NttTables tb,
-                                                         int logN, NttIO io, uint32_t n_polys, uint32_t per_xcd) {
-    constexpr int T = 1 << LOGT;
-    constexpr int BLKS = kTile / T;
-    constexpr int TP = row_stride<T>();
-    __shared__ __align__(16) uint64_t lds[BLKS * TP];
+template <int RA, int RB, bool FWD, int IO, bool FAST>
+__global__ __launch_bounds__(kThreads) void k_ntt_cols(uint64_t *__restrict__ data, LimbMap mp, NttTables tb, int logN,
+                                                       NttIO io) {
+    constexpr int C = col_width(RA, RB);
+    __shared__ uint64_t lds[RB == 0 ? 1 : C << (RA + RB)];
     const size_t N = size_t(1) << logN;
-    const uint32_t tiles = (uint32_t)(N / kTile);
-    const uint32_t O = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
-    if (O >= n_polys * mp.n_active * tiles) return;  // whole block, before any barrier
-    const uint32_t pz = O % n_polys, rest = O / n_polys;
-    const uint32_t z = pz * mp.n_active + rest / tiles;
-    const int t0 = (int)(rest % tiles) * kTile;
+    const uint32_t z = blockIdx.x / (kRow / C);
+    const uint32_t c0 = (blockIdx.x % (kRow / C)) * C;
     uint32_t poly, k, prime;
     limb_of(mp, z, poly, k, prime);
-    uint64_t *base = data + poly * mp.poly_stride + (size_t)k * N + t0;
-    // block b (global index t0/T + b) has group id N1 + b at its first stage
-    const uint32_t N1 = (uint32_t)(N >> LOGT);
-    const uint64_t q = tb.mods[prime].q, q2 = q << 1;
-    const uint64_t *ld = IO == IO_GATHER ? io.acc_p.p[poly] + (size_t)k * N + t0 : base;
-    // LDS slot of tile word i
-    auto slot = [](int i) { return (i / T) * TP + swz<T>(i % T); };
-    // Word pair (i, i + 1), i even, to and from LDS. In a full-width tile the
-    // swizzle keeps the pair in one aligned 16-byte slot, swapped when bit 4 of i
-    // is set, so a lane moves it with one 16-byte LDS access (a wave covers 1 KB
-    // of consecutive slots: no bank conflicts).
-    auto lds_put = [&](int i, u64x2 v) {
-        if (T >= kTile) {
-            const bool sw = (i >> 4) & 1;
-            u64x2 o;
-            o.x = sw ? v.y : v.x;
-            o.y = sw ? v.x : v.y;
-            *reinterpret_cast<u64x2 *>(&lds[swz<T>(i) & ~1]) = o;
-        } else {
-            lds[slot(i)] = v.x;
-            lds[slot(i + 1)] = v.y;
-        }
-    };
-    auto lds_get = [&](int i) -> u64x2 {
-        u64x2 v;
-        if (T >= kTile) {
-            const bool sw = (i >> 4) & 1;
-            const u64x2 o = *reinterpret_cast<const u64x2 *>(&lds[swz<T>(i) & ~1]);
-            v.x = sw ? o.y : o.x;
-            v.y = sw ? o.x : o.y;
-        } else {
-            v.x = lds[slot(i)];
-            v.y = lds[slot(i + 1)];
-        }
-        return v;
-    };
-    // the tile comes in two words per lane (16-byte loads; the launcher checks the
-    // alignment). Plain outputs leave one word per lane: 16-byte stores measured slower.
-    constexpr int PAIRS = kTile / (2 * NT);  // pairs per lane
-#pragma unroll
-    for (int j = 0; j < PAIRS; j++) {
-        const int i = 2 * (threadIdx.x + j * NT);
-        lds_put(i, __builtin_nontemporal_load(reinterpret_cast<const u64x2 *>(ld + i)));
+    uint64_t *base = data + poly * mp.poly_stride + (size_t)k * N;
+    const u32x4 *col = tb.col + (size_t)prime * kNttCols;
+    if constexpr (FAST) {
+        col_pass<RA, RB, FWD, IO>(FoldK<false>(tb, prime), lds, base, col, c0, tb, prime, poly, N, io);
+    } else {
+        if (tb.fold[prime].pw)
+            col_pass<RA, RB, FWD, IO>(FoldK<true>(tb, prime), lds, base, col, c0, tb, prime, poly, N, io);
+        else
+            col_pass<RA, RB, FWD, IO>(HarveyK(tb, prime), lds, base, col, c0, tb, prime, poly, N, io);
     }
-    // rescale: the accumulator words are loaded before the last round, so they
-    // arrive during it (loading them before all rounds cost occupancy)
-    constexpr int PER = kTile / NT;
+}
+
+// LDS word of row word i. Each round's accesses of a unit differ by constants (8 words of a
+// lane lie 64, 8 or 1 apart), and lanes a row apart by 8 words fall 9 apart: 32 lanes reach
+// 32 banks in every round.
+__device__ __forceinline__ int row_slot(int i) { return i + (i >> 3); }
+
+// Orders a wave's own LDS writes before its later reads of them (a wave's LDS accesses
+// execute in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Row pass: one wave per row of 512 words, 8 words per lane. Unit words of a lane: round 1
+// lane + 64 l; round 2 64 (lane / 8) + lane % 8 + 8 l; round 3 8 lane + l.
+template <bool FWD, int IO, typename K>
+__device__ __forceinline__ void row_pass(const K &k, uint64_t *lds, uint64_t *base, const u32x4 *__restrict__ tw,
+                                         const u32x4 *w2, const u32x4 (&w3)[7], uint64_t (&x)[8],
+                                         const NttTables &tb, uint32_t prime, uint32_t poly, uint32_t limb,
+                                         uint32_t row0, uint32_t n_active, size_t N, int lane, const NttIO &io,
+                                         const typename K::Const &qi) {
+    const int i1 = row_slot(lane), i2 = row_slot(64 * (lane >> 3) + (lane & 7)), i3 = 9 * lane;
+    auto tw1 = [&](int e) { return w2[e]; };
+    auto tw2 = [&](int e) { return w2[8 + 8 * e + (lane >> 3)]; };
+    auto tw3 = [&](int e) { return w3[e]; };
+    auto put1 = [&](const uint64_t *x) {
+#pragma unroll
+        for (int l = 0; l < 8; l++) lds[i1 + 72 * l] = x[l];
+    };
+    auto put2 = [&](const uint64_t *x) {
+#pragma unroll
+        for (int l = 0; l < 8; l++) lds[i2 + 9 * l] = x[l];
+    };
+    auto put3 = [&](const uint64_t *x) {
+#pragma unroll
+        for (int l = 0; l < 8; l++) lds[i3 + l] = x[l];
+    };
+    auto get1 = [&](uint64_t *x) {
+        wave_lds_order();
+#pragma unroll
+        for (int l = 0; l < 8; l++) x[l] = lds[i1 + 72 * l];
+    };
+    auto get2 = [&](uint64_t *x) {
+        wave_lds_order();
+#pragma unroll
+        for (int l = 0; l < 8; l++) x[l] = lds[i2 + 9 * l];
+    };
+    auto get3 = [&](uint64_t *x) {
+        wave_lds_order();
+#pragma unroll
+        for (int l = 0; l < 8; l++) x[l] = lds[i3 + l];
+    };
+    if constexpr (!FWD) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int i = 2 * lane + 128 * j;
+            lds[row_slot(i)] = x[2 * j];
+            lds[row_slot(i) + 1] = x[2 * j + 1];
+        }
+        get3(x);
+        gs_unit<3>(x, k, tw3);
+        wave_lds_order();
+        put3(x);
+        get2(x);
+        gs_unit<3>(x, k, tw2);
+        wave_lds_order();
+        put2(x);
+        get1(x);
+        gs_unit<3>(x, k, tw1);
+#pragma unroll
+        for (int l = 0; l < 8; l++) base[lane + 64 * l] = x[l];
+        return;
+    }
+    ct_unit<3>(x, k, tw1);
+    put1(x);
+    get2(x);
+    ct_unit<3>(x, k, tw2);
+    wave_lds_order();
+    put2(x);
+    // rescale: the accumulator words are loaded before the last round, so they arrive during
+    // it; outputs leave in 16-byte pairs
     const uint64_t *accp = nullptr;
-    uint64_t *out = nullptr;
-    if (FWD && IO == IO_RESCALE) {
-        accp = io.packed ? io.acc_p.p[poly] + (size_t)k * N + t0
-                         : io.acc + ((size_t)poly * io.acc_limbs + k) * N + t0;
+    uint64_t *out = base;
+    if (IO == IO_RESCALE) {
+        accp = io.packed ? io.acc_p.p[poly] + (size_t)limb * N + row0
+                         : io.acc + ((size_t)poly * io.acc_limbs + limb) * N + row0;
         if (io.packed || io.out_packed) {
-            out = io.out_p.p[poly] + (size_t)k * N + t0;
+            out = io.out_p.p[poly] + (size_t)limb * N + row0;
         } else {
             uint64_t *ob = io.outs ? io.outs[poly / io.ppo] : io.out_single;
-            out = ob + ((size_t)(poly % io.ppo) * (io.out_limbs ? io.out_limbs : mp.n_active) + k) * N + t0;
+            out = ob + ((size_t)(poly % io.ppo) * (io.out_limbs ? io.out_limbs : n_active) + limb) * N + row0;
         }
     }
-    // accumulator and output in 16-byte pairs when both are aligned (block-uniform);
-    // lane word j is then tile word 2 (tid + (j / 2) NT) + j % 2, else tid + j NT
-    const bool vec = (((uintptr_t)accp | (uintptr_t)out) & 15) == 0;
-    auto word_of = [&](int j) {
-        return vec ? 2 * ((int)threadIdx.x + (j >> 1) * NT) + (j & 1) : (int)threadIdx.x + j * NT;
-    };
-    uint64_t accv[IO == IO_RESCALE ? PER : 1];
-    auto load_acc = [&] {
-        if (FWD && IO == IO_RESCALE) {
-            if (vec) {
+    auto pair_of = [&](int j) { return 2 * lane + 128 * j; };  // words i, i + 1
+    u64x2 accv[IO == IO_RESCALE ? 4 : 1];
+    if (IO == IO_RESCALE) {
 #pragma unroll
-                for (int j = 0; j < PER; j += 2) {
-                    const u64x2 v = __builtin_nontemporal_load(global_ptr(reinterpret_cast<const u64x2 *>(accp + word_of(j))));
-                    accv[j] = v.x;
-                    accv[j + 1] = v.y;
+        for (int j = 0; j < 4; j++)
+            accv[j] = __builtin_nontemporal_load(global_ptr(reinterpret_cast<const u64x2 *>(accp + pair_of(j))));
+    }
+    get3(x);
+    ct_unit<3>(x, k, tw3);
+    wave_lds_order();
+    put3(x);
+    wave_lds_order();
+    const bool addto = IO == IO_RESCALE && io.out_packed && poly < 64 && ((io.acc_mask >> poly) & 1);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = pair_of(j);
+        u64x2 y = {lds[row_slot(i)], lds[row_slot(i) + 1]};
+        if (IO == IO_RESCALE) {
+            y.x = k.sub_mul(accv[j].x, y.x, qi);
+            y.y = k.sub_mul(accv[j].y, y.y, qi);
+            if (addto) {
+                u64x2 o;
+                if (io.add_perm) {
+                    const auto src = global_ptr(io.add_src.p[poly] + (size_t)limb * N);
+                    const auto at = global_ptr(io.add_perm + row0 + i);
+                    o = u64x2{src[at[0]], src[at[1]]};
+                } else {
+                    o = *global_ptr(reinterpret_cast<const u64x2 *>(out + i));
                 }
-            } else {
-#pragma unroll
-                for (int j = 0; j < PER; j++) accv[j] = *global_ptr(accp + word_of(j));
-            }
-        }
-    };
-    __syncthreads();
-    const auto ar = arith_of<A>(tb, prime, N);
-    run_rounds<LOGT, FWD, NT>(lds, N1, 1u, (uint32_t)(t0 / T), ar, load_acc);
-    // canonical residue of a forward output: below 4q, below (4 + 4 log N) q when lazy,
-    // signed when folded
-    auto canon = [&](uint64_t v) -> uint64_t {
-        if constexpr (A == FOLD) return fold_canon(v, q, ar.f);
-        if (A == LAZY) return reduce64(v, tb.mods[prime]);
-        v = v >= q2 ? v - q2 : v;
-        return v >= q ? v - q : v;
-    };
-    if (FWD && IO == IO_RESCALE) {
-        const uint64_t qi = io.qinv[prime], qis = io.qinv_s[prime];
-        // unreduced outputs stay below (4 + 4 logN) q (< 2^64 for the lazy primes): acc - v
-        // is taken as acc + (4 + 4 logN) q - v, which the Shoup product accepts as it is
-        const uint64_t kq = (uint64_t)(4 + 4 * logN) * q;
-        const bool addto = io.out_packed && poly < 64 && ((io.acc_mask >> poly) & 1);
-        u32x4 qf = {0, 0, 0, 0};
-        if constexpr (A == FOLD) qf = fold_split(qi, qis, q, ar.f);
-        auto result = [&](uint64_t acc, uint64_t raw) -> uint64_t {
-            if constexpr (A == FOLD) return fold_canon(fold_mul(acc - raw, qf, ar.f), q, ar.f);
-            return A == LAZY ? mul_shoup(acc + kq - raw, qi, qis, q) : mul_shoup(sub_mod(acc, canon(raw), q), qi, qis, q);
-        };
-        auto addend = [&](int i) -> uint64_t {
-            return *global_ptr(io.add_src.p[poly] + (size_t)k * N + io.add_perm[t0 + i]);
-        };
-        if (vec) {
-#pragma unroll
-            for (int j = 0; j < PER; j += 2) {
-                const int i = word_of(j);
-                const u64x2 raw = lds_get(i);
-                u64x2 y;
-                y.x = result(accv[j], raw.x);
-                y.y = result(accv[j + 1], raw.y);
-                if (addto) {
-                    if (io.add_perm) {
-                        y.x = add_mod(y.x, addend(i), q);
-                        y.y = add_mod(y.y, addend(i + 1), q);
-                    } else {
-                        const u64x2 o = *global_ptr(reinterpret_cast<const u64x2 *>(out + i));
-                        y.x = add_mod(y.x, o.x, q);
-                        y.y = add_mod(y.y, o.y, q);
-                    }
-                }
-                __builtin_nontemporal_store(y, global_ptr(reinterpret_cast<u64x2 *>(out + i)));
+                y.x = add_mod(y.x, o.x, k.q);
+                y.y = add_mod(y.y, o.y, k.q);
             }
         } else {
+            y.x = k.canon(y.x);
+            y.y = k.canon(y.y);
+        }
+        __builtin_nontemporal_store(y, global_ptr(reinterpret_cast<u64x2 *>(out + i)));
+    }
+}
+
+// One wave per row and up to `chunk` polynomials of one prime: the row's twiddles are loaded
+// once (round 3 into registers, rounds 1 and 2 into LDS), and the next polynomial's words are
+// requested before the current one's stages. 118 VGPRs, 4 waves per SIMD: the prefetch and
+// the shared twiddles (a row's twiddles are twice its data) gave more than 8 waves did.
+// Work order: workgroups are dispatched to the 8 XCDs round-robin, so block
+// b runs on XCD b % 8. Each XCD takes a contiguous range of blocks' row indices
+// O = (limb * rows + row) * chunks + chunk: the polynomials that share one prime and row
+// (hence one run of twiddles) run back to back on the same L2.
+template <bool FWD, int IO, bool FAST, int NT>
+__global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data, LimbMap mp, NttTables tb, int logN,
+                                                 NttIO io, uint32_t n_polys, uint32_t per_xcd, uint32_t chunk) {
+    __shared__ uint64_t lds[NT / 64][kRowLds];
+    const size_t N = size_t(1) << logN;
+    const uint32_t rows = (uint32_t)(N / kRow);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t O = ((blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3)) * (NT / 64) + wave;
+    if (O >= (n_polys + chunk - 1) / chunk * mp.n_active * rows) return;  // no barrier in this kernel
+    const uint32_t chunks = (n_polys + chunk - 1) / chunk;
+    const uint32_t ch = O % chunks, rest = O / chunks;
+    const uint32_t p0 = ch * chunk, p1 = min(p0 + chunk, n_polys);
+    const uint32_t row = rest % rows;
+    uint32_t poly0, limb, prime;
+    limb_of(mp, rest / rows, poly0, limb, prime);  // limb of the first polynomial
+    const uint32_t row0 = row * kRow;
+    const u32x4 *tw = tb.row + (size_t)prime * N + row0;
+    auto src_of = [&](uint32_t p) -> const uint64_t * {
+        return IO == IO_GATHER ? io.acc_p.p[p] + (size_t)limb * N + row0
+                               : data + p * mp.poly_stride + (size_t)limb * N + row0;
+    };
+    auto load = [&](uint64_t (&x)[8], uint32_t p) {
+        const uint64_t *ld = src_of(p);
+        if constexpr (FWD) {
 #pragma unroll
-            for (int j = 0; j < PER; j++) {
-                const int i = word_of(j);
-                uint64_t y = result(accv[j], lds[slot(i)]);
-                if (addto) y = add_mod(y, io.add_perm ? addend(i) : *global_ptr(out + i), q);
-                __builtin_nontemporal_store(y, global_ptr(out + i));
+            for (int l = 0; l < 8; l++) x[l] = __builtin_nontemporal_load(global_ptr(ld + lane + 64 * l));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const u64x2 v = __builtin_nontemporal_load(global_ptr(reinterpret_cast<const u64x2 *>(ld + 2 * lane + 128 * j)));
+                x[2 * j] = v.x;
+                x[2 * j + 1] = v.y;
             }
         }
-    } else if (FWD) {
+    };
+    uint64_t x[8], nx[8];
+    load(x, p0);
+    __shared__ __align__(16) u32x4 lds2[NT / 64][64];
+    u32x4 *w2 = lds2[wave];
+    u32x4 w3[7];
+    w2[lane] = tw[lane];
 #pragma unroll
-        for (int j = 0; j < kTile / NT; j++) {
-            const int i = threadIdx.x + j * NT;
-            __builtin_nontemporal_store(canon(lds[slot(i)]), &base[i]);
+    for (int e = 0; e < 7; e++) w3[e] = tw[64 + 64 * e + lane];
+    wave_lds_order();
+    auto loop = [&](const auto &k) {
+        const auto qi = IO == IO_RESCALE ? k.constant(io.qinv[prime], io.qinv_s[prime]) : k.constant(0, 0);
+        for (uint32_t p = p0; p < p1; p++) {
+            if (p + 1 < p1) load(nx, p + 1);
+            uint64_t *base = data + p * mp.poly_stride + (size_t)limb * N + row0;
+            row_pass<FWD, IO>(k, lds[wave], base, tw, w2, w3, x, tb, prime, p, limb, row0, mp.n_active, N, lane, io, qi);
+            wave_lds_order();
+#pragma unroll
+            for (int l = 0; l < 8; l++) x[l] = nx[l];
         }
+    };
+    if constexpr (FAST) {
+        loop(FoldK<false>(tb, prime));
     } else {
-#pragma unroll
-        for (int j = 0; j < kTile / NT; j++) {
-            const int i = threadIdx.x + j * NT;
-            base[i] = lds[slot(i)];
-        }
+        if (tb.fold[prime].pw)
+            loop(FoldK<true>(tb, prime));
+        else
+            loop(HarveyK(tb, prime));
     }
 }
 
@@ -626,104 +585,88 @@ template <bool FWD, int IOA, int IOB>
 void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t total_limbs, hipStream_t s,
                 const NttIO &io = NttIO{}) {
     if (total_limbs == 0) return;
-    if (c.N < (size_t)kTile) throw InvalidArgument("NTT requires N >= 4096");
+    if (c.N < (size_t)4096) throw InvalidArgument("NTT requires N >= 4096");
     if (total_limbs % mp.n_active != 0) throw LogicError("NTT limb count is not a multiple of the polynomial size");
     const int logN = c.logN;
-    // Phase B takes whole 4096-word tiles (12 stages) and phase A the rest:
-    // with few column stages, phase A moves rows of >= 2 KB contiguous words
-    // (N >> log1 >= 4096 / 2^log1 columns of a tile) instead of short strided
-    // segments.
-    const int log2b = std::min(12, logN - 4);
-    const int log1 = logN - log2b;
     const size_t N = c.N;
-    const unsigned grid_cols = (unsigned)(total_limbs * ((N >> log1) / kThreads));
+    const int stages = logN - 9;                       // of the column pass
+    const int unit = stages == 4 || stages >= 7 ? 4 : 3;  // of its longest unit
     const uint32_t n_polys = (uint32_t)(total_limbs / mp.n_active);
-    const uint32_t per_xcd = (uint32_t)((total_limbs * (N / kTile) + 7) / 8);
-    const unsigned grid_blk = 8u * per_xcd;
     NttTables tb{c.mods(),
-                 FWD ? c.tw.as<uint64_t>() : c.itw.as<uint64_t>(),
-                 FWD ? c.tw_s.as<uint64_t>() : c.itw_s.as<uint64_t>(),
+                 c.d_fold.as<FoldMod>(),
+                 FWD ? c.tw_col.as<u32x4>() : c.itw_col.as<u32x4>(),
+                 FWD ? c.tw_row.as<u32x4>() : c.itw_row.as<u32x4>(),
                  c.ninv.as<uint64_t>(),
-                 c.ninv_s.as<uint64_t>(),
-                 FWD ? c.tw_f.as<u32x4>() : c.itw_f.as<u32x4>(),
-                 c.d_fold.as<FoldMod>()};
-    // tile passes in 512-thread blocks of radix-8 rounds (the default): the lazy forward
-    // passes and the inverse ones; the forward passes of primes above the lazy bound keep
-    // 256-thread radix-16 rounds (their fused form would spill at 80 registers)
-    const bool tile512 = ks_tuning().ntt_tile_threads == 512;
-    // Split products when every prime of the launch has them and the signed words cannot
-    // overflow: forward, input (below 4q, or a residue of another prime of the context)
-    // plus log N products plus the fused epilogue's operand; inverse, the sums of one unit.
-    // Otherwise forward butterflies leave a unreduced when (5 + 4 log N) q < 2^64 for every
-    // prime: values below (4 + 4 log N) q, plus one q of the fused epilogue's operand.
-    bool lazy = FWD, fold = true;
-    const uint64_t lazy_max = ~uint64_t(0) / (uint64_t)(5 + 4 * c.logN);
+                 c.ninv_s.as<uint64_t>()};
+    // FAST when every prime of the launch has a split form and the signed words cannot
+    // overflow: forward, input (below 4q, or a residue of another prime of the context, or an
+    // encoder's coefficient) plus log N products plus the fused epilogue's operand; inverse,
+    // the sums of one unit, which start from products or folded words.
+    bool fast = true;
     const uint64_t q_any = *std::max_element(c.q.begin(), c.q.end());
-    for (uint32_t j = 0; j < mp.n_active && (lazy || fold); j++) {
+    for (uint32_t j = 0; j < mp.n_active && fast; j++) {
         uint32_t k = mp.lo + j;
         if (k >= mp.skip_lo) k += mp.skip_width;
         const uint32_t prime = k < mp.Ql ? mp.first_prime + k : mp.nQ + (k - mp.Ql);
         const uint64_t q = c.q.at(prime), r = c.fold_bound.at(prime);
-        lazy = lazy && q < lazy_max;
         const uint64_t in = IOA == IO_REDUCE ? std::max(q_any, 4 * q) : 4 * q;
         const uint64_t top = (uint64_t(1) << 63) - 1 - 2 * q;
-        fold = fold && r != 0 && (FWD ? in < top && r <= (top - in) / (uint64_t)c.logN
-                                       : r < (uint64_t(1) << (63 - std::max(log1, tile512 ? 3 : 4))));
+        fast = r != 0 && !c.fold_twice.at(prime) && (FWD ? in < top && r <= (top - in) / (uint64_t)logN
+                              : r < (uint64_t(1) << (63 - std::max(unit, 3))));
     }
-    const int arith = fold ? FOLD : lazy ? LAZY : HARVEY;
-    // the tile pass reads its input in 16-byte pairs of words
+    // the row pass moves its words in 16-byte pairs (outs are ciphertext buffers of the pool)
     bool aligned = ((uintptr_t)data & 15) == 0 && mp.poly_stride % 2 == 0;
     if (IOB == IO_GATHER)
         for (uint32_t p = 0; p < n_polys; p++) aligned = aligned && ((uintptr_t)io.acc_p.p[p] & 15) == 0;
+    if (IOB == IO_RESCALE) {
+        aligned = aligned && (((uintptr_t)io.acc | (uintptr_t)io.out_single) & 15) == 0;
+        for (uint32_t p = 0; p < n_polys && (io.packed || io.out_packed); p++)
+            aligned = aligned && (((uintptr_t)io.out_p.p[p] | (io.packed ? (uintptr_t)io.acc_p.p[p] : 0)) & 15) == 0;
+    }
     if (!aligned) throw InvalidArgument("NTT operands must be 16-byte aligned");
-#define SHM_COLS_A(L, A) k_ntt_cols<L, FWD, IOA, A><<<grid_cols, kThreads, 0, s>>>(data, mp, tb, logN, io)
-#define SHM_BLKS_A(L, A, NT) \
-    k_ntt_blocks<L, FWD, IOB, A, NT><<<grid_blk, NT, 0, s>>>(data, mp, tb, logN, io, n_polys, per_xcd)
-#define SHM_COLS(L)                                 \
-    case L:                                         \
-        if (arith == FOLD)                          \
-            SHM_COLS_A(L, FOLD);                    \
-        else if (arith == LAZY)                     \
-            SHM_COLS_A(L, (FWD ? LAZY : HARVEY));   \
-        else                                        \
-            SHM_COLS_A(L, HARVEY);                  \
-        break;
-#define SHM_BLKS(L)                                 \
-    case L:                                         \
-        if (arith == FOLD && tile512)               \
-            SHM_BLKS_A(L, FOLD, 512);               \
-        else if (arith == FOLD)                     \
-            SHM_BLKS_A(L, FOLD, 256);               \
-        else if (arith == LAZY && tile512)          \
-            SHM_BLKS_A(L, (FWD ? LAZY : HARVEY), 512); \
-        else if (arith == LAZY)                     \
-            SHM_BLKS_A(L, (FWD ? LAZY : HARVEY), 256); \
-        else if (!FWD && tile512)                   \
-            SHM_BLKS_A(L, HARVEY, (FWD ? 256 : 512)); \
-        else                                        \
-            SHM_BLKS_A(L, HARVEY, 256);             \
-        break;
+    const int row_threads = ks_tuning().ntt_tile_threads;
+    // up to 4 polynomials per wave share a row's twiddles in registers and prefetch each
+    // other's words, while 8192 waves (8 per SIMD) remain: the plain forward pass of a
+    // shared-a chunk's launches 96 -> 75 us (8 polynomials measured the same)
+    uint32_t chunk = 1;
+    while (chunk < 4 && chunk < n_polys &&
+           (size_t)((n_polys + 2 * chunk - 1) / (2 * chunk)) * mp.n_active * (N / kRow) >= 8192)
+        chunk *= 2;
+    const size_t row_waves = (size_t)((n_polys + chunk - 1) / chunk) * mp.n_active * (N / kRow);
+    const uint32_t per_xcd = (uint32_t)((row_waves + row_threads / 64 * 8 - 1) / (row_threads / 64 * 8));
     auto cols = [&]() {
-        switch (log1) {
-            SHM_COLS(4)
-            SHM_COLS(5)
+#define SHM_COLS(S, RA, RB)                                                                            \
+    case S: {                                                                                          \
+        const unsigned grid = (unsigned)(total_limbs * (kRow / col_width(RA, RB)));                    \
+        if (fast)                                                                                      \
+            k_ntt_cols<RA, RB, FWD, IOA, true><<<grid, kThreads, 0, s>>>(data, mp, tb, logN, io);      \
+        else                                                                                           \
+            k_ntt_cols<RA, RB, FWD, IOA, false><<<grid, kThreads, 0, s>>>(data, mp, tb, logN, io);     \
+        break;                                                                                         \
+    }
+        switch (stages) {
+            SHM_COLS(3, 3, 0)
+            SHM_COLS(4, 4, 0)
+            SHM_COLS(5, 3, 2)
+            SHM_COLS(6, 3, 3)
+            SHM_COLS(7, 4, 3)
+            SHM_COLS(8, 4, 4)
             default: throw InvalidArgument("unsupported ring degree for NTT");
         }
-    };
-    auto blks = [&]() {
-        switch (log2b) {
-            SHM_BLKS(8)
-            SHM_BLKS(9)
-            SHM_BLKS(10)
-            SHM_BLKS(11)
-            SHM_BLKS(12)
-            default: throw InvalidArgument("unsupported ring degree for NTT");
-        }
-    };
 #undef SHM_COLS
-#undef SHM_BLKS
-#undef SHM_COLS_A
-#undef SHM_BLKS_A
+    };
+    auto rows = [&]() {
+#define SHM_ROWS(F, NT) k_ntt_rows<FWD, IOB, F, NT><<<8u * per_xcd, NT, 0, s>>>(data, mp, tb, logN, io, n_polys, per_xcd, chunk)
+        if (fast && row_threads == 512)
+            SHM_ROWS(true, 512);
+        else if (fast)
+            SHM_ROWS(true, 256);
+        else if (row_threads == 512)
+            SHM_ROWS(false, 512);
+        else
+            SHM_ROWS(false, 256);
+#undef SHM_ROWS
+    };
     if (FWD) {
         cols();
         const bool timed = IOB == IO_RESCALE && g_rescale_tile_ev[0] && g_rescale_tile_ev[1];
@@ -759,17 +702,52 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
             }
         }
         if (pe[0]) SHM_HIP(hipEventRecord(pe[0], s));
-        blks();
+        rows();
         if (pe[1]) SHM_HIP(hipEventRecord(pe[1], s));
         if (timed) SHM_HIP(hipEventRecord(g_rescale_tile_ev[1], s));
     } else {
-        blks();
+        rows();
         cols();
     }
     SHM_HIP(hipGetLastError());
 }
 
+// One thread per twiddle i = 1 .. N - 1 of prime blockIdx.y.
+__global__ void k_ntt_tables(const uint64_t *__restrict__ tw, const DevMod *__restrict__ mods,
+                             const FoldMod *__restrict__ fold, u32x4 *__restrict__ col, u32x4 *__restrict__ row,
+                             uint32_t N) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, p = blockIdx.y;
+    if (i == 0 || i >= N) return;
+    const DevMod m = mods[p];
+    const FoldMod f = fold[p];
+    const uint64_t w = tw[(size_t)p * N + i], ws = shoup_companion(w, m);
+    const u32x4 e = f.pw ? fold_split(w, ws, m.q, f)
+                         : u32x4{(uint32_t)w, (uint32_t)(w >> 32), (uint32_t)ws, (uint32_t)(ws >> 32)};
+    const uint32_t rows = N / kRow;
+    if (i < rows) {
+        col[(size_t)p * kNttCols + i] = e;
+        return;
+    }
+    // row stage j = 3 round + u has rows 2^j groups: group `loc` of its row, of which unit
+    // loc >> u holds entry 2^u - 1 + (loc mod 2^u)
+    const int j = (31 - __clz(i)) - (31 - __clz(rows)), r = j / 3, u = j % 3;
+    const uint32_t g = i - (rows << j), loc = g & ((1u << j) - 1);
+    const uint32_t en = (1u << u) - 1 + (loc & ((1u << u) - 1)), un = loc >> u;
+    const uint32_t at = r == 0 ? en : r == 1 ? 8 + 8 * en + un : 64 + 64 * en + un;
+    row[(size_t)p * N + (size_t)(g >> j) * kRow + at] = e;
+}
+
 }  // namespace
+
+void ntt_make_tables(const Context &c, const uint64_t *tw, DevBuf &col, DevBuf &row) {
+    const size_t QP = c.nQP();
+    col.alloc(QP * kNttCols * sizeof(u32x4));
+    row.alloc(QP * c.N * sizeof(u32x4));
+    if (c.N < 4096) return;  // the transforms refuse such rings
+    k_ntt_tables<<<dim3((unsigned)((c.N + 255) / 256), (unsigned)QP), 256>>>(
+        tw, c.mods(), c.d_fold.as<FoldMod>(), col.as<u32x4>(), row.as<u32x4>(), (uint32_t)c.N);
+    SHM_HIP(hipGetLastError());
+}
 
 void ntt_forward(const Context &c, uint64_t *data, size_t n_polys, size_t n_limbs, size_t first_prime,
                  hipStream_t s) {
