@@ -207,6 +207,25 @@ __device__ __forceinline__ u32x4 fold_split(uint64_t w, uint64_t ws, uint64_t q,
     return u32x4{(uint32_t)(w >> f.s), (uint32_t)w & m, (uint32_t)(w1 >> f.s), (uint32_t)w1 & m};
 }
 
+// Base conversions sum A <= 6 products of residues y_i by constants c_i mod p, so their
+// constants are split lower: c = h0 2^s + l0, 2^32 c mod p = h1 2^s + l1 with s = b - 27
+// (h < 2^27), which leaves room for the sums H and L of all terms in 64 bits;
+// 2^(s + 32) = 2^(b + 5) = 32 delta (mod p).
+struct ConvAcc {
+    uint64_t H, L;
+};
+__device__ __forceinline__ void conv_mac(ConvAcc &a, uint32_t yl, uint32_t yh, u32x4 c) {
+    a.H += (uint64_t)yl * c.x;
+    a.L += (uint64_t)yl * c.y;
+    a.H += (uint64_t)yh * c.z;
+    a.L += (uint64_t)yh * c.w;
+}
+// congruent to the sum, below conv_bound (context.hip)
+__device__ __forceinline__ uint64_t conv_value(const ConvAcc &a, const FoldMod &f) {
+    const uint64_t r = (uint64_t)(uint32_t)a.H * (f.pw << 3) + a.L;
+    return (uint64_t)(uint32_t)(a.H >> 32) * ((uint32_t)f.d << 5) + r;
+}
+
 // [v]_q of an integral double v with |v| < 2^128; negative v maps to q - (|v| mod q),
 // which is q itself when |v| is a multiple of q (callers reduce when they need [0, q)).
 __device__ __forceinline__ uint64_t residue_of_rounded(double v, const DevMod &m) {

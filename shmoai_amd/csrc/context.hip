@@ -134,6 +134,48 @@ bool fold_form(uint64_t q, FoldMod *f, uint64_t *bound) {
     return true;
 }
 
+// Split conversion constants (ConvAcc): out[g][k][i], i < terms, from
+// hat[g sg + k sk + i si], and out[g][k][terms] from p - dig[g n_out + k]; output k has the
+// prime of position k among QlP limbs.
+__global__ void k_conv_table(const uint64_t *__restrict__ hat, const uint64_t *__restrict__ dig,
+                             const DevMod *__restrict__ mods, const FoldMod *__restrict__ fold,
+                             u32x4 *__restrict__ out, uint32_t digits, uint32_t n_out, uint32_t terms, uint32_t sg,
+                             uint32_t sk, uint32_t si, uint32_t Ql, uint32_t nQ) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= digits * n_out * (terms + 1)) return;
+    const uint32_t i = t % (terms + 1), gk = t / (terms + 1), k = gk % n_out, g = gk / n_out;
+    const uint32_t prime = k < Ql ? k : nQ + (k - Ql);
+    const DevMod m = mods[prime];
+    const uint64_t w = i < terms ? hat[(size_t)g * sg + (size_t)k * sk + (size_t)i * si] : neg_mod(dig[gk], m.q);
+    const uint64_t w1 = mul_mod(w, uint64_t(1) << 32, m);
+    const uint32_t s = fold[prime].s + 3, mask = (1u << s) - 1;
+    out[t] = u32x4{(uint32_t)(w >> s), (uint32_t)w & mask, (uint32_t)(w1 >> s), (uint32_t)w1 & mask};
+}
+
+void conv_table(const Context &c, const DevBuf &hat, const DevBuf &dig, DevBuf &out, size_t digits, size_t n_out,
+                size_t terms, size_t sg, size_t sk, size_t si, size_t Ql) {
+    const size_t n = digits * n_out * (terms + 1);
+    out.alloc(n * sizeof(u32x4));
+    k_conv_table<<<(unsigned)((n + 255) / 256), 256>>>(hat.as<uint64_t>(), dig.as<uint64_t>(), c.mods(),
+                                                       c.d_fold.as<FoldMod>(), out.as<u32x4>(), (uint32_t)digits,
+                                                       (uint32_t)n_out, (uint32_t)terms, (uint32_t)sg, (uint32_t)sk,
+                                                       (uint32_t)si, (uint32_t)Ql, (uint32_t)c.nQ);
+    SHM_HIP(hipGetLastError());
+}
+
+// Largest value conv_value leaves of `terms` products (and the rounding term): H < 1.02
+// terms 2^59 + 2^32, so its high word times 32 delta; its low word times 2^s, s = b - 27;
+// and L < 1.02 terms 2^(32+s) + 2^(5+s).
+uint64_t conv_bound(uint64_t q, size_t terms) {
+    int b = 0;
+    while (b < 64 && (q >> b)) b++;
+    const hu128 delta = ((hu128)1 << b) - q;
+    const hu128 hi = (((hu128)terms << 27) * 102 / 100 + 2) * 32 * delta;
+    const hu128 lo = ((hu128)(terms * 102 + 200) << (b + 5)) / 100;
+    const hu128 r = hi + lo;
+    return r >> 63 ? ~uint64_t(0) : (uint64_t)r;
+}
+
 template <class T>
 void upload(DevBuf &b, const std::vector<T> &v) {
     b.alloc(std::max<size_t>(v.size() * sizeof(T), 8));
@@ -396,6 +438,15 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
         if (!fold_form(c->q[p], &fold[p], &c->fold_bound[p])) fold[p] = FoldMod{};
     for (const FoldMod &f : fold) c->fold_twice.push_back(f.twice != 0);
     upload(c->d_fold, fold);
+    // split conversion constants: 2 to 5 special primes; delta below 2^27 (32 delta in 32
+    // bits), at most 54 bits, and value plus log N products within a signed word
+    c->conv_ok = nP >= 2 && nP <= 5;
+    for (size_t p = 0; p < QP; p++) {
+        const uint64_t q = c->q[p], r = c->fold_bound[p], in = conv_bound(q, nP + 1);
+        const uint64_t top = (uint64_t(1) << 63) - 1 - 2 * q;
+        c->conv_ok = c->conv_ok && r != 0 && !c->fold_twice[p] && fold[p].d < (1 << 27) && q < (uint64_t(1) << 54) &&
+                     in < top && r <= (top - in) / (uint64_t)logN;
+    }
     {
         DevBuf t;
         upload(t, tw);
@@ -438,6 +489,16 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
     upload(c->phat_inv, phinv);
     upload(c->phat_inv_s, phinvs);
     upload(c->phat_mod, phmod);
+    std::vector<uint64_t> phn(nP), phns(nP);
+    for (size_t j = 0; j < nP; j++) {
+        const uint64_t p = c->q[nQ + j];
+        // one special prime: the conversion takes the word itself (phat_inv = 1)
+        phn[j] = h_mulmod(phinv[j], ninv[nQ + j], p);
+        phns[j] = h_shoup(phn[j], p);
+    }
+    upload(c->phat_ninv, phn);
+    upload(c->phat_ninv_s, phns);
+    if (c->conv_ok) conv_table(*c, c->phat_mod, c->pmod, c->conv_down, 1, nQ, nP, 0, nP, 1, nQ);
 
     // Per-level constants (rns.cu:63-94 rescale; rns.cu:131-186 modup).
     c->levels.resize(nQ + 1);
@@ -507,12 +568,20 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
                     bhm[i * nb + j] = h;
                 }
             }
+            std::vector<uint64_t> bhn(nb), bhns(nb);
+            for (size_t j = 0; j < nb; j++) {
+                bhn[j] = h_mulmod(bhi[j], ninv[j == 0 ? Ql - 1 : nQ + j - 1], bprime[j]);
+                bhns[j] = h_shoup(bhn[j], bprime[j]);
+            }
+            upload(L->bhat_ninv, bhn);
+            upload(L->bhat_ninv_s, bhns);
             upload(L->bhat_inv, bhi);
             upload(L->bhat_inv_s, bhis);
             upload(L->bhat_mod, bhm);
             upload(L->bmod, bm);
             upload(L->binv, bi);
             upload(L->binv_s, bis);
+            if (c->conv_ok) conv_table(*c, L->bhat_mod, L->bmod, L->conv_rescale, 1, L1, nb, 0, nb, 1, nQ);
         }
         upload(L->qlast_inv, qi);
         upload(L->qlast_inv_s, qis);
@@ -520,6 +589,15 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
         upload(L->hat_inv_s, his);
         upload(L->hat_mod, hm);
         upload(L->dig_mod, dm);
+        std::vector<uint64_t> hn(Ql), hns(Ql);
+        for (size_t i = 0; i < Ql; i++) {
+            hn[i] = h_mulmod(hi[i], ninv[i], c->q[i]);
+            hns[i] = h_shoup(hn[i], c->q[i]);
+        }
+        upload(L->hat_ninv, hn);
+        upload(L->hat_ninv_s, hns);
+        if (c->conv_ok)
+            conv_table(*c, L->hat_mod, L->dig_mod, L->conv_up, L->beta, QlP, alpha, alpha * QlP, 1, QlP, Ql);
         c->levels[Ql] = std::move(L);
     }
 

@@ -123,6 +123,8 @@ struct LevelConsts {
     DevBuf hat_inv, hat_inv_s;
     // modup: [qhat_i]_{p_k} for digit g, local i, out limb k: [beta][alpha][QlP]
     DevBuf hat_mod;
+    // hat_inv N^-1 (value, shoup): the premultiplication folded into the inverse NTT
+    DevBuf hat_ninv, hat_ninv_s;
     // modup: [D_g]_{p_k}, D_g = product of digit g's primes: [beta][QlP]
     DevBuf dig_mod;
     // ModDown merged with the rescale: basis B = {q_last, p_0 .. p_(nP-1)} (the
@@ -130,6 +132,10 @@ struct LevelConsts {
     // (value, shoup); bhat_mod[i][j] = (B/b_j) mod q_i, i < Ql-1; bmod[i] = B mod
     // q_i; binv[i] = B^-1 mod q_i (value, shoup)
     DevBuf bhat_inv, bhat_inv_s, bhat_mod, bmod, binv, binv_s;
+    DevBuf bhat_ninv, bhat_ninv_s;
+    // split constants (ConvAcc) of the conversions, u32x4 [g][k][terms + 1]: hat_mod (or
+    // bhat_mod) of each term, then -[D_g]_{p_k} (or -B): with Context::conv_ok only
+    DevBuf conv_up, conv_rescale;
 };
 
 struct Context {
@@ -154,6 +160,11 @@ struct Context {
     DevBuf pmod, pmod_s;    // P mod q_i, i < nQ
     DevBuf phat_inv, phat_inv_s;  // [nP] (P/p_j)^-1 mod p_j
     DevBuf phat_mod;        // [nQ][nP] (P/p_j) mod q_i
+    DevBuf phat_ninv, phat_ninv_s;  // phat_inv N^-1
+    DevBuf conv_down;       // ModDown's split constants [nQ][nP + 1], as LevelConsts::conv_up
+    // 2 to 5 special primes, and every prime takes split conversion constants whose sums
+    // and transforms fit (context.hip)
+    bool conv_ok = false;
     std::vector<std::unique_ptr<LevelConsts>> levels;  // index Ql (0 unused)
 
     // psi^(N/2) per prime (value, shoup): the NTT-slot factor of X^(N/2)
@@ -316,13 +327,46 @@ constexpr int kPolyPack = 64;
 struct PolyPack {
     uint64_t *p[kPolyPack];
 };
+
+// Base conversion fused with the column stages of the forward NTT of its outputs. Digit g of
+// member m holds min(alpha, total - g alpha) source words y (premultiplied, coefficient form)
+// per coefficient, at src + m src_stride + (src_lo + g alpha + i) N; output limb k < n_out
+// (prime of position k among QlP limbs) of polynomial m digits + g, at out + that out_stride
+// + k N, gets the column stages of sum_i y_i conv[g][k][i] (minus round(sum_i y_i / q_i) D_g
+// when rounded). With skip_own, the limbs of the digit itself are left out. The row stages
+// follow (ntt_rows_digits, moddown_rows_fused).
+struct ConvertJob {
+    const uint64_t *src;
+    size_t src_stride;
+    uint32_t src_lo, alpha, total, digits, members;
+    uint64_t *out;
+    size_t out_stride;
+    uint32_t n_out, Ql;
+    bool skip_own, rounded;
+    const u32x4 *conv;
+};
+// whether convert_cols covers conversions of `terms` source limbs: always one (plain
+// reduction), else with conv_ok
+bool convert_covers(const Context &c, size_t terms);
+void convert_cols(const Context &c, const ConvertJob &job, hipStream_t s);
+// Row stages of digits converted by convert_cols (polynomial m beta + g): the digit's own
+// limbs are copied from own.p[m] (its NTT-form words) with `copy_own`, else left untouched.
+void ntt_rows_digits(const Context &c, uint64_t *d, size_t Ql, size_t beta, size_t members, const PolyPack &own,
+                     bool copy_own, hipStream_t s);
+// Inverse NTT whose last pass multiplies limb k by scale[k - scale_lo] (value, Shoup
+// companion: N^-1 times a conversion's premultiplication) instead of N^-1.
+void ntt_inverse_gather_scaled(const Context &c, const PolyPack &in, uint64_t *out, size_t n_polys, size_t n_limbs,
+                               const uint64_t *scale, const uint64_t *scale_s, hipStream_t s);
+void ntt_inverse_qlp_scaled(const Context &c, uint64_t *data, size_t Ql, size_t lo, size_t hi, size_t n_polys,
+                            size_t poly_stride, const uint64_t *scale, const uint64_t *scale_s, hipStream_t s);
+
 // Forward NTT of the ModDown correction delta (n_polys x Ql limbs, in place)
 // whose last pass writes (cx - NTT(delta)) * pinv to out.p[p] (adding onto it
 // when bit p of acc_mask is set); cx holds cx_limbs limbs per polynomial.
 void moddown_ntt_fused(const Context &c, uint64_t *delta, const uint64_t *cx, size_t Ql, size_t cx_limbs,
                        const PolyPack &out, size_t n_polys, uint64_t acc_mask, const uint64_t *pinv,
                        const uint64_t *pinv_s, hipStream_t s, const PolyPack *add_src = nullptr,
-                       const uint32_t *add_perm = nullptr);
+                       const uint32_t *add_perm = nullptr, bool columns_done = false);
 // ntt_inverse of polynomials held in separate buffers: limb k of polynomial p is read
 // from in.p[p] + k N (n_limbs limbs each, at most 64 polynomials) and the result is
 // written to out ([n_polys][n_limbs][N]); the inputs are left as they are.

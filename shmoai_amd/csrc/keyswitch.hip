@@ -629,6 +629,35 @@ void ks_counters_reset() {
     }
 }
 
+// ModUp of m members with the conversion fused into the NTT's column stages: the inverse
+// transforms leave y_i = [x_i (D_g/q_i)^-1]_{q_i}, convert_cols takes every digit to its other
+// limbs' column stages, and the row stages finish them (copying the digits' own limbs, c2's
+// NTT-form words, where the caller reads them from d).
+static void modup_fused(const Context &c, const PolyPack &c2, size_t m, size_t Ql, uint64_t *d, bool own,
+                        hipStream_t s, bool rounded) {
+    const size_t N = c.N, alpha = c.nP, QlP = Ql + alpha;
+    const LevelConsts &L = c.level(Ql);
+    Scratch tcoef(m * Ql * N * sizeof(uint64_t), s);
+    ntt_inverse_gather_scaled(c, c2, tcoef.as<uint64_t>(), m, Ql, L.hat_ninv.as<uint64_t>(),
+                              L.hat_ninv_s.as<uint64_t>(), s);
+    ConvertJob job{};
+    job.src = tcoef.as<uint64_t>();
+    job.src_stride = Ql * N;
+    job.alpha = (uint32_t)alpha;
+    job.total = (uint32_t)Ql;
+    job.digits = (uint32_t)L.beta;
+    job.members = (uint32_t)m;
+    job.out = d;
+    job.out_stride = QlP * N;
+    job.n_out = (uint32_t)QlP;
+    job.Ql = (uint32_t)Ql;
+    job.skip_own = true;
+    job.rounded = rounded;
+    job.conv = L.conv_up.as<u32x4>();
+    convert_cols(c, job, s);
+    ntt_rows_digits(c, d, Ql, L.beta, m, c2, own, s);
+}
+
 void ks_modup(const Context &c, const uint64_t *c2, size_t Ql, uint64_t *d, hipStream_t s, bool rounded) {
     const size_t N = c.N, alpha = c.nP, QlP = Ql + alpha;
     const LevelConsts &L = c.level(Ql);
@@ -638,6 +667,12 @@ void ks_modup(const Context &c, const uint64_t *c2, size_t Ql, uint64_t *d, hipS
     // the key)
     if (beta > c.dnum) throw LogicError("key switching key has too few digits for this level");
     bump(g_cnt_modup, Ql, 1);
+    if (convert_covers(c, alpha)) {
+        PolyPack in{};
+        in.p[0] = const_cast<uint64_t *>(c2);  // read only
+        modup_fused(c, in, 1, Ql, d, true, s, rounded);
+        return;
+    }
     Scratch tcoef(Ql * N * sizeof(uint64_t), s);
     PolyPack in{};
     in.p[0] = const_cast<uint64_t *>(c2);  // read only
@@ -711,6 +746,26 @@ void ks_moddown_pack(const Context &c, uint64_t *cx, size_t npolys, size_t Ql, c
     if (npolys == 0 || npolys > 64) throw InvalidArgument("ks_moddown: 1..64 polynomials");
     bump(g_cnt_moddown, Ql, npolys);
     Scratch delta(npolys * Ql * N * sizeof(uint64_t), s);
+    if (convert_covers(c, nP)) {
+        ntt_inverse_qlp_scaled(c, cx, Ql, Ql, QlP, npolys, QlP * N, c.phat_ninv.as<uint64_t>(),
+                               c.phat_ninv_s.as<uint64_t>(), s);
+        ConvertJob job{};
+        job.src = cx;
+        job.src_stride = QlP * N;
+        job.src_lo = (uint32_t)Ql;
+        job.alpha = job.total = (uint32_t)nP;
+        job.digits = 1;
+        job.members = (uint32_t)npolys;
+        job.out = delta.as<uint64_t>();
+        job.out_stride = Ql * N;
+        job.n_out = job.Ql = (uint32_t)Ql;
+        job.rounded = rounded;
+        job.conv = c.conv_down.as<u32x4>();
+        convert_cols(c, job, s);
+        moddown_ntt_fused(c, delta.as<uint64_t>(), cx, Ql, QlP, out, npolys, acc_mask, c.pinv.as<uint64_t>(),
+                          c.pinv_s.as<uint64_t>(), s, add_src, perm, true);
+        return;
+    }
     ntt_inverse_qlp(c, cx, Ql, Ql, QlP, npolys, QlP * N, s);
     if (nP > (size_t)kMaxAlpha) throw InvalidArgument("at most 16 special primes");
     with_alpha_bound(nP, [&](auto bound) {
@@ -754,6 +809,10 @@ void ks_modup_batch(const Context &c, const PolyPack &c2, size_t m, size_t Ql, u
     if (beta > c.dnum) throw LogicError("key switching key has too few digits for this level");
     if (alpha > (size_t)kMaxAlpha) throw InvalidArgument("at most 16 special primes");
     bump(g_cnt_modup, Ql, m);
+    if (convert_covers(c, alpha)) {
+        modup_fused(c, c2, m, Ql, d, false, s, rounded);
+        return;
+    }
     // iNTT of the members into one buffer, conversion, NTT over m beta QlP limbs
     Scratch tcoef(m * Ql * N * sizeof(uint64_t), s);
     ntt_inverse_gather(c, c2, tcoef.as<uint64_t>(), m, Ql, 0, s);
@@ -849,8 +908,29 @@ void keyswitch_rescale_batch(const Context &c, const PolyPack &c2, const PolyPac
     // other Ql - 1 primes, and the NTT of the correction whose last pass writes
     // (cx - delta) B^-1 into the outputs
     bump(g_cnt_moddown, Ql, 2 * m);
-    ntt_inverse_qlp(c, cx.as<uint64_t>(), Ql, Ql - 1, QlP, 2 * m, QlP * N, s);
     Scratch delta(2 * m * (Ql - 1) * N * sizeof(uint64_t), s);
+    if (nP > 1 && convert_covers(c, nP + 1)) {
+        ntt_inverse_qlp_scaled(c, cx.as<uint64_t>(), Ql, Ql - 1, QlP, 2 * m, QlP * N, L.bhat_ninv.as<uint64_t>(),
+                               L.bhat_ninv_s.as<uint64_t>(), s);
+        ConvertJob job{};
+        job.src = cx.as<uint64_t>();
+        job.src_stride = QlP * N;
+        job.src_lo = (uint32_t)(Ql - 1);
+        job.alpha = job.total = (uint32_t)(nP + 1);
+        job.digits = 1;
+        job.members = (uint32_t)(2 * m);
+        job.out = delta.as<uint64_t>();
+        job.out_stride = (Ql - 1) * N;
+        job.n_out = (uint32_t)(Ql - 1);
+        job.Ql = (uint32_t)Ql;
+        job.rounded = true;
+        job.conv = L.conv_rescale.as<u32x4>();
+        convert_cols(c, job, s);
+        moddown_ntt_fused(c, delta.as<uint64_t>(), cx.as<uint64_t>(), Ql - 1, QlP, out, 2 * m, 0,
+                          L.binv.as<uint64_t>(), L.binv_s.as<uint64_t>(), s, nullptr, nullptr, true);
+        return;
+    }
+    ntt_inverse_qlp(c, cx.as<uint64_t>(), Ql, Ql - 1, QlP, 2 * m, QlP * N, s);
     with_alpha_bound(nP, [&](auto bound) {
         constexpr int A = decltype(bound)::value;
         (c.primes52 ? k_moddown_rescale_bconv<true, A>

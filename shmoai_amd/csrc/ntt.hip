@@ -79,6 +79,23 @@ __device__ __forceinline__ const __attribute__((address_space(1))) V *global_ptr
     return (const __attribute__((address_space(1))) V *)p;
 }
 
+// Tables that no kernel writes while it reads them: wave-uniform reads through this
+// pointer stay scalar loads also after the kernel's own stores.
+template <typename V>
+__device__ __forceinline__ const __attribute__((address_space(4))) V *table_ptr(const V *p) {
+    return (const __attribute__((address_space(4))) V *)(uintptr_t)p;
+}
+__device__ __forceinline__ FoldMod table_fold(const FoldMod *p) {
+    static_assert(sizeof(FoldMod) == 5 * sizeof(uint64_t), "FoldMod is read in words");
+    uint64_t w[5];
+    const auto q = table_ptr(reinterpret_cast<const uint64_t *>(p));
+#pragma unroll
+    for (int i = 0; i < 5; i++) w[i] = q[i];
+    FoldMod f;
+    __builtin_memcpy(&f, w, sizeof f);
+    return f;
+}
+
 // Twiddle and constant tables of one launch (forward or inverse set).
 struct NttTables {
     const DevMod *mods;
@@ -92,7 +109,7 @@ struct NttTables {
 // being the entry of group i at unit stage u, e = 2^u - 1 + i.
 struct HarveyK {
     uint64_t q;
-    __device__ HarveyK(const NttTables &tb, uint32_t prime) : q(tb.mods[prime].q) {}
+    __device__ HarveyK(const NttTables &tb, uint32_t prime) : q(table_ptr(&tb.mods[prime].q)[0]) {}
     static __device__ __forceinline__ uint64_t lo(u32x4 w) { return ((uint64_t)w.y << 32) | w.x; }
     static __device__ __forceinline__ uint64_t hi(u32x4 w) { return ((uint64_t)w.w << 32) | w.z; }
     __device__ __forceinline__ void fwd(uint64_t &a, uint64_t &b, u32x4 w) const {
@@ -129,6 +146,11 @@ struct HarveyK {
         return y;
     }
     __device__ __forceinline__ uint64_t load_rounded(double v, const DevMod &m) const { return residue_of_rounded(v, m); }
+    __device__ __forceinline__ uint64_t load_signed(uint64_t v, const DevMod &m) const {
+        const bool neg = (int64_t)v < 0;
+        const uint64_t y = reduce64(neg ? 0 - v : v, m);
+        return neg ? neg_mod(y, q) : y;
+    }
 };
 
 // SAFE folds a unit's words every second stage, so only a few products ever add up (for
@@ -138,7 +160,8 @@ template <bool SAFE>
 struct FoldK {
     uint64_t q;
     FoldMod f;
-    __device__ FoldK(const NttTables &tb, uint32_t prime) : q(tb.mods[prime].q), f(tb.fold[prime]) {}
+    __device__ FoldK(const NttTables &tb, uint32_t prime)
+        : q(table_ptr(&tb.mods[prime].q)[0]), f(table_fold(tb.fold + prime)) {}
     __device__ __forceinline__ void fwd(uint64_t &a, uint64_t &b, u32x4 w) const {
         const uint64_t t = fold_mul(b, w, f), s = a;
         a = s + t;
@@ -172,6 +195,7 @@ struct FoldK {
         return center && v > center ? v - (2 * center + 1) : v;
     }
     __device__ __forceinline__ uint64_t load_rounded(double v, const DevMod &m) const { return residue_of_rounded(v, m); }
+    __device__ __forceinline__ uint64_t load_signed(uint64_t v, const DevMod &) const { return v; }
 };
 
 template <int R, typename K, typename TW>
@@ -216,7 +240,10 @@ __device__ __forceinline__ void gs_unit(uint64_t *x, const K &k, TW tw) {
 //                rounded coefficient of the encoder's FFT output fft[p] (index
 //                i < N/2: round(re), i >= N/2: round(im) of entry i - N/2) as a
 //                residue, i.e. the encoder's decompose step fused into the load.
-enum { IO_PLAIN = 0, IO_REDUCE = 1, IO_RESCALE = 2, IO_ENCODE = 3, IO_GATHER = 4 };
+//   IO_DIGITS  : (phase B, forward) polynomial m digits + g is digit g of member m: its own
+//                limbs [g alpha, (g + 1) alpha) below Ql are copied from acc_p.p[m] (copy_own)
+//                or left untouched, the others transformed.
+enum { IO_PLAIN = 0, IO_REDUCE = 1, IO_RESCALE = 2, IO_ENCODE = 3, IO_GATHER = 4, IO_DIGITS = 5 };
 
 struct NttIO {
     const uint64_t *src;      // IO_REDUCE: [n_polys][N]
@@ -236,6 +263,10 @@ struct NttIO {
     const uint32_t *add_perm; // IO_RESCALE with out_packed: add add_src.p[p] read through this
     PolyPack add_src;         // NTT-domain permutation instead of out_p[p] (acc_mask bit p set)
     const double2 *fft;       // IO_ENCODE: [n_polys][N/2]
+    const uint64_t *scale;    // inverse, phase A: limb k is multiplied by scale[k - scale_lo]
+    const uint64_t *scale_s;  // (value, Shoup companion) instead of N^-1, unless null
+    uint32_t scale_lo;
+    uint32_t digits, alpha, copy_own;  // IO_DIGITS
 };
 
 // Column pass, log N1 = RA + RB stages. A block takes C columns (consecutive words of a
@@ -250,8 +281,8 @@ constexpr int col_width(int ra, int rb) { return rb == 0 ? kThreads : kThreads >
 
 template <int RA, int RB, bool FWD, int IO, typename K>
 __device__ __forceinline__ void col_pass(const K &k, uint64_t *lds, uint64_t *base, const u32x4 *__restrict__ col,
-                                         uint32_t c0, const NttTables &tb, uint32_t prime, uint32_t poly, size_t N,
-                                         const NttIO &io) {
+                                         uint32_t c0, const NttTables &tb, uint32_t prime, uint32_t poly, uint32_t limb,
+                                         size_t N, const NttIO &io) {
     constexpr int C = col_width(RA, RB);
     constexpr int UNITS = RB == 0 ? 1 : (C << RA) / kThreads;  // round-2 units per thread
     const uint32_t cl = threadIdx.x % C, c = c0 + cl;
@@ -330,7 +361,8 @@ __device__ __forceinline__ void col_pass(const K &k, uint64_t *lds, uint64_t *ba
             for (int l = 0; l < (1 << RA); l++) x[l] = lds[(r0 + (l << RB)) * C + cl];
         }
         gs_unit<RA>(x, k, tw1);
-        const auto ni = k.constant(tb.ninv[prime], tb.ninv_s[prime]);
+        const auto ni = io.scale ? k.constant(io.scale[limb - io.scale_lo], io.scale_s[limb - io.scale_lo])
+                                 : k.constant(tb.ninv[prime], tb.ninv_s[prime]);
 #pragma unroll
         for (int l = 0; l < (1 << RA); l++)
             __builtin_nontemporal_store(k.mul(x[l], ni), &base[(size_t)(r0 + (l << RB)) * kRow + c]);
@@ -350,12 +382,166 @@ __global__ __launch_bounds__(kThreads) void k_ntt_cols(uint64_t *__restrict__ da
     uint64_t *base = data + poly * mp.poly_stride + (size_t)k * N;
     const u32x4 *col = tb.col + (size_t)prime * kNttCols;
     if constexpr (FAST) {
-        col_pass<RA, RB, FWD, IO>(FoldK<false>(tb, prime), lds, base, col, c0, tb, prime, poly, N, io);
+        col_pass<RA, RB, FWD, IO>(FoldK<false>(tb, prime), lds, base, col, c0, tb, prime, poly, k, N, io);
     } else {
         if (tb.fold[prime].pw)
-            col_pass<RA, RB, FWD, IO>(FoldK<true>(tb, prime), lds, base, col, c0, tb, prime, poly, N, io);
+            col_pass<RA, RB, FWD, IO>(FoldK<true>(tb, prime), lds, base, col, c0, tb, prime, poly, k, N, io);
         else
-            col_pass<RA, RB, FWD, IO>(HarveyK(tb, prime), lds, base, col, c0, tb, prime, poly, N, io);
+            col_pass<RA, RB, FWD, IO>(HarveyK(tb, prime), lds, base, col, c0, tb, prime, poly, k, N, io);
+    }
+}
+
+// Base conversion into the column stages (ConvertJob). A block keeps the source words of its
+// columns in registers (A words per coefficient, 16 coefficients a thread at N = 2^16: 160 of
+// its 256 VGPRs for 5 special primes) and loops over a run of output limbs: sums of split
+// products, column stages, store. One exchange through LDS per limb, double-buffered, so one
+// barrier; the limb's column twiddles come through LDS too, requested a limb ahead. Against a
+// conversion kernel that writes every limb and a column pass that reads it back, the words
+// in between (and their reduction to canonical residues) are gone: a shared-a chunk's
+// conversions and forward column passes at N = 2^16 took 29.0 ms apart and take 18.3 ms
+// here; one top-level rotation's 154 and 87 us. Bound by VALU issue at 2 waves per SIMD
+// (8 words a thread, which halves the registers, needs a third exchange at 7 stages).
+template <int RA, int RB, int A, bool FAST>
+__global__ __launch_bounds__(kThreads, 2) void k_convert_cols(ConvertJob job, NttTables tb, int logN, uint32_t nQ,
+                                                              uint32_t run) {
+    constexpr int C = col_width(RA, RB), U = 1 << RA, N1 = 1 << (RA + RB);
+    constexpr int UNITS = RB == 0 ? 1 : (C << RA) / kThreads;
+    __shared__ uint64_t lds[2][RB == 0 ? 1 : C * N1];
+    __shared__ __align__(16) u32x4 ltw[2][N1];
+    const size_t N = size_t(1) << logN;
+    const uint32_t cl = threadIdx.x % C, c = blockIdx.x * C + cl, r0 = RB == 0 ? 0 : threadIdx.x / C;
+    const uint32_t poly = blockIdx.y, g = poly % job.digits, start = g * job.alpha;
+    const uint32_t size = min(job.alpha, job.total - start);
+    const uint64_t *src = job.src + (size_t)(poly / job.digits) * job.src_stride + (size_t)(job.src_lo + start) * N + c;
+    auto prime_of = [&](uint32_t k) { return k < job.Ql ? k : nQ + (k - job.Ql); };
+    // source words in halves, and each coefficient's rounding (at most A < 16) in 4 bits
+    uint32_t yl[A][U], yh[A][U], r[(U + 7) / 8] = {};
+    {
+        uint64_t y[A][U];
+        double v[U];
+#pragma unroll
+        for (int l = 0; l < U; l++) v[l] = 0.0;
+#pragma unroll
+        for (int i = 0; i < A; i++) {
+            if ((uint32_t)i < size) {
+#pragma unroll
+                for (int l = 0; l < U; l++) y[i][l] = src[(size_t)i * N + (size_t)(r0 + (l << RB)) * kRow];
+            } else {
+#pragma unroll
+                for (int l = 0; l < U; l++) y[i][l] = 0;
+            }
+        }
+        if (job.rounded) {
+#pragma unroll
+            for (int i = 0; i < A; i++) {
+                if ((uint32_t)i < size) {
+                    const double q = (double)table_ptr(&tb.mods[prime_of(job.src_lo + start + i)].q)[0];
+#pragma unroll
+                    for (int l = 0; l < U; l++) v[l] = __dadd_rn(v[l], __ddiv_rn((double)y[i][l], q));
+                }
+            }
+#pragma unroll
+            for (int l = 0; l < U; l++) r[l / 8] |= (uint32_t)(uint64_t)__dadd_rn(v[l], 0.5) << (4 * (l % 8));
+            if (A == 1) {  // one source limb: the signed word itself
+                const uint64_t q = table_ptr(&tb.mods[prime_of(job.src_lo + start)].q)[0];
+#pragma unroll
+                for (int l = 0; l < U; l++) y[0][l] -= ((r[l / 8] >> (4 * (l % 8))) & 15) ? q : 0;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < A; i++)
+#pragma unroll
+            for (int l = 0; l < U; l++) {
+                yl[i][l] = (uint32_t)y[i][l];
+                yh[i][l] = (uint32_t)(y[i][l] >> 32);
+            }
+    }
+    const uint32_t k_end = min((blockIdx.z + 1) * run, job.n_out);
+    uint64_t *out = job.out + (size_t)poly * job.out_stride + c;
+    // the next limb to convert from k on (uniform over the block)
+    auto next = [&](uint32_t k) {
+        return job.skip_own && k >= start && k < start + size ? start + size : k;
+    };
+    auto tw_of = [&](uint32_t k) {
+        return k < k_end && threadIdx.x < N1 ? tb.col[(size_t)prime_of(k) * kNttCols + threadIdx.x] : u32x4{0, 0, 0, 0};
+    };
+    uint32_t k = next(blockIdx.z * run);
+    u32x4 tw_next = tw_of(k);
+    int buf = 0;
+    while (k < k_end) {
+        const uint32_t prime = prime_of(k), k_next = next(k + 1);
+        if (threadIdx.x < N1) ltw[buf][threadIdx.x] = tw_next;
+        tw_next = tw_of(k_next);
+        // The halves pass through an empty statement each turn: their widening stays inside
+        // the loop, next to the multiply-adds it belongs to (hoisted, it doubles the registers
+        // and turns every product into a 64 x 64 one).
+#pragma unroll
+        for (int i = 0; i < A; i++)
+#pragma unroll
+            for (int l = 0; l < U; l++) asm("" : "+v"(yl[i][l]), "+v"(yh[i][l]));
+#pragma unroll
+        for (int l = 0; l < (U + 7) / 8; l++) asm("" : "+v"(r[l]));
+        auto body = [&](const auto &kk) {
+            uint64_t x[U];
+            if constexpr (A == 1) {
+                DevMod m{};
+                if (!FAST) m = tb.mods[prime];
+#pragma unroll
+                for (int l = 0; l < U; l++) x[l] = kk.load_signed(((uint64_t)yh[0][l] << 32) | yl[0][l], m);
+            } else if constexpr (FAST) {
+                const auto cv = table_ptr(job.conv + ((size_t)g * job.n_out + k) * (job.alpha + 1));
+                u32x4 w[A + 1];
+#pragma unroll
+                for (int i = 0; i < A; i++) w[i] = (uint32_t)i < job.alpha ? cv[i] : u32x4{0, 0, 0, 0};
+                w[A] = cv[job.alpha];
+#pragma unroll
+                for (int l = 0; l < U; l++) {
+                    ConvAcc acc{0, 0};
+#pragma unroll
+                    for (int i = 0; i < A; i++) conv_mac(acc, yl[i][l], yh[i][l], w[i]);
+                    if (job.rounded) {
+                        const uint32_t rl = (r[l / 8] >> (4 * (l % 8))) & 15;
+                        acc.H += (uint64_t)rl * w[A].x;
+                        acc.L += (uint64_t)rl * w[A].y;
+                    }
+                    x[l] = conv_value(acc, kk.f);
+                }
+            }
+            const auto col = table_ptr(tb.col + (size_t)prime * kNttCols);
+            ct_unit<RA>(x, kk, [&](int e) -> u32x4 { return col[e + 1]; });
+            if constexpr (RB == 0) {
+#pragma unroll
+                for (int l = 0; l < U; l++) __builtin_nontemporal_store(x[l], &out[(size_t)k * N + (size_t)l * kRow]);
+            } else {
+#pragma unroll
+                for (int l = 0; l < U; l++) lds[buf][(r0 + (l << RB)) * C + cl] = x[l];
+                __syncthreads();
+#pragma unroll
+                for (int m = 0; m < UNITS; m++) {
+                    const uint32_t u0 = threadIdx.x / C + m * (kThreads / C);
+                    uint64_t z[1 << RB];
+#pragma unroll
+                    for (int l = 0; l < (1 << RB); l++) z[l] = lds[buf][((u0 << RB) + l) * C + cl];
+                    ct_unit<RB>(z, kk, [&](int e) -> u32x4 {
+                        const int u = e >= 7 ? 3 : e >= 3 ? 2 : e >= 1 ? 1 : 0;
+                        return ltw[buf][(((1u << RA) + u0) << u) + (uint32_t)(e - ((1 << u) - 1))];
+                    });
+#pragma unroll
+                    for (int l = 0; l < (1 << RB); l++)
+                        __builtin_nontemporal_store(z[l], &out[(size_t)k * N + (size_t)((u0 << RB) + l) * kRow]);
+                }
+            }
+        };
+        if constexpr (FAST) {
+            body(FoldK<false>(tb, prime));
+        } else {
+            if (tb.fold[prime].pw)
+                body(FoldK<true>(tb, prime));
+            else
+                body(HarveyK(tb, prime));
+        }
+        buf ^= 1;
+        k = k_next;
     }
 }
 
@@ -516,11 +702,17 @@ __global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data,
     limb_of(mp, rest / rows, poly0, limb, prime);  // limb of the first polynomial
     const uint32_t row0 = row * kRow;
     const u32x4 *tw = tb.row + (size_t)prime * N + row0;
+    auto own = [&](uint32_t p) {  // whether this limb is digit p's own
+        const uint32_t lo = p % io.digits * io.alpha;
+        return limb >= lo && limb < min(lo + io.alpha, mp.Ql);
+    };
     auto src_of = [&](uint32_t p) -> const uint64_t * {
+        if (IO == IO_DIGITS && io.copy_own && own(p)) return io.acc_p.p[p / io.digits] + (size_t)limb * N + row0;
         return IO == IO_GATHER ? io.acc_p.p[p] + (size_t)limb * N + row0
                                : data + p * mp.poly_stride + (size_t)limb * N + row0;
     };
     auto load = [&](uint64_t (&x)[8], uint32_t p) {
+        if (IO == IO_DIGITS && !io.copy_own && own(p)) return;
         const uint64_t *ld = src_of(p);
         if constexpr (FWD) {
 #pragma unroll
@@ -548,7 +740,14 @@ __global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data,
         for (uint32_t p = p0; p < p1; p++) {
             if (p + 1 < p1) load(nx, p + 1);
             uint64_t *base = data + p * mp.poly_stride + (size_t)limb * N + row0;
-            row_pass<FWD, IO>(k, lds[wave], base, tw, w2, w3, x, tb, prime, p, limb, row0, mp.n_active, N, lane, io, qi);
+            if (IO == IO_DIGITS && own(p)) {
+                if (io.copy_own)
+#pragma unroll
+                    for (int l = 0; l < 8; l++) __builtin_nontemporal_store(x[l], base + lane + 64 * l);
+            } else {
+                row_pass<FWD, IO>(k, lds[wave], base, tw, w2, w3, x, tb, prime, p, limb, row0, mp.n_active, N, lane, io,
+                                  qi);
+            }
             wave_lds_order();
 #pragma unroll
             for (int l = 0; l < 8; l++) x[l] = nx[l];
@@ -583,14 +782,14 @@ struct FusedProbe {
 
 template <bool FWD, int IOA, int IOB>
 void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t total_limbs, hipStream_t s,
-                const NttIO &io = NttIO{}) {
+                const NttIO &io = NttIO{}, bool columns_done = false) {
     if (total_limbs == 0) return;
     if (c.N < (size_t)4096) throw InvalidArgument("NTT requires N >= 4096");
     if (total_limbs % mp.n_active != 0) throw LogicError("NTT limb count is not a multiple of the polynomial size");
     const int logN = c.logN;
     const size_t N = c.N;
     const int stages = logN - 9;                       // of the column pass
-    const int unit = stages == 4 || stages >= 7 ? 4 : 3;  // of its longest unit
+    const int unit = stages >= 7 ? 4 : 3;  // of its longest unit
     const uint32_t n_polys = (uint32_t)(total_limbs / mp.n_active);
     NttTables tb{c.mods(),
                  c.d_fold.as<FoldMod>(),
@@ -646,7 +845,7 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
     }
         switch (stages) {
             SHM_COLS(3, 3, 0)
-            SHM_COLS(4, 4, 0)
+            SHM_COLS(4, 2, 2)
             SHM_COLS(5, 3, 2)
             SHM_COLS(6, 3, 3)
             SHM_COLS(7, 4, 3)
@@ -668,11 +867,11 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
 #undef SHM_ROWS
     };
     if (FWD) {
-        cols();
+        if (!columns_done) cols();
         const bool timed = IOB == IO_RESCALE && g_rescale_tile_ev[0] && g_rescale_tile_ev[1];
         if (timed) SHM_HIP(hipEventRecord(g_rescale_tile_ev[0], s));
         hipEvent_t pe[2] = {nullptr, nullptr};
-        if (IOB == IO_PLAIN) {
+        if (IOB == IO_PLAIN || IOB == IO_DIGITS) {
             std::lock_guard<std::mutex> lk(g_probe.mu);
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
             if (g_probe.on && hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
@@ -889,7 +1088,8 @@ void rescale_ntt_fused_window(const Context &c, const uint64_t *last, const uint
 
 void moddown_ntt_fused(const Context &c, uint64_t *delta, const uint64_t *cx, size_t Ql, size_t cx_limbs,
                        const PolyPack &out, size_t n_polys, uint64_t acc_mask, const uint64_t *pinv,
-                       const uint64_t *pinv_s, hipStream_t s, const PolyPack *add_src, const uint32_t *add_perm) {
+                       const uint64_t *pinv_s, hipStream_t s, const PolyPack *add_src, const uint32_t *add_perm,
+                       bool columns_done) {
     if (n_polys == 0 || n_polys > (size_t)kPolyPack) throw InvalidArgument("ModDown: 1..64 polynomials per batch");
     if ((add_src == nullptr) != (add_perm == nullptr)) throw LogicError("ModDown: permuted addend needs both parts");
     LimbMap mp{(uint32_t)Ql, 0, 0xffffffffu, 0, 0xffffffffu, (uint32_t)c.nQ, 0, (uint64_t)Ql * c.N};
@@ -905,7 +1105,90 @@ void moddown_ntt_fused(const Context &c, uint64_t *delta, const uint64_t *cx, si
         io.add_src = *add_src;
         io.add_perm = add_perm;
     }
-    launch_ntt<true, IO_PLAIN, IO_RESCALE>(c, delta, mp, n_polys * Ql, s, io);
+    launch_ntt<true, IO_PLAIN, IO_RESCALE>(c, delta, mp, n_polys * Ql, s, io, columns_done);
+}
+
+bool convert_covers(const Context &c, size_t terms) { return terms == 1 || (c.conv_ok && terms <= 6); }
+
+void convert_cols(const Context &c, const ConvertJob &job, hipStream_t s) {
+    if (!convert_covers(c, job.alpha)) throw LogicError("conversion outside the fused form");
+    const int logN = c.logN, stages = logN - 9;
+    NttTables tb{c.mods(), c.d_fold.as<FoldMod>(), c.tw_col.as<u32x4>(), nullptr, nullptr, nullptr};
+    const unsigned polys = job.members * job.digits;
+    // one source limb: the word is below 2^61, any sum of products is folded (GENERAL) unless
+    // conv_ok says they all fit
+    const bool fast = c.conv_ok;
+    auto launch = [&](auto fn, int width) {
+        const unsigned blocks = (unsigned)(kRow / width) * polys;
+        // a run of output limbs per block, shorter (but at least 4) where that leaves fewer
+        // than 6 blocks a CU: every run reads the digit's source words again
+        unsigned runs = std::max(1u, std::min((1536u + blocks - 1) / blocks, (job.n_out + 3) / 4));
+        const unsigned run = (job.n_out + runs - 1) / runs;
+        runs = (job.n_out + run - 1) / run;
+        fn<<<dim3(kRow / width, polys, runs), kThreads, 0, s>>>(job, tb, logN, (uint32_t)c.nQ, run);
+    };
+#define SHM_CONV_A(RA, RB)                                                                                   \
+    if (job.alpha == 1 && !fast)                                                                             \
+        launch(k_convert_cols<RA, RB, 1, false>, col_width(RA, RB));                                         \
+    else if (job.alpha == 1)                                                                                 \
+        launch(k_convert_cols<RA, RB, 1, true>, col_width(RA, RB));                                          \
+    else if (job.alpha == 2)                                                                                 \
+        launch(k_convert_cols<RA, RB, 2, true>, col_width(RA, RB));                                          \
+    else if (job.alpha == 3)                                                                                 \
+        launch(k_convert_cols<RA, RB, 3, true>, col_width(RA, RB));                                          \
+    else if (job.alpha == 4)                                                                                 \
+        launch(k_convert_cols<RA, RB, 4, true>, col_width(RA, RB));                                          \
+    else if (job.alpha == 5)                                                                                 \
+        launch(k_convert_cols<RA, RB, 5, true>, col_width(RA, RB));                                          \
+    else                                                                                                     \
+        launch(k_convert_cols<RA, RB, 6, true>, col_width(RA, RB));                                          \
+    break;
+    switch (stages) {
+        case 3: SHM_CONV_A(3, 0)
+        case 4: SHM_CONV_A(2, 2)
+        case 5: SHM_CONV_A(3, 2)
+        case 6: SHM_CONV_A(3, 3)
+        case 7: SHM_CONV_A(4, 3)
+        case 8: SHM_CONV_A(4, 4)
+        default: throw InvalidArgument("unsupported ring degree for NTT");
+    }
+#undef SHM_CONV_A
+    SHM_HIP(hipGetLastError());
+}
+
+void ntt_rows_digits(const Context &c, uint64_t *d, size_t Ql, size_t beta, size_t members, const PolyPack &own,
+                     bool copy_own, hipStream_t s) {
+    const size_t QlP = Ql + c.nP;
+    LimbMap mp{(uint32_t)QlP, 0, 0xffffffffu, 0, (uint32_t)Ql, (uint32_t)c.nQ, 0, (uint64_t)QlP * c.N};
+    NttIO io{};
+    io.acc_p = own;
+    io.digits = (uint32_t)beta;
+    io.alpha = (uint32_t)c.nP;
+    io.copy_own = copy_own ? 1 : 0;
+    launch_ntt<true, IO_PLAIN, IO_DIGITS>(c, d, mp, members * beta * QlP, s, io, true);
+}
+
+void ntt_inverse_gather_scaled(const Context &c, const PolyPack &in, uint64_t *out, size_t n_polys, size_t n_limbs,
+                               const uint64_t *scale, const uint64_t *scale_s, hipStream_t s) {
+    if (n_polys == 0) return;
+    if (n_polys > (size_t)kPolyPack) throw InvalidArgument("inverse NTT: 1..64 polynomials per batch");
+    LimbMap mp{(uint32_t)n_limbs, 0, 0xffffffffu, 0, 0xffffffffu, (uint32_t)c.nQ, 0, (uint64_t)n_limbs * c.N};
+    NttIO io{};
+    io.acc_p = in;
+    io.scale = scale;
+    io.scale_s = scale_s;
+    launch_ntt<false, IO_PLAIN, IO_GATHER>(c, out, mp, n_polys * n_limbs, s, io);
+}
+
+void ntt_inverse_qlp_scaled(const Context &c, uint64_t *data, size_t Ql, size_t lo, size_t hi, size_t n_polys,
+                            size_t poly_stride, const uint64_t *scale, const uint64_t *scale_s, hipStream_t s) {
+    LimbMap mp{(uint32_t)(hi - lo), (uint32_t)lo, 0xffffffffu, 0, (uint32_t)Ql, (uint32_t)c.nQ, 0,
+               (uint64_t)poly_stride};
+    NttIO io{};
+    io.scale = scale;
+    io.scale_s = scale_s;
+    io.scale_lo = (uint32_t)lo;
+    launch_ntt<false, IO_PLAIN, IO_PLAIN>(c, data, mp, n_polys * (hi - lo), s, io);
 }
 
 void rescale_ntt_fused_pack(const Context &c, const uint64_t *last, const PolyPack &in, const PolyPack &out,
