@@ -163,6 +163,47 @@ void conv_table(const Context &c, const DevBuf &hat, const DevBuf &dig, DevBuf &
     SHM_HIP(hipGetLastError());
 }
 
+// LevelConsts::compose of the first Ql primes.
+std::vector<uint64_t> compose_table(const std::vector<uint64_t> &q, size_t Ql) {
+    const size_t W = Ql;
+    std::vector<uint64_t> t(2 * W + 2 + 2 * Ql + Ql * W, 0);
+    uint64_t *Q = t.data(), *half = Q + W, *inv01 = half + W, *qhinv = inv01 + 2, *qhinv_s = qhinv + Ql,
+             *qhat = qhinv_s + Ql;
+    auto mul_small = [&](uint64_t *a, uint64_t b) {
+        hu128 carry = 0;
+        for (size_t w = 0; w < W; w++) {
+            const hu128 v = (hu128)a[w] * b + carry;
+            a[w] = (uint64_t)v;
+            carry = v >> 64;
+        }
+    };
+    Q[0] = 1;
+    for (size_t i = 0; i < Ql; i++) mul_small(Q, q[i]);
+    for (size_t i = 0; i < Ql; i++) {
+        uint64_t *h = qhat + i * W, r = 1;
+        h[0] = 1;
+        for (size_t k = 0; k < Ql; k++)
+            if (k != i) {
+                mul_small(h, q[k]);
+                r = h_mulmod(r, q[k] % q[i], q[i]);
+            }
+        qhinv[i] = h_inv(r, q[i]);
+        qhinv_s[i] = h_shoup(qhinv[i], q[i]);
+    }
+    hu128 carry = 1;  // (Q + 1) / 2
+    for (size_t w = 0; w < W; w++) {
+        const hu128 v = (hu128)Q[w] + carry;
+        half[w] = (uint64_t)v;
+        carry = v >> 64;
+    }
+    for (size_t w = 0; w < W; w++) half[w] = (half[w] >> 1) | (w + 1 < W ? half[w + 1] << 63 : 0);
+    if (Ql >= 2) {
+        inv01[0] = h_inv(q[0], q[1]);
+        inv01[1] = h_shoup(inv01[0], q[1]);
+    }
+    return t;
+}
+
 // Largest value conv_value leaves of `terms` products (and the rounding term): H < 1.02
 // terms 2^59 + 2^32, so its high word times 32 delta; its low word times 2^s, s = b - 27;
 // and L < 1.02 terms 2^(32+s) + 2^(5+s).
@@ -589,6 +630,7 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
         upload(L->hat_inv_s, his);
         upload(L->hat_mod, hm);
         upload(L->dig_mod, dm);
+        if (Ql <= 64) upload(L->compose, compose_table(c->q, Ql));
         std::vector<uint64_t> hn(Ql), hns(Ql);
         for (size_t i = 0; i < Ql; i++) {
             hn[i] = h_mulmod(hi[i], ninv[i], c->q[i]);
@@ -661,6 +703,7 @@ std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, si
         pos = (pos * 5) & (m - 1);
     }
     upload(c->enc_group, grp);
+    encoder_tables(*c);
     SHM_HIP(hipDeviceSynchronize());
     return c;
 }

@@ -136,6 +136,9 @@ struct LevelConsts {
     // split constants (ConvAcc) of the conversions, u32x4 [g][k][terms + 1]: hat_mod (or
     // bhat_mod) of each term, then -[D_g]_{p_k} (or -B): with Context::conv_ok only
     DevBuf conv_up, conv_rescale;
+    // decoder's CRT composition (Ql <= 64), 64-bit words: Q [Ql], (Q + 1) / 2 [Ql], q_0^-1
+    // mod q_1 (value, shoup), then (Q/q_i)^-1 mod q_i [Ql] (values, shoups) and Q/q_i [Ql][Ql]
+    DevBuf compose;
 };
 
 struct Context {
@@ -173,6 +176,7 @@ struct Context {
     // encoder
     DevBuf enc_roots;       // complex<double>[2N] (re, im interleaved)
     DevBuf enc_group;       // uint32[N/4]
+    DevBuf enc_fwd, enc_inv; // complex<double>[N/2]: FFT twiddles by stage (encoder.hip)
 
     // Galois permutation tables cache: elt -> uint32[N]
     std::mutex galois_mu;
@@ -197,6 +201,8 @@ struct Context {
     } aux;
     hipStream_t aux_stream();
 };
+
+void encoder_tables(Context &c);  // enc_fwd, enc_inv from enc_roots and enc_group
 
 std::unique_ptr<Context> make_context(int logN, const std::vector<int> &bits, size_t nP);
 
