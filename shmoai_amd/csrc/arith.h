@@ -200,6 +200,14 @@ __device__ __forceinline__ uint64_t fold_canon(uint64_t x, uint64_t q, const Fol
     return csub(y, q);
 }
 
+// Congruent to a signed x, |x| <= 2^63 - q, in [0, 2q) (primes that fold once).
+__device__ __forceinline__ uint64_t fold_positive(uint64_t x, const FoldMod &f) {
+    const uint64_t y = x + f.off;
+    const uint32_t yh = (uint32_t)(y >> 32);
+    const uint64_t lo = ((uint64_t)(yh & f.mask) << 32) | (uint32_t)y;
+    return (uint64_t)(yh >> f.sh) * (uint32_t)f.d + lo;
+}
+
 // The split form of a constant w < q given its Shoup companion.
 __device__ __forceinline__ u32x4 fold_split(uint64_t w, uint64_t ws, uint64_t q, const FoldMod &f) {
     const uint64_t w1 = mul_shoup(uint64_t(1) << 32, w, ws, q);

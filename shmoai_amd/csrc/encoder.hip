@@ -493,7 +493,7 @@ void encode_columns_batch(const Context &c, const double *X, size_t num_x, size_
 }
 
 void encode_masked_batch(const Context &c, const double *w, const double *fix, const uint8_t *mask, size_t B,
-                         size_t Ql, uint64_t *out, double2 *fftbuf, hipStream_t s) {
+                         size_t Ql, uint64_t *out, double2 *fftbuf, hipStream_t s, bool rows) {
     const size_t n = c.N / 2;
     if (B == 0) return;
     if (B > 65535) throw InvalidArgument("encode_masked_batch: at most 65535 plaintexts");
@@ -504,7 +504,10 @@ void encode_masked_batch(const Context &c, const double *w, const double *fix, c
     ifft<FFT_MASK>(c, fftbuf, (uint32_t)n, logn, B, io, fix, 0.0, s);
     SHM_HIP(hipGetLastError());
     // decompose (round, residue per prime) fused into the NTT's column pass
-    ntt_forward_encoded(c, fftbuf, out, B, Ql, s);
+    if (rows)
+        ntt_forward_encoded(c, fftbuf, out, B, Ql, s);
+    else
+        ntt_encoded_columns(c, fftbuf, out, B, Ql, s);
 }
 
 void encode_scalar(const Context &c, double value, size_t Ql, double scale, uint64_t *out, hipStream_t s) {

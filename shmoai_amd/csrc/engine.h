@@ -350,6 +350,7 @@ struct ConvertJob {
     uint32_t n_out, Ql;
     bool skip_own, rounded;
     const u32x4 *conv;
+    const double2 *fft;  // instead of src: rounded encoder output [members][N/2] (alpha = 1)
 };
 // whether convert_cols covers conversions of `terms` source limbs: always one (plain
 // reduction), else with conv_ok
@@ -359,6 +360,33 @@ void convert_cols(const Context &c, const ConvertJob &job, hipStream_t s);
 // limbs are copied from own.p[m] (its NTT-form words) with `copy_own`, else left untouched.
 void ntt_rows_digits(const Context &c, uint64_t *d, size_t Ql, size_t beta, size_t members, const PolyPack &own,
                      bool copy_own, hipStream_t s);
+// Row stages fused with their products: polynomial e ge + t gt of data (column stages done) is
+// term t of group e; output o of group e is sum_t term_t operand_(t,o) over `limbs` limbs
+// (primes of positions among QlP limbs), at out + (2 e + o) out_stride.
+//   key != null: operands are key rows (term stride 2 op_stride, output stride op_stride, by
+//     prime); the group's own limbs of digit t come from op.p[e]; with add_on, P add.p[2 e + o]
+//     is added on the data limbs.
+//   else: operand (t, o) is op.p[t] + o op_stride, by limb; with accumulate, onto the output.
+struct MacJob {
+    const uint64_t *data;
+    size_t stride;
+    uint32_t groups, terms, ge, gt, limbs, Ql, alpha;
+    const uint64_t *key;
+    size_t op_stride;
+    PolyPack op;
+    uint64_t *out;
+    size_t out_stride;
+    bool accumulate, add_on;
+    PolyPack add;
+    const uint64_t *pmod, *pmod_s;
+};
+// whether rows_mac covers n_data data limbs (and the special ones): primes in (2^45, 2^52)
+// with split forms, 1 to 16 terms
+bool rows_mac_covers(const Context &c, size_t n_data, bool special, size_t terms);
+void rows_mac(const Context &c, const MacJob &job, hipStream_t s);
+// Rounded encoder output through the column stages alone (ntt_forward_encoded's first half).
+void ntt_encoded_columns(const Context &c, const double2 *fft, uint64_t *out, size_t n_polys, size_t n_limbs,
+                         hipStream_t s);
 // Inverse NTT whose last pass multiplies limb k by scale[k - scale_lo] (value, Shoup
 // companion: N^-1 times a conversion's premultiplication) instead of N^-1.
 void ntt_inverse_gather_scaled(const Context &c, const PolyPack &in, uint64_t *out, size_t n_polys, size_t n_limbs,
@@ -516,7 +544,7 @@ void encode_columns_batch(const Context &c, const double *X, size_t num_x, size_
 // {mask[t] ? w[b] : 0} (t < N/2) at scale fix[b] * N/2, exactly as encode() does
 // for that vector. w, fix, mask are device arrays; fftbuf holds B * N/2 double2.
 void encode_masked_batch(const Context &c, const double *w, const double *fix, const uint8_t *mask, size_t B,
-                         size_t Ql, uint64_t *out, double2 *fftbuf, hipStream_t s);
+                         size_t Ql, uint64_t *out, double2 *fftbuf, hipStream_t s, bool rows = true);
 void decode(const Context &c, const uint64_t *pt, size_t Ql, double scale, double *re, double *im, size_t n,
             hipStream_t s);
 

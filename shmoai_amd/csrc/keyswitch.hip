@@ -629,12 +629,18 @@ void ks_counters_reset() {
     }
 }
 
+// Rows (of 512 words, over limbs and members) from which the row stages and the products run
+// fused, one wave each for all digits: 2 waves per SIMD. Below, the digits' rows run side by
+// side in the separate kernels instead of one after the other in too few waves.
+constexpr size_t kFusedRows = 2048;
+
 // ModUp of m members with the conversion fused into the NTT's column stages: the inverse
 // transforms leave y_i = [x_i (D_g/q_i)^-1]_{q_i}, convert_cols takes every digit to its other
 // limbs' column stages, and the row stages finish them (copying the digits' own limbs, c2's
 // NTT-form words, where the caller reads them from d).
+// Without `rows`, the row stages are left to the caller (rows_mac).
 static void modup_fused(const Context &c, const PolyPack &c2, size_t m, size_t Ql, uint64_t *d, bool own,
-                        hipStream_t s, bool rounded) {
+                        hipStream_t s, bool rounded, bool rows = true) {
     const size_t N = c.N, alpha = c.nP, QlP = Ql + alpha;
     const LevelConsts &L = c.level(Ql);
     Scratch tcoef(m * Ql * N * sizeof(uint64_t), s);
@@ -655,7 +661,44 @@ static void modup_fused(const Context &c, const PolyPack &c2, size_t m, size_t Q
     job.rounded = rounded;
     job.conv = L.conv_up.as<u32x4>();
     convert_cols(c, job, s);
-    ntt_rows_digits(c, d, Ql, L.beta, m, c2, own, s);
+    if (rows) ntt_rows_digits(c, d, Ql, L.beta, m, c2, own, s);
+}
+
+// ModUp of m members and their inner products with one key, cx[m][2][QlP][N], the digits' row
+// stages fused with the products (and P d01 added on the data limbs). Returns false, with
+// nothing done, where that does not apply: primes outside the split sums, or too few rows to
+// fill the GPU with one wave per row and member.
+static bool modup_inner_fused(const Context &c, const PolyPack &c2, size_t m, size_t Ql, const uint64_t *key,
+                              uint64_t *d, uint64_t *cx, hipStream_t s, bool rounded, const PolyPack *add) {
+    const size_t N = c.N, alpha = c.nP, QlP = Ql + alpha, beta = c.level(Ql).beta;
+    if (!convert_covers(c, alpha) || !rows_mac_covers(c, Ql, true, beta) || beta > c.dnum) return false;
+    if (m * QlP * (N / 512) < kFusedRows) return false;
+    bump(g_cnt_modup, Ql, m);
+    bump(g_cnt_inner, Ql, 2 * m);
+    modup_fused(c, c2, m, Ql, d, false, s, rounded, false);
+    MacJob job{};
+    job.data = d;
+    job.stride = QlP * N;
+    job.groups = (uint32_t)m;
+    job.terms = (uint32_t)beta;
+    job.ge = (uint32_t)beta;
+    job.gt = 1;
+    job.limbs = (uint32_t)QlP;
+    job.Ql = (uint32_t)Ql;
+    job.alpha = (uint32_t)alpha;
+    job.key = key;
+    job.op_stride = c.nQP() * N;
+    job.op = c2;
+    job.out = cx;
+    job.out_stride = QlP * N;
+    if (add) {
+        job.add_on = true;
+        job.add = *add;
+        job.pmod = c.pmod.as<uint64_t>();
+        job.pmod_s = c.pmod_s.as<uint64_t>();
+    }
+    rows_mac(c, job, s);
+    return true;
 }
 
 void ks_modup(const Context &c, const uint64_t *c2, size_t Ql, uint64_t *d, hipStream_t s, bool rounded) {
@@ -787,11 +830,15 @@ void keyswitch(const Context &c, const uint64_t *c2, const uint64_t *key, size_t
     if (beta > c.dnum) throw LogicError("key switching key has too few digits for this level");
     Scratch d(beta * QlP * N * sizeof(uint64_t), s);
     Scratch cx(2 * QlP * N * sizeof(uint64_t), s);
-    ks_modup(c, c2, Ql, d.as<uint64_t>(), s, rounded);
-    bump(g_cnt_inner, Ql, 2);
-    k_ks_inner<<<grid_for(QlP * N), kBlock, 0, s>>>(d.as<uint64_t>(), key, cx.as<uint64_t>(), c.mods(), Ql, c.nQ,
-                                                    c.nQP(), alpha, beta, N);
-    SHM_HIP(hipGetLastError());
+    PolyPack in{};
+    in.p[0] = const_cast<uint64_t *>(c2);  // read only
+    if (!modup_inner_fused(c, in, 1, Ql, key, d.as<uint64_t>(), cx.as<uint64_t>(), s, rounded, nullptr)) {
+        ks_modup(c, c2, Ql, d.as<uint64_t>(), s, rounded);
+        bump(g_cnt_inner, Ql, 2);
+        k_ks_inner<<<grid_for(QlP * N), kBlock, 0, s>>>(d.as<uint64_t>(), key, cx.as<uint64_t>(), c.mods(), Ql, c.nQ,
+                                                        c.nQP(), alpha, beta, N);
+        SHM_HIP(hipGetLastError());
+    }
     if (ct1 == ct0 + Ql * N) {
         ks_moddown(c, cx.as<uint64_t>(), 2, Ql, ct0, Ql * N, add_to_ct1 ? 3 : 1, s, rounded);
     } else {
@@ -884,10 +931,12 @@ void keyswitch_batch(const Context &c, const PolyPack &c2, size_t m, const uint6
     const size_t N = c.N, QlP = Ql + c.nP, beta = c.level(Ql).beta;
     if (m == 0 || 2 * m > (size_t)kPolyPack) throw InvalidArgument("keyswitch_batch: 1..32 members");
     Scratch d(m * beta * QlP * N * sizeof(uint64_t), s);
-    ks_modup_batch(c, c2, m, Ql, d.as<uint64_t>(), s, rounded);
     // inner products: each key word read once for the group
     Scratch cx(2 * m * QlP * N * sizeof(uint64_t), s);
-    ks_inner_batch(c, d.as<uint64_t>(), m, Ql, key, cx.as<uint64_t>(), s, nullptr, &c2);
+    if (!modup_inner_fused(c, c2, m, Ql, key, d.as<uint64_t>(), cx.as<uint64_t>(), s, rounded, nullptr)) {
+        ks_modup_batch(c, c2, m, Ql, d.as<uint64_t>(), s, rounded);
+        ks_inner_batch(c, d.as<uint64_t>(), m, Ql, key, cx.as<uint64_t>(), s, nullptr, &c2);
+    }
     // ModDown of the 2m polynomials into the members' (c0, c1)
     ks_moddown_pack(c, cx.as<uint64_t>(), 2 * m, Ql, ct01, acc_mask, s, rounded);
 }
@@ -900,10 +949,12 @@ void keyswitch_rescale_batch(const Context &c, const PolyPack &c2, const PolyPac
     if (nP > (size_t)kMaxAlpha) throw InvalidArgument("at most 16 special primes");
     const LevelConsts &L = c.level(Ql);
     Scratch d(m * beta * QlP * N * sizeof(uint64_t), s);
-    ks_modup_batch(c, c2, m, Ql, d.as<uint64_t>(), s, true);
     // cx = P (d0, d1) + the inner products: the value the merged step divides
     Scratch cx(2 * m * QlP * N * sizeof(uint64_t), s);
-    ks_inner_batch(c, d.as<uint64_t>(), m, Ql, key, cx.as<uint64_t>(), s, nullptr, &c2, &d01);
+    if (!modup_inner_fused(c, c2, m, Ql, key, d.as<uint64_t>(), cx.as<uint64_t>(), s, true, &d01)) {
+        ks_modup_batch(c, c2, m, Ql, d.as<uint64_t>(), s, true);
+        ks_inner_batch(c, d.as<uint64_t>(), m, Ql, key, cx.as<uint64_t>(), s, nullptr, &c2, &d01);
+    }
     // B = {q_last, P}: inverse NTT of those limbs, exact centred conversion to the
     // other Ql - 1 primes, and the NTT of the correction whose last pass writes
     // (cx - delta) B^-1 into the outputs

@@ -242,6 +242,7 @@ void ctpt_matmul_masked(const Context &c, const std::vector<const Ciphertext *> 
     SHM_HIP(hipMemcpyAsync(dmask.as<void>(), mask, n, hipMemcpyHostToDevice, s));
     SHM_HIP(hipMemcpyAsync(dW.as<void>(), W, row_w * col_w * sizeof(double), hipMemcpyHostToDevice, s));
     SHM_HIP(hipMemcpyAsync(dfixj.as<void>(), fixj.data(), row_w * sizeof(double), hipMemcpyHostToDevice, s));
+    const bool fused = rows_mac_covers(c, Ql, false, JB);
     for (size_t c0 = 0; c0 < col_w; c0 += CB) {
         const int cb = (int)std::min(CB, col_w - c0);
         for (size_t j0 = 0; j0 < row_w; j0 += JB) {
@@ -249,7 +250,25 @@ void ctpt_matmul_masked(const Context &c, const std::vector<const Ciphertext *> 
             k_mask_weights<<<1, kBlock, 0, s>>>(dW.as<double>(), dfixj.as<double>(), dw.as<double>(),
                                                  dfix.as<double>(), j0, c0, jb, cb, col_w);
             encode_masked_batch(c, dw.as<double>(), dfix.as<double>(), dmask.as<uint8_t>(), (size_t)(jb * cb), Ql,
-                                pt.as<uint64_t>(), fft.as<double2>(), s);
+                                pt.as<uint64_t>(), fft.as<double2>(), s, !fused);
+            if (fused) {
+                // the plaintexts' row stages, multiplied by the inputs and summed on the way
+                MacJob job{};
+                job.data = pt.as<uint64_t>();
+                job.stride = S;
+                job.groups = (uint32_t)cb;
+                job.terms = (uint32_t)jb;
+                job.ge = 1;
+                job.gt = (uint32_t)cb;
+                job.limbs = job.Ql = (uint32_t)Ql;
+                job.op_stride = S;
+                for (int jj = 0; jj < jb; jj++) job.op.p[jj] = X[j0 + jj]->data();
+                job.out = acc.as<uint64_t>() + c0 * 2 * S;
+                job.out_stride = S;
+                job.accumulate = j0 != 0;
+                rows_mac(c, job, s);
+                continue;
+            }
             XBlock xb{};
             for (int jj = 0; jj < jb; jj++) xb.p[jj] = X[j0 + jj]->data();
             k_mask_mac<<<grid_for(S), kBlock, 0, s>>>(xb, jb, pt.as<uint64_t>(), cb, acc.as<uint64_t>() + c0 * 2 * S,

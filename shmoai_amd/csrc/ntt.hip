@@ -145,7 +145,6 @@ struct HarveyK {
         if (center && v > center) y = sub_mod(y, reduce64(2 * center + 1, m), q);
         return y;
     }
-    __device__ __forceinline__ uint64_t load_rounded(double v, const DevMod &m) const { return residue_of_rounded(v, m); }
     __device__ __forceinline__ uint64_t load_signed(uint64_t v, const DevMod &m) const {
         const bool neg = (int64_t)v < 0;
         const uint64_t y = reduce64(neg ? 0 - v : v, m);
@@ -194,7 +193,6 @@ struct FoldK {
     __device__ __forceinline__ uint64_t load_residue(uint64_t v, uint64_t center, const DevMod &) const {
         return center && v > center ? v - (2 * center + 1) : v;
     }
-    __device__ __forceinline__ uint64_t load_rounded(double v, const DevMod &m) const { return residue_of_rounded(v, m); }
     __device__ __forceinline__ uint64_t load_signed(uint64_t v, const DevMod &) const { return v; }
 };
 
@@ -236,14 +234,10 @@ __device__ __forceinline__ void gs_unit(uint64_t *x, const K &k, TW tw) {
 //   IO_GATHER  : (phase B, inverse) limb k of polynomial p is read from
 //                acc_p.p[p] + k N (separate input buffers) and the transform is
 //                written to `data`: the gather copy fused into the first pass.
-//   IO_ENCODE  : (phase A, forward) the input of limb k of polynomial p is the
-//                rounded coefficient of the encoder's FFT output fft[p] (index
-//                i < N/2: round(re), i >= N/2: round(im) of entry i - N/2) as a
-//                residue, i.e. the encoder's decompose step fused into the load.
 //   IO_DIGITS  : (phase B, forward) polynomial m digits + g is digit g of member m: its own
 //                limbs [g alpha, (g + 1) alpha) below Ql are copied from acc_p.p[m] (copy_own)
 //                or left untouched, the others transformed.
-enum { IO_PLAIN = 0, IO_REDUCE = 1, IO_RESCALE = 2, IO_ENCODE = 3, IO_GATHER = 4, IO_DIGITS = 5 };
+enum { IO_PLAIN = 0, IO_REDUCE = 1, IO_RESCALE = 2, IO_GATHER = 4, IO_DIGITS = 5 };
 
 struct NttIO {
     const uint64_t *src;      // IO_REDUCE: [n_polys][N]
@@ -262,7 +256,6 @@ struct NttIO {
     PolyPack acc_p, out_p;    // IO_RESCALE with packed / out_packed; IO_GATHER inputs in acc_p
     const uint32_t *add_perm; // IO_RESCALE with out_packed: add add_src.p[p] read through this
     PolyPack add_src;         // NTT-domain permutation instead of out_p[p] (acc_mask bit p set)
-    const double2 *fft;       // IO_ENCODE: [n_polys][N/2]
     const uint64_t *scale;    // inverse, phase A: limb k is multiplied by scale[k - scale_lo]
     const uint64_t *scale_s;  // (value, Shoup companion) instead of N^-1, unless null
     uint32_t scale_lo;
@@ -310,16 +303,6 @@ __device__ __forceinline__ void col_pass(const K &k, uint64_t *lds, uint64_t *ba
 #pragma unroll
             for (int l = 0; l < (1 << RA); l++)
                 x[l] = k.load_residue(src[(size_t)(r0 + (l << RB)) * kRow], io.center, m);
-        } else if (IO == IO_ENCODE) {
-            const DevMod m = tb.mods[prime];
-            const double2 *fb = io.fft + (size_t)poly * (N / 2) + c;
-            // rows below N1/2 are real parts; row r + N1/2 is the imaginary part of the same entry
-#pragma unroll
-            for (int l = 0; l < (1 << RA) / 2; l++) {
-                const double2 v = fb[(size_t)(r0 + (l << RB)) * kRow];
-                x[l] = k.load_rounded(round(v.x), m);
-                x[l + (1 << RA) / 2] = k.load_rounded(round(v.y), m);
-            }
         } else {
 #pragma unroll
             for (int l = 0; l < (1 << RA); l++) x[l] = base[(size_t)(r0 + (l << RB)) * kRow + c];
@@ -416,11 +399,25 @@ __global__ __launch_bounds__(kThreads, 2) void k_convert_cols(ConvertJob job, Nt
     auto prime_of = [&](uint32_t k) { return k < job.Ql ? k : nQ + (k - job.Ql); };
     // source words in halves, and each coefficient's rounding (at most A < 16) in 4 bits
     uint32_t yl[A][U], yh[A][U], r[(U + 7) / 8] = {};
+    bool big = false;
     {
         uint64_t y[A][U];
         double v[U];
 #pragma unroll
         for (int l = 0; l < U; l++) v[l] = 0.0;
+        if (A == 1 && job.fft) {
+            // rounded encoder coefficients: rows below N1 / 2 are real parts, row r + N1 / 2 the
+            // imaginary part of the same entry. Those of 2^60 and more are reduced per prime.
+            const double2 *fb = job.fft + (size_t)poly * (N / 2) + c;
+#pragma unroll
+            for (int l = 0; l < U; l++) {
+                const uint32_t row = r0 + (l << RB);
+                const double2 z = fb[(size_t)(row & (N1 / 2 - 1)) * kRow];
+                const double t = round(row < N1 / 2 ? z.x : z.y);
+                big = big || !(fabs(t) < 1152921504606846976.0);
+                y[0][l] = (uint64_t)(int64_t)t;
+            }
+        } else
 #pragma unroll
         for (int i = 0; i < A; i++) {
             if ((uint32_t)i < size) {
@@ -488,6 +485,18 @@ __global__ __launch_bounds__(kThreads, 2) void k_convert_cols(ConvertJob job, Nt
                 if (!FAST) m = tb.mods[prime];
 #pragma unroll
                 for (int l = 0; l < U; l++) x[l] = kk.load_signed(((uint64_t)yh[0][l] << 32) | yl[0][l], m);
+                if (big) {
+                    const double2 *fb = job.fft + (size_t)poly * (N / 2) + c;
+                    const DevMod mp = tb.mods[prime];
+#pragma unroll 1
+                    for (int l = 0; l < U; l++) {
+                        const uint32_t row = r0 + (l << RB);
+                        const double2 z = fb[(size_t)(row & (N1 / 2 - 1)) * kRow];
+                        const uint64_t t = residue_of_rounded(round(row < N1 / 2 ? z.x : z.y), mp);
+#pragma unroll
+                        for (int i = 0; i < U; i++) x[i] = i == l ? t : x[i];
+                    }
+                }
             } else if constexpr (FAST) {
                 const auto cv = table_ptr(job.conv + ((size_t)g * job.n_out + k) * (job.alpha + 1));
                 u32x4 w[A + 1];
@@ -557,74 +566,72 @@ __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// Row pass: one wave per row of 512 words, 8 words per lane. Unit words of a lane: round 1
-// lane + 64 l; round 2 64 (lane / 8) + lane % 8 + 8 l; round 3 8 lane + l.
+// Unit words of a lane: round 1 lane + 64 l; round 2 64 (lane / 8) + lane % 8 + 8 l; round 3
+// 8 lane + l.
+struct RowWords {
+    uint64_t *lds;
+    int i1, i2, i3;
+    __device__ RowWords(uint64_t *l, int lane)
+        : lds(l), i1(row_slot(lane)), i2(row_slot(64 * (lane >> 3) + (lane & 7))), i3(9 * lane) {}
+    template <int STEP>
+    __device__ __forceinline__ void put(int i, const uint64_t *x) const {
+#pragma unroll
+        for (int l = 0; l < 8; l++) lds[i + STEP * l] = x[l];
+    }
+    template <int STEP>
+    __device__ __forceinline__ void get(int i, uint64_t *x) const {
+        wave_lds_order();
+#pragma unroll
+        for (int l = 0; l < 8; l++) x[l] = lds[i + STEP * l];
+        wave_lds_order();
+    }
+};
+
+// The forward row stages of x (words lane + 64 l); the results are left in LDS.
+template <typename K, typename T1, typename T2, typename T3, typename H>
+__device__ __forceinline__ void row_forward(const K &k, const RowWords &w, uint64_t (&x)[8], T1 tw1, T2 tw2, T3 tw3,
+                                            H before_last) {
+    ct_unit<3>(x, k, tw1);
+    w.template put<72>(w.i1, x);
+    w.template get<9>(w.i2, x);
+    ct_unit<3>(x, k, tw2);
+    w.template put<9>(w.i2, x);
+    before_last();
+    w.template get<1>(w.i3, x);
+    ct_unit<3>(x, k, tw3);
+    w.template put<1>(w.i3, x);
+    wave_lds_order();
+}
+
+// Row pass: one wave per row of 512 words, 8 words per lane.
 template <bool FWD, int IO, typename K>
-__device__ __forceinline__ void row_pass(const K &k, uint64_t *lds, uint64_t *base, const u32x4 *__restrict__ tw,
-                                         const u32x4 *w2, const u32x4 (&w3)[7], uint64_t (&x)[8],
-                                         const NttTables &tb, uint32_t prime, uint32_t poly, uint32_t limb,
+__device__ __forceinline__ void row_pass(const K &k, uint64_t *lds, uint64_t *base, const u32x4 *w2,
+                                         const u32x4 (&w3)[7], uint64_t (&x)[8], uint32_t poly, uint32_t limb,
                                          uint32_t row0, uint32_t n_active, size_t N, int lane, const NttIO &io,
                                          const typename K::Const &qi) {
-    const int i1 = row_slot(lane), i2 = row_slot(64 * (lane >> 3) + (lane & 7)), i3 = 9 * lane;
+    const RowWords w(lds, lane);
     auto tw1 = [&](int e) { return w2[e]; };
     auto tw2 = [&](int e) { return w2[8 + 8 * e + (lane >> 3)]; };
     auto tw3 = [&](int e) { return w3[e]; };
-    auto put1 = [&](const uint64_t *x) {
-#pragma unroll
-        for (int l = 0; l < 8; l++) lds[i1 + 72 * l] = x[l];
-    };
-    auto put2 = [&](const uint64_t *x) {
-#pragma unroll
-        for (int l = 0; l < 8; l++) lds[i2 + 9 * l] = x[l];
-    };
-    auto put3 = [&](const uint64_t *x) {
-#pragma unroll
-        for (int l = 0; l < 8; l++) lds[i3 + l] = x[l];
-    };
-    auto get1 = [&](uint64_t *x) {
-        wave_lds_order();
-#pragma unroll
-        for (int l = 0; l < 8; l++) x[l] = lds[i1 + 72 * l];
-    };
-    auto get2 = [&](uint64_t *x) {
-        wave_lds_order();
-#pragma unroll
-        for (int l = 0; l < 8; l++) x[l] = lds[i2 + 9 * l];
-    };
-    auto get3 = [&](uint64_t *x) {
-        wave_lds_order();
-#pragma unroll
-        for (int l = 0; l < 8; l++) x[l] = lds[i3 + l];
-    };
+    auto pair_of = [&](int j) { return 2 * lane + 128 * j; };  // words i, i + 1
     if constexpr (!FWD) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int i = 2 * lane + 128 * j;
-            lds[row_slot(i)] = x[2 * j];
-            lds[row_slot(i) + 1] = x[2 * j + 1];
+            lds[row_slot(pair_of(j))] = x[2 * j];
+            lds[row_slot(pair_of(j)) + 1] = x[2 * j + 1];
         }
-        get3(x);
+        w.template get<1>(w.i3, x);
         gs_unit<3>(x, k, tw3);
-        wave_lds_order();
-        put3(x);
-        get2(x);
+        w.template put<1>(w.i3, x);
+        w.template get<9>(w.i2, x);
         gs_unit<3>(x, k, tw2);
-        wave_lds_order();
-        put2(x);
-        get1(x);
+        w.template put<9>(w.i2, x);
+        w.template get<72>(w.i1, x);
         gs_unit<3>(x, k, tw1);
 #pragma unroll
         for (int l = 0; l < 8; l++) base[lane + 64 * l] = x[l];
         return;
     }
-    ct_unit<3>(x, k, tw1);
-    put1(x);
-    get2(x);
-    ct_unit<3>(x, k, tw2);
-    wave_lds_order();
-    put2(x);
-    // rescale: the accumulator words are loaded before the last round, so they arrive during
-    // it; outputs leave in 16-byte pairs
     const uint64_t *accp = nullptr;
     uint64_t *out = base;
     if (IO == IO_RESCALE) {
@@ -637,18 +644,16 @@ __device__ __forceinline__ void row_pass(const K &k, uint64_t *lds, uint64_t *ba
             out = ob + ((size_t)(poly % io.ppo) * (io.out_limbs ? io.out_limbs : n_active) + limb) * N + row0;
         }
     }
-    auto pair_of = [&](int j) { return 2 * lane + 128 * j; };  // words i, i + 1
+    // rescale: the accumulator words are loaded before the last round, so they arrive during
+    // it; outputs leave in 16-byte pairs
     u64x2 accv[IO == IO_RESCALE ? 4 : 1];
-    if (IO == IO_RESCALE) {
+    row_forward(k, w, x, tw1, tw2, tw3, [&] {
+        if (IO == IO_RESCALE) {
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            accv[j] = __builtin_nontemporal_load(global_ptr(reinterpret_cast<const u64x2 *>(accp + pair_of(j))));
-    }
-    get3(x);
-    ct_unit<3>(x, k, tw3);
-    wave_lds_order();
-    put3(x);
-    wave_lds_order();
+            for (int j = 0; j < 4; j++)
+                accv[j] = __builtin_nontemporal_load(global_ptr(reinterpret_cast<const u64x2 *>(accp + pair_of(j))));
+        }
+    });
     const bool addto = IO == IO_RESCALE && io.out_packed && poly < 64 && ((io.acc_mask >> poly) & 1);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -745,8 +750,7 @@ __global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data,
 #pragma unroll
                     for (int l = 0; l < 8; l++) __builtin_nontemporal_store(x[l], base + lane + 64 * l);
             } else {
-                row_pass<FWD, IO>(k, lds[wave], base, tw, w2, w3, x, tb, prime, p, limb, row0, mp.n_active, N, lane, io,
-                                  qi);
+                row_pass<FWD, IO>(k, lds[wave], base, w2, w3, x, p, limb, row0, mp.n_active, N, lane, io, qi);
             }
             wave_lds_order();
 #pragma unroll
@@ -760,6 +764,110 @@ __global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data,
             loop(FoldK<true>(tb, prime));
         else
             loop(HarveyK(tb, prime));
+    }
+}
+
+// Row stages fused with the products that consume them (MacJob): a wave takes one row of one
+// limb for one group, runs the row stages of each term's polynomial and multiplies its words
+// by two operand rows into split sums (Acc52), so transformed words never reach memory. The
+// next term's words and this term's operand rows are requested before the stages. Per wave 8
+// KB of twiddles and 4.6 KB of exchange in LDS; 96 registers hold the sums, 2 waves per SIMD.
+// Groups of one row are neighbours in launch order, so operand rows that groups share (a
+// key's, or the inputs' of a product) come from L2 after the first. Bound by VALU issue (about
+// 480 slots per term and word group). Against row pass and product kernels apart at N = 2^16:
+// one top-level rotation's 66 + 96 us in 102; relinearisations of 16 members, 18 per shared-a
+// chunk, 20.7 ms in 15.2; 128 masked plaintexts of 24 limbs 500 + 517 us in 660.
+template <bool KEY>
+__global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, int logN, uint32_t nQ, uint32_t per_xcd) {
+    __shared__ uint64_t lds[4][kRowLds];
+    __shared__ __align__(16) u32x4 ltw[4][kRow];
+    const size_t N = size_t(1) << logN;
+    const uint32_t rows = (uint32_t)(N / kRow);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t O = ((blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3)) * 4 + wave;
+    if (O >= job.groups * job.limbs * rows) return;  // no barrier in this kernel
+    const uint32_t e = O % job.groups, rest = O / job.groups, row0 = rest % rows * kRow, limb = rest / rows;
+    const uint32_t prime = limb < job.Ql ? limb : nQ + (limb - job.Ql);
+    const size_t at = (size_t)limb * N + row0;
+    const FoldK<false> k(tb, prime);
+    {
+        const u32x4 *tw = tb.row + (size_t)prime * N + row0;
+#pragma unroll
+        for (int j = 0; j < 8; j++) ltw[wave][lane + 64 * j] = tw[lane + 64 * j];
+    }
+    const u32x4 *lt = ltw[wave];
+    const RowWords w(lds[wave], lane);
+    auto pair_of = [&](int j) { return 2 * lane + 128 * j; };
+    auto own = [&](uint32_t t) { return KEY && limb < job.Ql && limb / job.alpha == t; };
+    auto load = [&](uint64_t (&x)[8], uint32_t t) {
+        if (own(t)) return;
+        const uint64_t *p = job.data + (size_t)(e * job.ge + t * job.gt) * job.stride + at;
+#pragma unroll
+        for (int l = 0; l < 8; l++) x[l] = __builtin_nontemporal_load(global_ptr(p + lane + 64 * l));
+    };
+    uint64_t x[8], nx[8];
+    Acc52 acc[2][8];
+#pragma unroll
+    for (int o = 0; o < 2; o++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[o][j] = Acc52{0, 0, 0};
+    load(x, 0);
+    for (uint32_t t = 0; t < job.terms; t++) {
+        if (t + 1 < job.terms) load(nx, t + 1);
+        const uint64_t *op = KEY ? job.key + (size_t)t * 2 * job.op_stride + (size_t)prime * N + row0 : job.op.p[t] + at;
+        u64x2 a[2][4];
+#pragma unroll
+        for (int o = 0; o < 2; o++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                a[o][j] = *global_ptr(reinterpret_cast<const u64x2 *>(op + o * job.op_stride + pair_of(j)));
+        u64x2 y[4];
+        if (own(t)) {
+            const uint64_t *p = job.op.p[e] + at;
+#pragma unroll
+            for (int j = 0; j < 4; j++) y[j] = *global_ptr(reinterpret_cast<const u64x2 *>(p + pair_of(j)));
+        } else {
+            wave_lds_order();
+            row_forward(k, w, x, [&](int i) { return lt[i]; }, [&](int i) { return lt[8 + 8 * i + (lane >> 3)]; },
+                        [&](int i) { return lt[64 + 64 * i + lane]; }, [] {});
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int i = row_slot(pair_of(j));
+                y[j] = u64x2{fold_positive(lds[wave][i], k.f), fold_positive(lds[wave][i + 1], k.f)};
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const Split26 s0 = split26(y[j].x), s1 = split26(y[j].y);
+#pragma unroll
+            for (int o = 0; o < 2; o++) {
+                mac52(acc[o][2 * j], s0, a[o][j].x);
+                mac52(acc[o][2 * j + 1], s1, a[o][j].y);
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < 8; l++) x[l] = nx[l];
+    }
+    const DevMod m = tb.mods[prime];
+#pragma unroll
+    for (int o = 0; o < 2; o++) {
+        uint64_t *out = job.out + (size_t)(2 * e + o) * job.out_stride + at;
+        const bool add_on = KEY && job.add_on && limb < job.Ql;
+        const uint64_t *add = add_on ? job.add.p[2 * e + o] + at : nullptr;
+        const uint64_t pm = add_on ? job.pmod[limb] : 0, pms = add_on ? job.pmod_s[limb] : 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const auto at2 = global_ptr(reinterpret_cast<u64x2 *>(out + pair_of(j)));
+            u64x2 v = {reduce52(acc[o][2 * j], m), reduce52(acc[o][2 * j + 1], m)};
+            if (job.accumulate) {
+                const u64x2 c = *at2;
+                v = u64x2{add_mod(v.x, c.x, m.q), add_mod(v.y, c.y, m.q)};
+            } else if (add_on) {
+                const u64x2 c = *global_ptr(reinterpret_cast<const u64x2 *>(add + pair_of(j)));
+                v = u64x2{add_mod(v.x, mul_shoup(c.x, pm, pms, m.q), m.q), add_mod(v.y, mul_shoup(c.y, pm, pms, m.q), m.q)};
+            }
+            __builtin_nontemporal_store(v, at2);
+        }
     }
 }
 
@@ -779,6 +887,13 @@ struct FusedProbe {
     size_t last_plain_launches = 0;
     double last_plain_ms = 0.0, last_plain_bytes = 0.0;
 } g_probe;
+
+// Whether the limb's prime has a split form, one fold of a word ends below 2q, and an input of
+// magnitude `in` plus log N products (and one residue) fit a signed word.
+bool forward_fits(const Context &c, uint32_t prime, uint64_t in) {
+    const uint64_t q = c.q.at(prime), r = c.fold_bound.at(prime), top = (uint64_t(1) << 63) - 1 - 2 * q;
+    return r != 0 && !c.fold_twice.at(prime) && in < top && r <= (top - in) / (uint64_t)c.logN;
+}
 
 template <bool FWD, int IOA, int IOB>
 void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t total_limbs, hipStream_t s,
@@ -808,10 +923,10 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
         if (k >= mp.skip_lo) k += mp.skip_width;
         const uint32_t prime = k < mp.Ql ? mp.first_prime + k : mp.nQ + (k - mp.Ql);
         const uint64_t q = c.q.at(prime), r = c.fold_bound.at(prime);
-        const uint64_t in = IOA == IO_REDUCE ? std::max(q_any, 4 * q) : 4 * q;
-        const uint64_t top = (uint64_t(1) << 63) - 1 - 2 * q;
-        fast = r != 0 && !c.fold_twice.at(prime) && (FWD ? in < top && r <= (top - in) / (uint64_t)logN
-                              : r < (uint64_t(1) << (63 - std::max(unit, 3))));
+        if (FWD)
+            fast = forward_fits(c, prime, IOA == IO_REDUCE ? std::max(q_any, 4 * q) : 4 * q);
+        else
+            fast = r != 0 && !c.fold_twice.at(prime) && r < (uint64_t(1) << (63 - std::max(unit, 3)));
     }
     // the row pass moves its words in 16-byte pairs (outs are ciphertext buffers of the pool)
     bool aligned = ((uintptr_t)data & 15) == 0 && mp.poly_stride % 2 == 0;
@@ -1006,12 +1121,44 @@ void set_rescale_tile_events(hipEvent_t start, hipEvent_t stop) {
     g_rescale_tile_ev[1] = stop;
 }
 
+void ntt_encoded_columns(const Context &c, const double2 *fft, uint64_t *out, size_t n_polys, size_t n_limbs,
+                         hipStream_t s) {
+    ConvertJob job{};
+    job.fft = fft;
+    job.alpha = job.total = job.digits = 1;
+    job.members = (uint32_t)n_polys;
+    job.out = out;
+    job.out_stride = n_limbs * c.N;
+    job.n_out = job.Ql = (uint32_t)n_limbs;
+    convert_cols(c, job, s);
+}
+
 void ntt_forward_encoded(const Context &c, const double2 *fft, uint64_t *out, size_t n_polys, size_t n_limbs,
                          hipStream_t s) {
+    ntt_encoded_columns(c, fft, out, n_polys, n_limbs, s);
     LimbMap mp{(uint32_t)n_limbs, 0, 0xffffffffu, 0, 0xffffffffu, (uint32_t)c.nQ, 0, (uint64_t)n_limbs * c.N};
-    NttIO io{};
-    io.fft = fft;
-    launch_ntt<true, IO_ENCODE, IO_PLAIN>(c, out, mp, n_polys * n_limbs, s, io);
+    launch_ntt<true, IO_PLAIN, IO_PLAIN>(c, out, mp, n_polys * n_limbs, s, NttIO{}, true);
+}
+
+bool rows_mac_covers(const Context &c, size_t n_data, bool special, size_t terms) {
+    if (terms == 0 || terms > 16) return false;
+    for (size_t p = 0; p < n_data + (special ? c.nP : 0); p++) {
+        const uint32_t prime = (uint32_t)(p < n_data ? p : c.nQ + (p - n_data));
+        const uint64_t q = c.q.at(prime);
+        if (!(q > (uint64_t(1) << 45) && q < (uint64_t(1) << 52)) || !forward_fits(c, prime, uint64_t(1) << 61)) return false;
+    }
+    return true;
+}
+
+void rows_mac(const Context &c, const MacJob &job, hipStream_t s) {
+    NttTables tb{c.mods(), c.d_fold.as<FoldMod>(), nullptr, c.tw_row.as<u32x4>(), nullptr, nullptr};
+    const size_t waves = (size_t)job.groups * job.limbs * (c.N / kRow);
+    const uint32_t per_xcd = (uint32_t)((waves + 31) / 32);
+    if (job.key)
+        k_rows_mac<true><<<8u * per_xcd, 256, 0, s>>>(job, tb, c.logN, (uint32_t)c.nQ, per_xcd);
+    else
+        k_rows_mac<false><<<8u * per_xcd, 256, 0, s>>>(job, tb, c.logN, (uint32_t)c.nQ, per_xcd);
+    SHM_HIP(hipGetLastError());
 }
 
 void ntt_inverse(const Context &c, uint64_t *data, size_t n_polys, size_t n_limbs, size_t first_prime,
@@ -1115,9 +1262,11 @@ void convert_cols(const Context &c, const ConvertJob &job, hipStream_t s) {
     const int logN = c.logN, stages = logN - 9;
     NttTables tb{c.mods(), c.d_fold.as<FoldMod>(), c.tw_col.as<u32x4>(), nullptr, nullptr, nullptr};
     const unsigned polys = job.members * job.digits;
-    // one source limb: the word is below 2^61, any sum of products is folded (GENERAL) unless
-    // conv_ok says they all fit
-    const bool fast = c.conv_ok;
+    // one source word: below 2^61 (2^60 from the encoder), and its transform fits or GENERAL
+    // kernels fold; more: conv_ok
+    bool fast = true;
+    for (uint32_t k = 0; k < job.n_out && job.alpha == 1 && fast; k++)
+        fast = forward_fits(c, k < job.Ql ? k : (uint32_t)c.nQ + (k - job.Ql), uint64_t(1) << (job.fft ? 60 : 61));
     auto launch = [&](auto fn, int width) {
         const unsigned blocks = (unsigned)(kRow / width) * polys;
         // a run of output limbs per block, shorter (but at least 4) where that leaves fewer

@@ -42,3 +42,18 @@ def test_decode_matches_oracle(oracle_lib, Ql, size):
     re, im = ref.decode(pt_words, Ql, scale)
     want = re + 1j * im
     assert np.max(np.abs(got - want)) <= 1e-12 * max(np.max(np.abs(want)), 1e-300)
+
+
+@pytest.mark.parametrize("bits", [[51] + [46] * 4 + [51], [50] * 3 + [60]], ids=["split", "mixed"])
+@pytest.mark.parametrize("scale", [2.0 ** 30, 2.0 ** 58, 2.0 ** 61, 2.0 ** 90])
+def test_encode_matches_oracle(oracle_lib, bits, scale):
+    """Coefficients below, around and above the 2^60 up to which they travel as one signed
+    word; above, each prime reduces them by itself. Whole words, bit-exact."""
+    import shmoai_amd as shm
+    ctx = shm.Context(13, bits, 1)
+    ref = oracle_lib.Ref(13, bits, 1)
+    Ql, n = len(bits) - 1, ref.N // 2
+    # one slot vector with a large constant coefficient beside small ones, one with all alike
+    for v in (np.concatenate([[3.75], np.zeros(n - 1)]), np.full(n, -1.625)):
+        got = shm.Encoder(ctx).encode(v, scale, 1).numpy()
+        assert np.array_equal(got, ref.encode(v, Ql, scale))

@@ -19,6 +19,9 @@ CASES = [
     (16, [51] + [46] * 9 + [51] * 5, 5, 10),
     (17, [51] + [46] * 3 + [51] * 2, 2, 3),
     (16, [40] * 3 + [50], 1, 3),
+    # 16 rows of limbs and more: row stages fused with the products (7 digits; a last digit of one)
+    (16, [51] + [46] * 13 + [51, 51], 2, 14),
+    (16, [51] + [46] * 15 + [51] * 4, 4, 13),
 ]
 
 
