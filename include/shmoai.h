@@ -121,6 +121,9 @@ int shm_ntt_inverse(shm_context *ctx, uint64_t *data, uint32_t n_polys, uint32_t
 /* ---- ciphertexts / plaintexts (PhantomCiphertext ciphertext.h:21-288,
  * PhantomPlaintext plaintext.h) -------------------------------------------- */
 int shm_ciphertext_create(shm_context *ctx, uint32_t size, uint32_t chain_index, shm_ciphertext **out);
+/* The same without the zero fill: for the output of a call that writes every word (a copy,
+ * an encryption, a matrix product, a bootstrap); its words are unspecified until then. */
+int shm_ciphertext_create_unfilled(shm_context *ctx, uint32_t size, uint32_t chain_index, shm_ciphertext **out);
 int shm_ciphertext_destroy(shm_ciphertext *ct);
 int shm_ciphertext_info(const shm_ciphertext *ct, uint32_t *size, uint32_t *chain_index, uint32_t *coeff_mod_size,
                         double *scale);

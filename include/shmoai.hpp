@@ -113,7 +113,7 @@ class PhantomCiphertext {
     ~PhantomCiphertext() { release(); }
     PhantomCiphertext(const PhantomCiphertext &o) : ctx_(o.ctx_) {
         if (o.h_) {
-            shm_check(shm_ciphertext_create(ctx_->handle(), o.size(), o.chain_index(), &h_));
+            shm_check(shm_ciphertext_create_unfilled(ctx_->handle(), o.size(), o.chain_index(), &h_));
             shm_check(shm_ciphertext_copy(o.h_, h_, nullptr));
         }
     }

@@ -92,6 +92,16 @@ class Ciphertext:
         check(_lib().shm_ciphertext_create(ctx.h, size, chain_index, C.byref(h)))
         self.h = h
 
+    @classmethod
+    def _output(cls, ctx: Context, size: int = 2, chain_index: int = 1) -> "Ciphertext":
+        """A ciphertext for a call that writes every word (no zero fill)."""
+        ct = cls.__new__(cls)
+        ct.ctx = ctx
+        h = C.c_void_p()
+        check(_lib().shm_ciphertext_create_unfilled(ctx.h, size, chain_index, C.byref(h)))
+        ct.h = h
+        return ct
+
     def __del__(self):
         try:
             if getattr(self, "h", None):
@@ -145,7 +155,7 @@ class Ciphertext:
 
     def copy(self, stream=None) -> "Ciphertext":
         s, ch, _, _ = self.info()
-        out = Ciphertext(self.ctx, s, ch)
+        out = Ciphertext._output(self.ctx, s, ch)
         check(_lib().shm_ciphertext_copy(self.h, out.h, stream))
         return out
 
@@ -289,7 +299,7 @@ class SecretKey:
         return PublicKey(self.ctx, h)
 
     def encrypt_symmetric(self, pt: Plaintext, seed: int, stream=None) -> Ciphertext:
-        ct = Ciphertext(self.ctx, 2, pt.chain_index)
+        ct = Ciphertext._output(self.ctx, 2, pt.chain_index)
         check(_lib().shm_encrypt_symmetric(self.ctx.h, self.h, pt.h, seed, ct.h, stream))
         return ct
 
@@ -322,7 +332,7 @@ class Encryptor:
         self.ctx, self.pk = ctx, pk
 
     def encrypt(self, pt: "Plaintext", seed: int, stream=None) -> "Ciphertext":
-        ct = Ciphertext(self.ctx, 2, 1)
+        ct = Ciphertext._output(self.ctx, 2, 1)
         check(_lib().shm_encrypt_asymmetric(self.ctx.h, self.pk.h, pt.h, seed, ct.h, stream))
         return ct
 
@@ -332,7 +342,7 @@ def batch_input(X: np.ndarray, scale: float, ctx: Context, pk: PublicKey, seed: 
     num_col ciphertexts, column i packed as slot num_X * k + j = X[j][k][i]."""
     X = np.ascontiguousarray(X, np.float64)
     num_x, num_row, num_col = X.shape
-    out = [Ciphertext(ctx, 2, 1) for _ in range(num_col)]
+    out = [Ciphertext._output(ctx, 2, 1) for _ in range(num_col)]
     hs = (C.c_void_p * max(num_col, 1))(*[o.h.value for o in out])
     check(_lib().shm_batch_input(ctx.h, pk.h, X.ctypes.data_as(C.POINTER(C.c_double)), num_x, num_row, num_col,
                                  float(scale), seed, hs, stream))
@@ -597,7 +607,7 @@ class Bootstrapper:
     def bootstrap_s2c_first(self, cts: Sequence[Ciphertext], gk: GaloisKeys, relin_key: KSwitchKey,
                             out_scale: float = 0.0, stream=None, out=None) -> list:
         """Enqueue-only; `out` reuses existing output ciphertexts."""
-        out = [Ciphertext(self.ctx, 2, 1) for _ in cts] if out is None else out
+        out = [Ciphertext._output(self.ctx, 2, 1) for _ in cts] if out is None else out
         ins = (C.c_void_p * len(cts))(*[c.h.value for c in cts])
         outs = (C.c_void_p * len(cts))(*[o.h.value for o in out])
         check(_lib().shm_bootstrap_s2c_first(self.h, ins, len(cts), outs, gk.h, relin_key.h, out_scale, stream))
@@ -682,7 +692,7 @@ def ct_pt_matrix_mul_wo_pre(enc_X: Sequence[Ciphertext], W: np.ndarray, col_X: i
         raise capi.ShmInvalidArgument(capi.SHM_ERR_INVALID_ARGUMENT, "enc_X size < row_W")
     chain = enc_X[0].chain_index
     if out is None:
-        out = [Ciphertext(context, 2, chain + 1) for _ in range(col_W)]
+        out = [Ciphertext._output(context, 2, chain + 1) for _ in range(col_W)]
     xs = (C.c_void_p * row_W)(*[x.h.value for x in enc_X[:row_W]])
     os_ = (C.c_void_p * col_W)(*[o.h.value for o in out])
     check(_lib().shm_ct_pt_matrix_mul(context.h, xs, row_W, Wm.ctypes.data_as(C.POINTER(C.c_double)), col_W, os_,
@@ -717,7 +727,7 @@ def ct_pt_matrix_mul_wo_pre_w_mask(enc_X: Sequence[Ciphertext], W: np.ndarray, b
     bv = np.ascontiguousarray(bias_vec, np.int32)
     chain = enc_X[0].chain_index
     if out is None:
-        out = [Ciphertext(context, 2, chain + 1) for _ in range(col_W)]
+        out = [Ciphertext._output(context, 2, chain + 1) for _ in range(col_W)]
     xs = (C.c_void_p * row_W)(*[x.h.value for x in enc_X[:row_W]])
     os_ = (C.c_void_p * col_W)(*[o.h.value for o in out])
     check(_lib().shm_ct_pt_matrix_mul_masked(context.h, xs, row_W, Wm.ctypes.data_as(C.POINTER(C.c_double)), col_W,
@@ -738,7 +748,7 @@ def ct_ct_matrix_mul_colpacking(enc_X: Sequence[Ciphertext], enc_W: Sequence[Cip
         raise capi.ShmInvalidArgument(capi.SHM_ERR_INVALID_ARGUMENT, "enc_X / enc_W hold fewer than col_X ciphertexts")
     chain = enc_X[0].chain_index
     if out is None:
-        out = [Ciphertext(context, 2, chain + 1) for _ in range(row_X)]
+        out = [Ciphertext._output(context, 2, chain + 1) for _ in range(row_X)]
     xs = (C.c_void_p * col_X)(*[x.h.value for x in enc_X[:col_X]])
     ws = (C.c_void_p * col_X)(*[w.h.value for w in enc_W[:col_X]])
     os_ = (C.c_void_p * row_X)(*[o.h.value for o in out])
@@ -758,7 +768,7 @@ def ct_ct_matrix_mul_diagpacking(enc_X: Sequence[Ciphertext], enc_W: Sequence[Ci
         raise capi.ShmInvalidArgument(capi.SHM_ERR_INVALID_ARGUMENT, "enc_X / enc_W hold too few ciphertexts")
     chain = enc_X[0].chain_index
     if out is None:
-        out = [Ciphertext(context, 2, chain + 1) for _ in range(col_W)]
+        out = [Ciphertext._output(context, 2, chain + 1) for _ in range(col_W)]
     xs = (C.c_void_p * col_X)(*[x.h.value for x in enc_X[:col_X]])
     ws = (C.c_void_p * col_W)(*[w.h.value for w in enc_W[:col_W]])
     os_ = (C.c_void_p * col_W)(*[o.h.value for o in out])
@@ -1036,7 +1046,7 @@ def bootstrap_shared_a_s2c_first(boot: "Bootstrapper", keys: SharedAKeys, cts: S
                                  relin_key: KSwitchKey, out_scale: float = 0.0, stream=None, out=None) -> list:
     """BatchBootstrap.cuh:719-820: shared-a S2C-first bootstrap of exactly keys.n ciphertexts
     (enqueue-only; `out` reuses existing output ciphertexts)."""
-    out = [Ciphertext(keys.ctx, 2, 1) for _ in cts] if out is None else out
+    out = [Ciphertext._output(keys.ctx, 2, 1) for _ in cts] if out is None else out
     check(_lib().shm_bootstrap_shared_a_s2c_first(boot.h, keys.h, _ptrs(cts), len(cts), _ptrs(out), relin_key.h,
                                                   out_scale, stream))
     return out
@@ -1046,7 +1056,7 @@ def bootstrap_shared_a_s2c_first_chunks(boot: "Bootstrapper", keys: SharedAKeys,
                                         relin_key: KSwitchKey, out_scale: float = 0.0, stream=None,
                                         out=None) -> list:
     """The shared-a bootstrap over k * keys.n ciphertexts, k chunks in order (enqueue-only)."""
-    out = [Ciphertext(keys.ctx, 2, 1) for _ in cts] if out is None else out
+    out = [Ciphertext._output(keys.ctx, 2, 1) for _ in cts] if out is None else out
     check(_lib().shm_bootstrap_shared_a_s2c_first_chunks(boot.h, keys.h, _ptrs(cts), len(cts), _ptrs(out),
                                                          relin_key.h, out_scale, stream))
     return out

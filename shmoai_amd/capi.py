@@ -62,6 +62,7 @@ _SIGS = {
     "shm_ntt_forward": (i32, [vp, vp, u32, u32, u32, vp]),
     "shm_ntt_inverse": (i32, [vp, vp, u32, u32, u32, vp]),
     "shm_ciphertext_create": (i32, [vp, u32, u32, pvp]),
+    "shm_ciphertext_create_unfilled": (i32, [vp, u32, u32, pvp]),
     "shm_ciphertext_destroy": (i32, [vp]),
     "shm_ciphertext_info": (i32, [vp, C.POINTER(u32), C.POINTER(u32), C.POINTER(u32), C.POINTER(dbl)]),
     "shm_ciphertext_set_scale": (i32, [vp, dbl]),

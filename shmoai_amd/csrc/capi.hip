@@ -241,7 +241,7 @@ int shm_ntt_inverse(shm_context *ctx, uint64_t *data, uint32_t n_polys, uint32_t
 }
 
 // ---- ciphertexts / plaintexts ------------------------------------------------
-int shm_ciphertext_create(shm_context *ctx, uint32_t size, uint32_t chain, shm_ciphertext **out) {
+static int ciphertext_create(shm_context *ctx, uint32_t size, uint32_t chain, shm_ciphertext **out, bool zero) {
     return guard([&] {
         need(ctx, "ctx");
         need(out, "out");
@@ -250,13 +250,21 @@ int shm_ciphertext_create(shm_context *ctx, uint32_t size, uint32_t chain, shm_c
         auto h = new shm_ciphertext();
         h->ct.ctx = ctx->c.get();
         try {
-            h->ct.resize(size, chain);
+            h->ct.resize(size, chain, nullptr, zero);
         } catch (...) {
             delete h;
             throw;
         }
         *out = h;
     });
+}
+
+int shm_ciphertext_create(shm_context *ctx, uint32_t size, uint32_t chain, shm_ciphertext **out) {
+    return ciphertext_create(ctx, size, chain, out, true);
+}
+
+int shm_ciphertext_create_unfilled(shm_context *ctx, uint32_t size, uint32_t chain, shm_ciphertext **out) {
+    return ciphertext_create(ctx, size, chain, out, false);
 }
 
 int shm_ciphertext_destroy(shm_ciphertext *ct) {
