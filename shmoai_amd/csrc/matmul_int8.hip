@@ -10,8 +10,9 @@
 // so Y = sum_d 256^d C_d + 128 * R * rowsum_i with C_d = sum_{a+b=d} W_b X'_a
 // and R = sum_a 256^a. Each W_b X'_a is a 16x16x64 int8 MFMA GEMM
 // accumulating straight into the int32 plane C_{a+b} (|C_d| < 2^24, exact).
-// The planes are recombined by Horner's rule in signed 128-bit integers and
-// reduced once with Barrett; the rowsum correction is added mod q.
+// The planes are recombined into three 64-bit sums at weights 1, 2^32 and 2^64, which two
+// split products (FoldMod) bring mod q for primes just below a power of two, a 128-bit
+// Barrett step otherwise; the rowsum correction is added before or after.
 //
 // Mapping: block = 4 waves = 64 coefficient columns of one (poly, limb); a
 // wave owns 16 columns and keeps their X digits as MFMA B fragments in
@@ -82,27 +83,37 @@ __global__ void k_weight_frags(const double *W, const double *scales, i8x16 *fra
     }
 }
 
-// corr[l][i] = [128 R rowsum_i - 2^106]_q (the 2^106 offset keeps the
-// recombined plane sum non-negative); mu[l] = floor(2^109 / q_l).
-__global__ void k_weight_corr(const double *W, const double *scales, uint64_t *corr, uint64_t *mu,
-                              const DevMod *mods, size_t row_w, size_t col_w, size_t Ql, int DX) {
-    const size_t total = Ql * col_w;
-    for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-        const size_t l = t / col_w, i = t % col_w;
+// corr[l][i] = [128 R rowsum_i (- 2^106)]_q (the 2^106 offset keeps the Barrett form's
+// recombined plane sum non-negative; the split form takes signed sums); one block per column
+// i: its 64 lanes sum the column's weights, then take the limbs. mu[l] = floor(2^109 / q_l);
+// fc[l] = the split forms of 2^32 and 2^64 mod q_l (primes that have one).
+__global__ __launch_bounds__(64) void k_weight_corr(const double *W, const double *scales, uint64_t *corr, uint64_t *mu,
+                                                    u32x4 *fc, const DevMod *mods, const FoldMod *fold, size_t row_w,
+                                                    size_t col_w, size_t Ql, int DX, int offset) {
+    const size_t i = blockIdx.x;
+    int64_t s = 0;
+    for (size_t j = threadIdx.x; j < row_w; j += 64) s += weight_int(W, scales, col_w, j, i);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
+    for (size_t l = threadIdx.x; l < Ql; l += 64) {
         const DevMod m = mods[l];
-        int64_t s = 0;
-        for (size_t j = 0; j < row_w; j++) s += weight_int(W, scales, col_w, j, i);
         uint64_t rs = reduce64((uint64_t)(s < 0 ? -s : s), m);
         if (s < 0 && rs) rs = m.q - rs;
         uint64_t R = 0;
         for (int a = 0; a < DX; a++) R = add_mod(mul_mod(R, 256, m), 1, m.q);
         const uint64_t c = mul_mod(128 % m.q, R, m);
-        uint64_t p106 = 1;
-        for (int e = 0; e < 106; e++) p106 = add_mod(p106, p106, m.q);
-        corr[t] = sub_mod(mul_mod(c, rs, m), p106, m.q);
+        const uint64_t p32 = reduce64(uint64_t(1) << 32, m), p64 = mul_mod(p32, p32, m);
+        uint64_t v = mul_mod(c, rs, m);
+        if (offset) v = sub_mod(v, mul_mod(p64, reduce64(uint64_t(1) << 42, m), m), m.q);
+        corr[l * col_w + i] = v;
         if (i == 0) {
             // floor(2^109 / q) from floor(2^128 / q): shift by 19 bits (fits 64 bits for q > 2^45)
             mu[l] = (m.mu_hi << 45) | (m.mu_lo >> 19);
+            const FoldMod f = fold[l];
+            if (f.pw) {
+                fc[2 * l] = fold_split(p32, shoup_companion(p32, m), m.q, f);
+                fc[2 * l + 1] = fold_split(p64, shoup_companion(p64, m), m.q, f);
+            }
         }
     }
 }
@@ -123,18 +134,23 @@ __device__ __forceinline__ void transpose4(uint32_t w0, uint32_t w1, uint32_t w2
     o[3] = bperm(t3, t1, 0x07060302u);
 }
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 // Registers: the X digit fragments (DX KS 4 VGPRs) and the 11 planes dominate.
 // Up to DX KS = 21 (e.g. 7 digits x 192 rows) the kernel is held to 3 waves per
 // SIMD (156 registers at 7 x 3, no spill), which measured faster than
 // prefetching the next phase's weight fragments at 2 waves per SIMD; larger
 // shapes get 2 waves per SIMD so that they do not spill.
-template <int DX, int DW, int KS, int RB>
+// The recombination is about a third of the vector work: with FOLD (every limb's prime has a
+// split form) an output word takes 33 issue slots instead of 90. 192 x 64
+// at 24 limbs of N = 2^16 1886 -> 1817 us (waits for its loads dominate there: matrix cores
+// busy 35%, vector issue 34%), 301 x 37 at 11 limbs of 2^15 976 -> 799 us with the smaller
+// phases of rb_for.
+template <int DX, int DW, int KS, int RB, bool FOLD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DX * KS <= 21 ? 3 : 2))) void k_contract_int8(const uint64_t *const *__restrict__ X,
                                                        const i8x16 *__restrict__ frag,
                                                        const uint64_t *__restrict__ corr,
                                                        const uint64_t *__restrict__ mu_arr,
+                                                       const u32x4 *__restrict__ fc,
+                                                       const FoldMod *__restrict__ fold,
                                                        uint64_t *__restrict__ acc_out,
                                                        const DevMod *__restrict__ mods, int row_w, int col_w,
                                                        int MB, size_t Ql, size_t N, int accumulate, int radix,
@@ -156,6 +172,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DX * KS <= 
     const size_t col = tile * 64 + 16 * wave + (lane & 15);
     const size_t off = lp * N + col;
     const uint64_t q = mods[l].q, mu = mu_arr[l];
+    FoldMod f{};
+    u32x4 c32{}, c64{};
+    if (FOLD) {
+        f = fold[l];
+        c32 = fc[2 * l];
+        c64 = fc[2 * l + 1];
+    }
     // row pointers staged in LDS once per block; rows k >= row_w point at row 0
     // so that every load is unconditional (their words are zeroed below)
     __shared__ const uint64_t *xl[KS * 64];
@@ -241,6 +264,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DX * KS <= 
                     const int64_t t = (int64_t)C[d][r] * (int64_t)pw[d & 3];
                     if (d < 4) g0 += t; else if (d < 8) g1 += t; else g2 += t;
                 }
+                if (FOLD) {
+                    // |g0| < 2^56 and two split products: signed, far below 2^63
+                    if (row < col_w) {
+                        uint64_t *dst = &acc_out[(size_t)row * 2 * Ql * N + off];
+                        uint64_t v = (uint64_t)g0 + fold_mul((uint64_t)g1, c32, f) + fold_mul((uint64_t)g2, c64, f) +
+                                     cl[row - 16 * RB * ph];
+                        // a later row chunk adds to the sum of the earlier ones
+                        if (accumulate) v += __builtin_nontemporal_load(dst);
+                        // streamed once by the rescale that follows: keep it out of the caches
+                        __builtin_nontemporal_store(fold_canon<false>(v, q, f), dst);
+                    }
+                    continue;
+                }
                 // T = S + 2^106 (0 < T < 2^107)
                 const uint64_t a_lo = (uint64_t)g1 << 32;
                 const uint64_t lo = (uint64_t)g0 + a_lo;
@@ -265,27 +301,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DX * KS <= 
     }
 }
 
-typedef void (*ContractFn)(const uint64_t *const *, const i8x16 *, const uint64_t *, const uint64_t *, uint64_t *,
-                           const DevMod *, int, int, int, size_t, size_t, int, int, int, int);
+typedef void (*ContractFn)(const uint64_t *const *, const i8x16 *, const uint64_t *, const uint64_t *, const u32x4 *,
+                           const FoldMod *, uint64_t *, const DevMod *, int, int, int, size_t, size_t, int, int, int, int);
 
-constexpr int rb_for(int KS) { return KS == 1 ? 4 : KS == 2 ? 4 : KS == 3 ? 3 : 2; }
+// Row blocks staged per phase: 3 blocks of 256 threads share a CU's LDS (6 weight digits of
+// 192 rows take 18 KB a row block, so two of them there).
+constexpr int rb_for(int KS, int DW) { return KS == 1 ? 4 : KS == 2 ? 4 : KS == 3 ? (DW > 5 ? 2 : 3) : 2; }
 
-ContractFn pick(int DX, int DW, int KS) {
-#define SHM_PICK(dx, dw)                                                           \
-    if (DX == dx && DW == dw) {                                                    \
-        if (KS == 1) return k_contract_int8<dx, dw, 1, rb_for(1)>;                 \
-        if (KS == 2) return k_contract_int8<dx, dw, 2, rb_for(2)>;                 \
-        if (KS == 3) return k_contract_int8<dx, dw, 3, rb_for(3)>;                 \
-        if (KS == 4) return k_contract_int8<dx, dw, 4, rb_for(4)>;                 \
-    }
+// The split form covers primes of up to 56 bits (at most 7 digits).
+template <int DX, int DW, bool FOLD>
+ContractFn pick_ks(int KS) {
+    if (KS == 1) return k_contract_int8<DX, DW, 1, rb_for(1, DW), FOLD>;
+    if (KS == 2) return k_contract_int8<DX, DW, 2, rb_for(2, DW), FOLD>;
+    if (KS == 3) return k_contract_int8<DX, DW, 3, rb_for(3, DW), FOLD>;
+    return k_contract_int8<DX, DW, 4, rb_for(4, DW), FOLD>;
+}
+
+ContractFn pick(int DX, int DW, int KS, bool fold) {
+    if (KS < 1 || KS > 4) return nullptr;
+#define SHM_PICK(dx, dw)                                   \
+    if (DX == dx && DW == dw) return fold ? pick_ks<dx, dw, true>(KS) : pick_ks<dx, dw, false>(KS);
     SHM_PICK(6, 4)
     SHM_PICK(6, 5)
     SHM_PICK(6, 6)
     SHM_PICK(7, 4)
     SHM_PICK(7, 5)
     SHM_PICK(7, 6)
-    SHM_PICK(8, 4)
 #undef SHM_PICK
+    if (DX == 8 && DW == 4) return pick_ks<8, 4, false>(KS);
     return nullptr;
 }
 
@@ -312,9 +355,16 @@ bool int8_supported(const Context &c, size_t Ql, const double *W, const double *
     // and mu fits 64 bits for q > 2^45; q < 2^62 keeps the byte split within 8 digits.
     if (qmin < 46 || qbits > 61) return false;
     const int DX = (qbits + 7) / 8;
+    // the largest |round(w scale)|: rounding is monotone, so it is the rounded largest product
     double mx = 0;
-    for (size_t j = 0; j < row_w; j++)
-        for (size_t i = 0; i < col_w; i++) mx = std::max(mx, std::fabs(std::round(W[j * col_w + i] * scales[j])));
+    for (size_t j = 0; j < row_w; j++) {
+        double m = 0;
+        for (size_t i = 0; i < col_w; i++) {
+            const double v = std::fabs(W[j * col_w + i] * scales[j]);
+            m = v > m ? v : m;
+        }
+        mx = std::max(mx, std::round(m));
+    }
     int DW = 1;
     // balanced digits: D digits cover |w| <= 127 * (256^D - 1) / 255
     while (DW < 9 && mx > 127.0 * (std::pow(256.0, DW) - 1) / 255.0) DW++;
@@ -323,7 +373,7 @@ bool int8_supported(const Context &c, size_t Ql, const double *W, const double *
     // limb, |x'| < 2^(8 DX - 1)) must stay below 2^106 in magnitude
     const size_t nch = (row_w + kChunkRows - 1) / kChunkRows, kc_max = (row_w + nch - 1) / nch;
     if ((double)kc_max * std::ldexp(1.0, 8 * DX - 1) * mx >= std::ldexp(1.0, 106)) return false;
-    if (!pick(DX, DW, 1)) return false;
+    if (!pick(DX, DW, 1, false)) return false;
     *dx_out = DX;
     *dw_out = DW;
     return true;
@@ -344,7 +394,7 @@ void ctpt_matmul_int8(const Context &c, const std::vector<const Ciphertext *> &X
     if (hook && nch != 1) throw LogicError("limb windows need one row chunk");
     const int MB = (int)((col_w + 15) / 16);
     auto frag_count = [&](int KS) {
-        const int RB = rb_for(KS), NPH = (MB + RB - 1) / RB;
+        const int RB = rb_for(KS, DW), NPH = (MB + RB - 1) / RB;
         return (size_t)NPH * DW * RB * KS * 64;
     };
     Scratch dW(row_w * col_w * sizeof(double), s);
@@ -352,6 +402,9 @@ void ctpt_matmul_int8(const Context &c, const std::vector<const Ciphertext *> &X
     Scratch frag(frag_count((int)((kc_max + 63) / 64)) * sizeof(i8x16), s);
     Scratch corr(Ql * col_w * sizeof(uint64_t), s);
     Scratch mu(Ql * sizeof(uint64_t), s);
+    Scratch fc(2 * Ql * sizeof(u32x4), s);
+    bool fold = DX <= 7;
+    for (size_t l = 0; l < Ql; l++) fold = fold && c.fold_bound[l] != 0 && !c.fold_twice[l];
     Scratch xptr(row_w * sizeof(uint64_t *), s);
     std::vector<const uint64_t *> xp(row_w);
     for (size_t j = 0; j < row_w; j++) xp[j] = X[j]->data();
@@ -363,19 +416,19 @@ void ctpt_matmul_int8(const Context &c, const std::vector<const Ciphertext *> &X
     for (size_t ch = 0; ch < nch; ch++) {
         // chunk rows [k0, k0 + kc): W rows are contiguous, so the chunk is a sub-matrix
         const size_t kc = row_w / nch + (ch < row_w % nch ? 1 : 0);
-        const int KS = (int)((kc + 63) / 64), RB = rb_for(KS);
+        const int KS = (int)((kc + 63) / 64), RB = rb_for(KS, DW);
         const size_t nfrag = frag_count(KS);
         const double *Wc = dW.as<double>() + k0 * col_w;
         const double *sc = dscale.as<double>() + k0;
         k_weight_frags<<<grid_for(nfrag), kBlock, 0, s>>>(Wc, sc, frag.as<i8x16>(), kc, col_w, DW, MB, KS, RB);
-        k_weight_corr<<<grid_for(Ql * col_w), kBlock, 0, s>>>(Wc, sc, corr.as<uint64_t>(), mu.as<uint64_t>(),
-                                                              c.mods(), kc, col_w, Ql, DX);
+        k_weight_corr<<<(unsigned)col_w, 64, 0, s>>>(Wc, sc, corr.as<uint64_t>(), mu.as<uint64_t>(), fc.as<u32x4>(),
+                                                     c.mods(), c.d_fold.as<FoldMod>(), kc, col_w, Ql, DX, fold ? 0 : 1);
         SHM_HIP(hipGetLastError());
-        ContractFn fn = pick(DX, DW, KS);
+        ContractFn fn = pick(DX, DW, KS, fold);
         auto launch = [&](size_t l_lo, size_t l_n) {
             hipLaunchKernelGGL(fn, dim3((unsigned)(2 * l_n * tiles)), dim3(256), 0, s,
                                xptr.as<const uint64_t *>() + k0, frag.as<i8x16>(), corr.as<uint64_t>(),
-                               mu.as<uint64_t>(), acc, c.mods(), (int)kc, (int)col_w, MB, Ql, N, ch > 0 ? 1 : 0, 256,
+                               mu.as<uint64_t>(), fc.as<u32x4>(), c.d_fold.as<FoldMod>(), acc, c.mods(), (int)kc, (int)col_w, MB, Ql, N, ch > 0 ? 1 : 0, 256,
                                (int)l_lo, (int)l_n);
             SHM_HIP(hipGetLastError());
         };
