@@ -377,6 +377,7 @@ struct MacJob {
     uint64_t *out;
     size_t out_stride;
     bool accumulate, add_on;
+    const uint32_t *own_perm;  // own limbs are read through this NTT-domain permutation, unless null
     PolyPack add;
     const uint64_t *pmod, *pmod_s;
 };
@@ -389,8 +390,10 @@ void ntt_encoded_columns(const Context &c, const double2 *fft, uint64_t *out, si
                          hipStream_t s);
 // Inverse NTT whose last pass multiplies limb k by scale[k - scale_lo] (value, Shoup
 // companion: N^-1 times a conversion's premultiplication) instead of N^-1.
+// With perm, the inputs are read through that NTT-domain permutation.
 void ntt_inverse_gather_scaled(const Context &c, const PolyPack &in, uint64_t *out, size_t n_polys, size_t n_limbs,
-                               const uint64_t *scale, const uint64_t *scale_s, hipStream_t s);
+                               const uint64_t *scale, const uint64_t *scale_s, hipStream_t s,
+                               const uint32_t *perm = nullptr);
 void ntt_inverse_qlp_scaled(const Context &c, uint64_t *data, size_t Ql, size_t lo, size_t hi, size_t n_polys,
                             size_t poly_stride, const uint64_t *scale, const uint64_t *scale_s, hipStream_t s);
 
@@ -425,6 +428,9 @@ void launch_square(const Context &c, const uint64_t *a, uint64_t *out3, size_t Q
                    size_t a_limbs = 0);
 // (d0, d1, d2) = 2 (a (x) b) - cval (t0, t1, 0), the Chebyshev step T_k = 2 T_a T_b - T_(a-b)
 // before relinearisation (b == a squares; t may be null); operands through their first Ql limbs
+// out3 = sum_i a_i (x) b_i over size-2 operands (sums of up to 15 products per launch)
+void launch_tensor_sum(const Context &c, const std::vector<const uint64_t *> &a, const std::vector<const uint64_t *> &b,
+                       uint64_t *out3, size_t Ql, size_t a_limbs, size_t b_limbs, hipStream_t s);
 void launch_tensor_cheb(const Context &c, const uint64_t *a, const uint64_t *b, const uint64_t *t, uint64_t cval,
                         uint64_t *out3, size_t Ql, hipStream_t s, size_t a_limbs, size_t b_limbs, size_t t_limbs);
 void launch_rescale(const Context &c, const uint64_t *in, uint64_t *out, size_t Ql, size_t npolys, hipStream_t s,
@@ -525,6 +531,12 @@ void keyswitch_rescale_batch(const Context &c, const PolyPack &c2, const PolyPac
 // Key switch of m polynomials c2.p[i] with one key; the switched pair of member
 // i goes to (ct01.p[2i], ct01.p[2i + 1]), accumulated where acc_mask has the
 // polynomial's bit. One launch per stage for the whole group.
+// Key switch of sigma(a_k) for m size-2 ciphertexts (a_k, b_k given unpermuted, sigma the
+// NTT-domain permutation `perm`) into out.p[2k], out.p[2k + 1] = (sigma(b_k) + ks_0, ks_1), no
+// permuted copy written; outputs must not overlap a or b. Returns false, with nothing done,
+// where the fused key switch does not apply.
+bool keyswitch_galois(const Context &c, const PolyPack &a, const PolyPack &b, size_t m, const uint64_t *key, size_t Ql,
+                      const PolyPack &out, const uint32_t *perm, hipStream_t s);
 void keyswitch_batch(const Context &c, const PolyPack &c2, size_t m, const uint64_t *key, size_t Ql,
                      const PolyPack &ct01, uint64_t acc_mask, hipStream_t s, bool rounded = false);
 

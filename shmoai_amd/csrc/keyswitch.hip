@@ -638,14 +638,15 @@ constexpr size_t kFusedRows = 2048;
 // transforms leave y_i = [x_i (D_g/q_i)^-1]_{q_i}, convert_cols takes every digit to its other
 // limbs' column stages, and the row stages finish them (copying the digits' own limbs, c2's
 // NTT-form words, where the caller reads them from d).
-// Without `rows`, the row stages are left to the caller (rows_mac).
+// Without `rows`, the row stages are left to the caller (rows_mac). With perm (and without
+// own), c2 is read through that NTT-domain permutation.
 static void modup_fused(const Context &c, const PolyPack &c2, size_t m, size_t Ql, uint64_t *d, bool own,
-                        hipStream_t s, bool rounded, bool rows = true) {
+                        hipStream_t s, bool rounded, bool rows = true, const uint32_t *perm = nullptr) {
     const size_t N = c.N, alpha = c.nP, QlP = Ql + alpha;
     const LevelConsts &L = c.level(Ql);
     Scratch tcoef(m * Ql * N * sizeof(uint64_t), s);
     ntt_inverse_gather_scaled(c, c2, tcoef.as<uint64_t>(), m, Ql, L.hat_ninv.as<uint64_t>(),
-                              L.hat_ninv_s.as<uint64_t>(), s);
+                              L.hat_ninv_s.as<uint64_t>(), s, perm);
     ConvertJob job{};
     job.src = tcoef.as<uint64_t>();
     job.src_stride = Ql * N;
@@ -664,18 +665,24 @@ static void modup_fused(const Context &c, const PolyPack &c2, size_t m, size_t Q
     if (rows) ntt_rows_digits(c, d, Ql, L.beta, m, c2, own, s);
 }
 
+static bool fused_rows(const Context &c, size_t m, size_t Ql) {
+    const size_t beta = c.level(Ql).beta;
+    return convert_covers(c, c.nP) && rows_mac_covers(c, Ql, true, beta) && beta <= c.dnum &&
+           m * (Ql + c.nP) * (c.N / 512) >= kFusedRows;
+}
+
 // ModUp of m members and their inner products with one key, cx[m][2][QlP][N], the digits' row
 // stages fused with the products (and P d01 added on the data limbs). Returns false, with
 // nothing done, where that does not apply: primes outside the split sums, or too few rows to
 // fill the GPU with one wave per row and member.
 static bool modup_inner_fused(const Context &c, const PolyPack &c2, size_t m, size_t Ql, const uint64_t *key,
-                              uint64_t *d, uint64_t *cx, hipStream_t s, bool rounded, const PolyPack *add) {
+                              uint64_t *d, uint64_t *cx, hipStream_t s, bool rounded, const PolyPack *add,
+                              const uint32_t *perm = nullptr) {
     const size_t N = c.N, alpha = c.nP, QlP = Ql + alpha, beta = c.level(Ql).beta;
-    if (!convert_covers(c, alpha) || !rows_mac_covers(c, Ql, true, beta) || beta > c.dnum) return false;
-    if (m * QlP * (N / 512) < kFusedRows) return false;
+    if (!fused_rows(c, m, Ql)) return false;
     bump(g_cnt_modup, Ql, m);
     bump(g_cnt_inner, Ql, 2 * m);
-    modup_fused(c, c2, m, Ql, d, false, s, rounded, false);
+    modup_fused(c, c2, m, Ql, d, false, s, rounded, false, perm);
     MacJob job{};
     job.data = d;
     job.stride = QlP * N;
@@ -689,6 +696,7 @@ static bool modup_inner_fused(const Context &c, const PolyPack &c2, size_t m, si
     job.key = key;
     job.op_stride = c.nQP() * N;
     job.op = c2;
+    job.own_perm = perm;
     job.out = cx;
     job.out_stride = QlP * N;
     if (add) {
@@ -924,6 +932,24 @@ void ks_inner_batch(const Context &c, const uint64_t *d, size_t m, size_t Ql, co
         const int lg = tuned_slots(tk, max_lg, g0 == 0, s, launch, &ran);
         if (!ran) launch(lg);
     }
+}
+
+bool keyswitch_galois(const Context &c, const PolyPack &a, const PolyPack &b, size_t m, const uint64_t *key, size_t Ql,
+                      const PolyPack &out, const uint32_t *perm, hipStream_t s) {
+    const size_t N = c.N, QlP = Ql + c.nP, beta = c.level(Ql).beta;
+    if (m == 0 || 2 * m > (size_t)kPolyPack) throw InvalidArgument("keyswitch_galois: 1..32 members");
+    if (!fused_rows(c, m, Ql)) return false;
+    Scratch d(m * beta * QlP * N * sizeof(uint64_t), s);
+    Scratch cx(2 * m * QlP * N * sizeof(uint64_t), s);
+    if (!modup_inner_fused(c, a, m, Ql, key, d.as<uint64_t>(), cx.as<uint64_t>(), s, false, nullptr, perm)) return false;
+    PolyPack src{};
+    uint64_t mask = 0;
+    for (size_t k = 0; k < m; k++) {
+        src.p[2 * k] = b.p[k];
+        mask |= uint64_t(1) << (2 * k);
+    }
+    ks_moddown_pack(c, cx.as<uint64_t>(), 2 * m, Ql, out, mask, s, false, &src, perm);
+    return true;
 }
 
 void keyswitch_batch(const Context &c, const PolyPack &c2, size_t m, const uint64_t *key, size_t Ql,

@@ -260,6 +260,7 @@ struct NttIO {
     const uint64_t *scale_s;  // (value, Shoup companion) instead of N^-1, unless null
     uint32_t scale_lo;
     uint32_t digits, alpha, copy_own;  // IO_DIGITS
+    const uint32_t *perm;     // IO_GATHER: inputs read through this NTT-domain permutation, unless null
 };
 
 // Column pass, log N1 = RA + RB stages. A block takes C columns (consecutive words of a
@@ -718,6 +719,16 @@ __global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data,
     };
     auto load = [&](uint64_t (&x)[8], uint32_t p) {
         if (IO == IO_DIGITS && !io.copy_own && own(p)) return;
+        if (IO == IO_GATHER && io.perm) {
+            const auto src = global_ptr(io.acc_p.p[p] + (size_t)limb * N);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const auto at = global_ptr(io.perm + row0 + 2 * lane + 128 * j);
+                x[2 * j] = src[at[0]];
+                x[2 * j + 1] = src[at[1]];
+            }
+            return;
+        }
         const uint64_t *ld = src_of(p);
         if constexpr (FWD) {
 #pragma unroll
@@ -823,9 +834,18 @@ __global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, i
                 a[o][j] = *global_ptr(reinterpret_cast<const u64x2 *>(op + o * job.op_stride + pair_of(j)));
         u64x2 y[4];
         if (own(t)) {
-            const uint64_t *p = job.op.p[e] + at;
+            if (job.own_perm) {
+                const auto p = global_ptr(job.op.p[e] + (size_t)limb * N);
 #pragma unroll
-            for (int j = 0; j < 4; j++) y[j] = *global_ptr(reinterpret_cast<const u64x2 *>(p + pair_of(j)));
+                for (int j = 0; j < 4; j++) {
+                    const auto i = global_ptr(job.own_perm + row0 + pair_of(j));
+                    y[j] = u64x2{p[i[0]], p[i[1]]};
+                }
+            } else {
+                const uint64_t *p = job.op.p[e] + at;
+#pragma unroll
+                for (int j = 0; j < 4; j++) y[j] = *global_ptr(reinterpret_cast<const u64x2 *>(p + pair_of(j)));
+            }
         } else {
             wave_lds_order();
             row_forward(k, w, x, [&](int i) { return lt[i]; }, [&](int i) { return lt[8 + 8 * i + (lane >> 3)]; },
@@ -1318,12 +1338,13 @@ void ntt_rows_digits(const Context &c, uint64_t *d, size_t Ql, size_t beta, size
 }
 
 void ntt_inverse_gather_scaled(const Context &c, const PolyPack &in, uint64_t *out, size_t n_polys, size_t n_limbs,
-                               const uint64_t *scale, const uint64_t *scale_s, hipStream_t s) {
+                               const uint64_t *scale, const uint64_t *scale_s, hipStream_t s, const uint32_t *perm) {
     if (n_polys == 0) return;
     if (n_polys > (size_t)kPolyPack) throw InvalidArgument("inverse NTT: 1..64 polynomials per batch");
     LimbMap mp{(uint32_t)n_limbs, 0, 0xffffffffu, 0, 0xffffffffu, (uint32_t)c.nQ, 0, (uint64_t)n_limbs * c.N};
     NttIO io{};
     io.acc_p = in;
+    io.perm = perm;
     io.scale = scale;
     io.scale_s = scale_s;
     launch_ntt<false, IO_PLAIN, IO_GATHER>(c, out, mp, n_polys * n_limbs, s, io);

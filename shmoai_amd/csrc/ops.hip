@@ -91,6 +91,23 @@ void apply_galois(Context &c, Ciphertext &ct, uint32_t elt, const GaloisKeys &gk
         ct = std::move(o);
         return;
     }
+    {
+        // both parts are read through the permutation where the key switch runs fused
+        Ciphertext o;
+        o.ctx = &c;
+        o.resize(2, ct.chain, s, false);  // the fused ModDown writes every word
+        o.scale = ct.scale;
+        o.ntt = true;
+        PolyPack a{}, b{}, op{};
+        a.p[0] = ct.poly(1);
+        b.p[0] = ct.poly(0);
+        op.p[0] = o.poly(0);
+        op.p[1] = o.poly(1);
+        if (keyswitch_galois(c, a, b, 1, it->second->k.as<uint64_t>(), Ql, op, table, s)) {
+            ct = std::move(o);
+            return;
+        }
+    }
     Scratch t0(Ql * N * sizeof(uint64_t), s), t1(Ql * N * sizeof(uint64_t), s);
     launch_permute(c, ct.poly(0), t0.as<uint64_t>(), table, Ql, s);
     launch_permute(c, ct.poly(1), t1.as<uint64_t>(), table, Ql, s);
@@ -642,22 +659,28 @@ void rotate_many(Context &c, const std::vector<const Ciphertext *> &in, const st
     for (size_t k0 = 0; k0 < in.size(); k0 += 32) {
         const size_t m = std::min<size_t>(32, in.size() - k0);
         const size_t Ql = in[k0]->Ql();
-        PolyPack c2{}, ct01{};
+        PolyPack c2{}, ct01{}, a{}, b{};
         for (size_t k = 0; k < m; k++) {
             const Ciphertext &x = *in[k0 + k];
             Ciphertext &o = *out[k0 + k];
             if (x.size != 2 || x.Ql() != Ql) throw InvalidArgument("rotate_many: size-2 ciphertexts at one level");
             o.ctx = &c;
-            o.resize(2, x.chain, s, false);  // both polynomials are written by the permutation
+            o.resize(2, x.chain, s, false);  // both polynomials are written below
             o.scale = x.scale;
             o.ntt = true;
-            launch_permute(c, x.poly(0), o.poly(0), table, Ql, s);
-            launch_permute(c, x.poly(1), o.poly(1), table, Ql, s);
+            b.p[k] = const_cast<uint64_t *>(x.poly(0));  // read only
+            a.p[k] = const_cast<uint64_t *>(x.poly(1));
             // the permuted c1 is the key switch input; ModDown overwrites it with
             // the new c1 after the inner products have read it
             c2.p[k] = o.poly(1);
             ct01.p[2 * k] = o.poly(0);
             ct01.p[2 * k + 1] = o.poly(1);
+        }
+        // both parts are read through the permutation where the key switch runs fused
+        if (keyswitch_galois(c, a, b, m, it->second->k.as<uint64_t>(), Ql, ct01, table, s)) continue;
+        for (size_t k = 0; k < m; k++) {
+            launch_permute(c, b.p[k], ct01.p[2 * k], table, Ql, s);
+            launch_permute(c, a.p[k], ct01.p[2 * k + 1], table, Ql, s);
         }
         const uint64_t add_c0 = 0x5555555555555555ull & ((m == 32) ? ~uint64_t(0) : (uint64_t(1) << (2 * m)) - 1);
         keyswitch_batch(c, c2, m, it->second->k.as<uint64_t>(), Ql, ct01, add_c0, s, false);
@@ -732,10 +755,12 @@ void ctct_matmul_colpacking(Context &c, const std::vector<const Ciphertext *> &X
         for (size_t i = i0; i < i1; i++) {
             const size_t step = i * (size_t)num_batch;
             if (step != 0) rotate_many(c, W, rotp, (int)step, gk, s);  // every W[j] by the same step
+            std::vector<const uint64_t *> xa(colX), wb(colX);
             for (size_t j = 0; j < colX; j++) {
-                const Ciphertext *w = step != 0 ? &rot[j] : W[j];
-                launch_tensor(c, X[j]->data(), w->data(), out[i]->data(), Ql, s, X[j]->Ql(), w->Ql(), j > 0);
+                xa[j] = X[j]->data();
+                wb[j] = step != 0 ? rot[j].data() : W[j]->data();
             }
+            launch_tensor_sum(c, xa, wb, out[i]->data(), Ql, Ql, Ql, s);
         }
         std::vector<Ciphertext *> chunk(out.begin() + i0, out.begin() + i1);
         relin_many(c, chunk, rk, Ql, s);
