@@ -654,7 +654,8 @@ __device__ __forceinline__ void row_pass(const K &k, uint64_t *lds, uint64_t *ba
         if (io.packed || io.out_packed) {
             out = io.out_p.p[poly] + (size_t)limb * N + row0;
         } else {
-            uint64_t *ob = io.outs ? io.outs[poly / io.ppo] : io.out_single;
+            uint64_t *ob = io.out_single;
+            if (io.outs) ob = table_ptr(io.outs)[poly / io.ppo];
             out = ob + ((size_t)(poly % io.ppo) * (io.out_limbs ? io.out_limbs : n_active) + limb) * N + row0;
         }
     }
@@ -668,7 +669,23 @@ __device__ __forceinline__ void row_pass(const K &k, uint64_t *lds, uint64_t *ba
                 accv[j] = __builtin_nontemporal_load(global_ptr(reinterpret_cast<const u64x2 *>(accp + pair_of(j))));
         }
     });
+    // words that are added on: all requested at once, since a load's wait behind a store of this
+    // loop would wait for the store as well
     const bool addto = IO == IO_RESCALE && io.out_packed && poly < 64 && ((io.acc_mask >> poly) & 1);
+    u64x2 ov[IO == IO_RESCALE ? 4 : 1];
+    if (addto) {
+        if (io.add_perm) {
+            const auto src = global_ptr(io.add_src.p[poly] + (size_t)limb * N);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const auto at = global_ptr(io.add_perm + row0 + pair_of(j));
+                ov[j] = u64x2{src[at[0]], src[at[1]]};
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) ov[j] = *global_ptr(reinterpret_cast<const u64x2 *>(out + pair_of(j)));
+        }
+    }
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int i = pair_of(j);
@@ -678,16 +695,8 @@ __device__ __forceinline__ void row_pass(const K &k, uint64_t *lds, uint64_t *ba
             y.x = kh.sub_mul(accv[j].x, y.x, qi);
             y.y = kh.sub_mul(accv[j].y, y.y, qi);
             if (addto) {
-                u64x2 o;
-                if (io.add_perm) {
-                    const auto src = global_ptr(io.add_src.p[poly] + (size_t)limb * N);
-                    const auto at = global_ptr(io.add_perm + row0 + i);
-                    o = u64x2{src[at[0]], src[at[1]]};
-                } else {
-                    o = *global_ptr(reinterpret_cast<const u64x2 *>(out + i));
-                }
-                y.x = add_mod(y.x, o.x, k.q);
-                y.y = add_mod(y.y, o.y, k.q);
+                y.x = add_mod(y.x, ov[j].x, k.q);
+                y.y = add_mod(y.y, ov[j].y, k.q);
             }
         } else {
             y.x = k.canon(y.x);
@@ -766,7 +775,13 @@ __global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data,
     for (int e = 0; e < 7; e++) w3[e] = tw[64 + 64 * e + lane];
     wave_lds_order();
     auto loop = [&](const auto &k) {
-        const auto qi = IO == IO_RESCALE ? k.constant(io.qinv[prime], io.qinv_s[prime]) : k.constant(0, 0);
+        const auto qi = IO == IO_RESCALE ? k.constant(table_ptr(io.qinv)[prime], table_ptr(io.qinv_s)[prime]) : k.constant(0, 0);
+        // the first words and the twiddles are waited for here: in the loop, that wait would take
+        // the next polynomial's words along
+#pragma unroll
+        for (int l = 0; l < 8; l++) asm volatile("" : "+v"(x[l]));
+#pragma unroll
+        for (int e = 0; e < 7; e++) asm volatile("" : "+v"(w3[e]));
         for (uint32_t p = p0; p < p1; p++) {
             if (p + 1 < p1) load(nx, p + 1);
             uint64_t *base = data + p * mp.poly_stride + (size_t)limb * N + row0;
@@ -815,12 +830,6 @@ __global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, i
     const uint32_t prime = limb < job.Ql ? limb : nQ + (limb - job.Ql);
     const size_t at = (size_t)limb * N + row0;
     const FoldK<false> k(tb, prime);
-    {
-        const u32x4 *tw = tb.row + (size_t)prime * N + row0;
-#pragma unroll
-        for (int j = 0; j < 8; j++) ltw[wave][lane + 64 * j] = tw[lane + 64 * j];
-    }
-    const u32x4 *lt = ltw[wave];
     const RowWords w(lds[wave], lane);
     auto pair_of = [&](int j) { return 2 * lane + 128 * j; };
     auto own = [&](uint32_t t) { return KEY && limb < job.Ql && limb / job.alpha == t; };
@@ -837,6 +846,19 @@ __global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, i
 #pragma unroll
         for (int j = 0; j < 8; j++) acc[o][j] = Acc52{0, 0, 0};
     load(x, 0);
+    const u32x4 *tw = tb.row + (size_t)prime * N + row0;
+#pragma unroll
+    for (int j = 0; j < 8; j++) ltw[wave][lane + 64 * j] = tw[lane + 64 * j];
+    const u32x4 *lt = ltw[wave];
+    u32x4 w1[7];
+#pragma unroll
+    for (int i = 0; i < 7; i++) {
+        w1[i] = table_ptr(tw)[i];
+        asm volatile("" : "+s"(w1[i]));  // loaded once
+    }
+    // the first words are waited for here: in the loop, that wait would take the next term's along
+#pragma unroll
+    for (int l = 0; l < 8; l++) asm volatile("" : "+v"(x[l]));
     for (uint32_t t = 0; t < job.terms; t++) {
         if (t + 1 < job.terms) load(nx, t + 1);
         const uint64_t *op = KEY ? job.key + (size_t)t * 2 * job.op_stride + (size_t)prime * N + row0 : job.op.p[t] + at;
@@ -862,8 +884,14 @@ __global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, i
             }
         } else {
             wave_lds_order();
-            row_forward(k, w, x, [&](int i) { return lt[i]; }, [&](int i) { return lt[8 + 8 * i + (lane >> 3)]; },
-                        [&](int i) { return lt[64 + 64 * i + lane]; }, [] {});
+            u32x4 w2[7], w3[7];
+#pragma unroll
+            for (int i = 0; i < 7; i++) w2[i] = lt[8 + 8 * i + (lane >> 3)];
+            row_forward(k, w, x, [&](int i) { return w1[i]; }, [&](int i) { return w2[i]; },
+                        [&](int i) { return w3[i]; }, [&] {
+#pragma unroll
+                            for (int i = 0; i < 7; i++) w3[i] = lt[64 + 64 * i + lane];
+                        });
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int i = row_slot(pair_of(j));
