@@ -807,18 +807,51 @@ __global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data,
     }
 }
 
+// Sums of products y a of words y < 2^(b + 1) and canonical a = ah 2^32 + al: y and
+// y 2^32 mod p (2^33 delta + 2^(b + 1) < 2^63, folded to 2^53) are split at 26 bits, so a term adds two
+// products to each of two sums (H 2^26 + L) and `a` needs no splitting. For a < 2^52 a term adds
+// less than 2^59 + 2^47 to H and 2^58 + 2^46 to L: 16 terms fit. Two sums take 4 registers a
+// word where 26-bit halves of both factors take 6, which is the third wave per SIMD of
+// k_rows_mac: 560 -> 516 us for 128 masked plaintexts, 754 -> 683 us per relinearisation launch
+// of a chunk of 8 shared-a refreshes.
+struct RowAcc {
+    uint64_t H, L;
+};
+struct RowWord {
+    uint32_t h0, l0, h1, l1;
+};
+__device__ __forceinline__ RowWord row_word(uint64_t y, const FoldMod &f) {
+    const uint64_t up = (uint64_t)((uint32_t)y & (2 * f.mask + 1)) << 32;
+    const uint32_t hi = __builtin_amdgcn_alignbit((uint32_t)(y >> 32), (uint32_t)y, f.sh + 1);  // y >> (b - 31)
+    uint64_t z = (uint64_t)hi * (2 * (uint32_t)f.d) + up;
+    const uint32_t zh = (uint32_t)(z >> 32);
+    z = (uint64_t)(zh >> f.sh) * (uint32_t)f.d + (((uint64_t)(zh & f.mask) << 32) | (uint32_t)z);
+    const Split26 s = split26(y), t = split26(z);
+    return RowWord{s.hi, s.lo, t.hi, t.lo};
+}
+__device__ __forceinline__ void row_mac(RowAcc &a, const RowWord &y, uint64_t x) {
+    const uint32_t xl = (uint32_t)x, xh = (uint32_t)(x >> 32);
+    a.H += (uint64_t)xl * y.h0;
+    a.L += (uint64_t)xl * y.l0;
+    a.H += (uint64_t)xh * y.h1;
+    a.L += (uint64_t)xh * y.l1;
+}
+__device__ __forceinline__ uint64_t row_sum(const RowAcc &a, const DevMod &m) { return reduce52(Acc52{a.L, a.H, 0}, m); }
+
 // Row stages fused with the products that consume them (MacJob): a wave takes one row of one
 // limb for one group, runs the row stages of each term's polynomial and multiplies its words
-// by two operand rows into split sums (Acc52), so transformed words never reach memory. The
+// by two operand rows into split sums (RowAcc), so transformed words never reach memory. The
 // next term's words and this term's operand rows are requested before the stages. Per wave 8
-// KB of twiddles and 4.6 KB of exchange in LDS; 96 registers hold the sums, 2 waves per SIMD.
+// KB of twiddles and 4.6 KB of exchange in LDS; 64 registers hold the sums, 3 waves per SIMD.
 // Groups of one row are neighbours in launch order, so operand rows that groups share (a
-// key's, or the inputs' of a product) come from L2 after the first. Bound by VALU issue (about
-// 480 slots per term and word group). Against row pass and product kernels apart at N = 2^16:
-// one top-level rotation's 66 + 96 us in 102; relinearisations of 16 members, 18 per shared-a
-// chunk, 20.7 ms in 15.2; 128 masked plaintexts of 24 limbs 500 + 517 us in 660.
+// key's, or the inputs' of a product) come from L2 after the first. Bound by VALU issue where
+// groups share operands (540 vector instructions per term and row of 512 words; 128 masked
+// plaintexts of 24 limbs in 516 us, about 400 of them issue), by its key's and digits' bytes
+// for a single rotation. Against row pass and product kernels apart at N = 2^16: one top-level
+// rotation's 66 + 96 us in 95; relinearisations of 16 members, 18 per shared-a chunk, 20.7 ms
+// in 12.3; the masked plaintexts 500 + 517 us in 516.
 template <bool KEY>
-__global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, int logN, uint32_t nQ, uint32_t per_xcd) {
+__global__ __launch_bounds__(256, 3) void k_rows_mac(MacJob job, NttTables tb, int logN, uint32_t nQ, uint32_t per_xcd) {
     __shared__ uint64_t lds[4][kRowLds];
     __shared__ __align__(16) u32x4 ltw[4][kRow];
     const size_t N = size_t(1) << logN;
@@ -840,11 +873,11 @@ __global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, i
         for (int l = 0; l < 8; l++) x[l] = __builtin_nontemporal_load(global_ptr(p + lane + 64 * l));
     };
     uint64_t x[8], nx[8];
-    Acc52 acc[2][8];
+    RowAcc acc[2][8];
 #pragma unroll
     for (int o = 0; o < 2; o++)
 #pragma unroll
-        for (int j = 0; j < 8; j++) acc[o][j] = Acc52{0, 0, 0};
+        for (int j = 0; j < 8; j++) acc[o][j] = RowAcc{0, 0};
     load(x, 0);
     const u32x4 *tw = tb.row + (size_t)prime * N + row0;
 #pragma unroll
@@ -884,14 +917,8 @@ __global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, i
             }
         } else {
             wave_lds_order();
-            u32x4 w2[7], w3[7];
-#pragma unroll
-            for (int i = 0; i < 7; i++) w2[i] = lt[8 + 8 * i + (lane >> 3)];
-            row_forward(k, w, x, [&](int i) { return w1[i]; }, [&](int i) { return w2[i]; },
-                        [&](int i) { return w3[i]; }, [&] {
-#pragma unroll
-                            for (int i = 0; i < 7; i++) w3[i] = lt[64 + 64 * i + lane];
-                        });
+            row_forward(k, w, x, [&](int i) { return w1[i]; }, [&](int i) { return lt[8 + 8 * i + (lane >> 3)]; },
+                        [&](int i) { return lt[64 + 64 * i + lane]; }, [] {});
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int i = row_slot(pair_of(j));
@@ -900,11 +927,12 @@ __global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, i
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const Split26 s0 = split26(y[j].x), s1 = split26(y[j].y);
+            const FoldK<false> kh = k.here();
+            const RowWord s0 = row_word(y[j].x, kh.f), s1 = row_word(y[j].y, kh.f);
 #pragma unroll
             for (int o = 0; o < 2; o++) {
-                mac52(acc[o][2 * j], s0, a[o][j].x);
-                mac52(acc[o][2 * j + 1], s1, a[o][j].y);
+                row_mac(acc[o][2 * j], s0, a[o][j].x);
+                row_mac(acc[o][2 * j + 1], s1, a[o][j].y);
             }
         }
 #pragma unroll
@@ -920,7 +948,7 @@ __global__ __launch_bounds__(256, 2) void k_rows_mac(MacJob job, NttTables tb, i
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const auto at2 = global_ptr(reinterpret_cast<u64x2 *>(out + pair_of(j)));
-            u64x2 v = {reduce52(acc[o][2 * j], m), reduce52(acc[o][2 * j + 1], m)};
+            u64x2 v = {row_sum(acc[o][2 * j], m), row_sum(acc[o][2 * j + 1], m)};
             if (job.accumulate) {
                 const u64x2 c = *at2;
                 v = u64x2{add_mod(v.x, c.x, m.q), add_mod(v.y, c.y, m.q)};

@@ -22,6 +22,8 @@ CASES = [
     # 16 rows of limbs and more: row stages fused with the products (7 digits; a last digit of one)
     (16, [51] + [46] * 13 + [51, 51], 2, 14),
     (16, [51] + [46] * 15 + [51] * 4, 4, 13),
+    # as many digits as the split sums of the fused products hold
+    (16, [51] * 17, 1, 16),
 ]
 
 
