@@ -34,6 +34,7 @@
 #include <algorithm>
 
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "engine.h"
@@ -478,6 +479,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_convert_cols(ConvertJob job, Nt
     };
     uint32_t k = next(blockIdx.z * run);
     u32x4 tw_next = tw_of(k);
+    // waited for here: in the loop, that wait would cover the previous limb's stores as well
+    asm volatile("" : "+v"(tw_next));
     int buf = 0;
     while (k < k_end) {
         const uint32_t prime = prime_of(k), k_next = next(k + 1);
@@ -512,23 +515,30 @@ __global__ __launch_bounds__(kThreads, 2) void k_convert_cols(ConvertJob job, Nt
                     }
                 }
             } else if constexpr (FAST) {
-                const auto cv = table_ptr(job.conv + ((size_t)g * job.n_out + k) * (job.alpha + 1));
+                // A is the table's number of terms. The branch on the rounding stands outside of
+                // the words: inside, every word's sums were a block of their own, a serial chain.
+                const auto cv = table_ptr(job.conv + ((size_t)g * job.n_out + k) * (A + 1));
                 u32x4 w[A + 1];
 #pragma unroll
-                for (int i = 0; i < A; i++) w[i] = (uint32_t)i < job.alpha ? cv[i] : u32x4{0, 0, 0, 0};
-                w[A] = cv[job.alpha];
+                for (int i = 0; i <= A; i++) w[i] = cv[i];
+                auto convert = [&](auto rounded) {
 #pragma unroll
-                for (int l = 0; l < U; l++) {
-                    ConvAcc acc{0, 0};
+                    for (int l = 0; l < U; l++) {
+                        ConvAcc acc{0, 0};
 #pragma unroll
-                    for (int i = 0; i < A; i++) conv_mac(acc, yl[i][l], yh[i][l], w[i]);
-                    if (job.rounded) {
-                        const uint32_t rl = (r[l / 8] >> (4 * (l % 8))) & 15;
-                        acc.H += (uint64_t)rl * w[A].x;
-                        acc.L += (uint64_t)rl * w[A].y;
+                        for (int i = 0; i < A; i++) conv_mac(acc, yl[i][l], yh[i][l], w[i]);
+                        if (decltype(rounded)::value) {
+                            const uint32_t rl = (r[l / 8] >> (4 * (l % 8))) & 15;
+                            acc.H += (uint64_t)rl * w[A].x;
+                            acc.L += (uint64_t)rl * w[A].y;
+                        }
+                        x[l] = conv_value(acc, kk.f);
                     }
-                    x[l] = conv_value(acc, kk.f);
-                }
+                };
+                if (job.rounded)
+                    convert(std::true_type{});
+                else
+                    convert(std::false_type{});
             }
             const auto col = table_ptr(tb.col + (size_t)prime * kNttCols);
             ct_unit<RA>(x, kk, [&](int e) -> u32x4 { return col[e + 1]; });
