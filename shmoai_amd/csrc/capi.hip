@@ -704,15 +704,29 @@ int shm_multiply_inplace(shm_context *ctx, shm_ciphertext *a, const shm_cipherte
         same_level(a->ct, b->ct);
         if (a->ct.size != 2 || b->ct.size != 2) throw InvalidArgument("multiply supports size-2 ciphertexts");
         Context &c = *ctx->c;
-        const size_t Ql = a->ct.Ql(), S3 = 3 * Ql * c.N;
+        const size_t Ql = a->ct.Ql();
         const hipStream_t s = S(st);
-        Scratch out(S3 * sizeof(uint64_t), s);
-        if (a == b)
-            launch_square(c, a->ct.data(), out.as<uint64_t>(), Ql, s);
+        // Every thread reads its words of both operands before it writes the three products at
+        // the same places: a buffer with room for three polynomials is written in place, any
+        // other is replaced by a new one. (Through scratch and back, 27 of 270 us at 22 limbs.)
+        DevBuf fresh;
+        const bool room = a->ct.cap_size >= 3;
+        if (room)
+            a->ct.buf.use_on(s);
         else
-            launch_tensor(c, a->ct.data(), b->ct.data(), out.as<uint64_t>(), Ql, s);
-        a->ct.resize(3, a->ct.chain, s);
-        launch_copy_words(a->ct.data(), out.as<uint64_t>(), S3, s);
+            fresh.alloc_async(3 * Ql * c.N * sizeof(uint64_t), s);
+        uint64_t *out = room ? a->ct.data() : fresh.as<uint64_t>();
+        if (a == b)
+            launch_square(c, a->ct.data(), out, Ql, s);
+        else
+            launch_tensor(c, a->ct.data(), b->ct.data(), out, Ql, s);
+        if (!room) {
+            a->ct.buf.use_on(s);
+            a->ct.buf = std::move(fresh);  // the old block returns to the pool after the products
+            a->ct.cap_size = 3;
+            a->ct.cap_limbs = Ql;
+        }
+        a->ct.size = 3;
         a->ct.scale = a->ct.scale * b->ct.scale;
     });
 }

@@ -1094,8 +1094,10 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
                 SHM_HIP(hipEventCreate(&pe[1]));
                 g_probe.ev_plain.push_back(pe[0]);
                 g_probe.ev_plain.push_back(pe[1]);
-                // the transform's algorithmic bytes: every limb read and written once
-                g_probe.bytes_plain += 16.0 * N * total_limbs;
+                // the transform's algorithmic bytes: every limb read and written once (not the
+                // digits' own limbs where they are neither)
+                const size_t own = IOB == IO_DIGITS && !io.copy_own ? n_polys / io.digits * (size_t)mp.Ql : 0;
+                g_probe.bytes_plain += 16.0 * N * (total_limbs - own);
             }
         }
         if (IOB == IO_RESCALE) {

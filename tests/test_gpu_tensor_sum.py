@@ -32,3 +32,28 @@ def test_tensor_sum_bitexact(oracle_lib, bits, cols):
                                           ctx, cols, 1, cols, 1, 0)
     exp = ref.ctct_matmul_colpacking(xs, ws, Ql, 1, 0, {}, ref.gen_relin_key(s_ref, 5))
     assert np.array_equal(out[0].numpy(), exp[0])
+
+
+@pytest.mark.parametrize("square", [False, True])
+def test_product_written_in_place_bitexact(oracle_lib, square):
+    """The first product replaces the two-polynomial buffer, the second (after relinearisation)
+    is written into the room for three."""
+    import shmoai_amd as shm
+    bits = [51, 46, 46, 51]
+    ctx = shm.Context(12, bits, 1)
+    ref = oracle_lib.Ref(12, bits, 1)
+    rng = np.random.default_rng(3)
+    sk = shm.SecretKey(ctx, seed=1, hamming_weight=64)
+    s_ref = ref.sk_ntt(ref.sample_ternary(1, 64))
+    rk, rkey = sk.gen_relinkey(seed=5), ref.gen_relin_key(s_ref, 5)
+    a, b = (np.stack([rng.integers(0, int(q), size=ref.N, dtype=np.uint64) for q in ref.primes[:3]] * 2).ravel()
+            for _ in range(2))
+    ev = shm.Evaluator(ctx)
+    ct, other = shm.Ciphertext(ctx, 2, ctx.chain(3)).load(a), shm.Ciphertext(ctx, 2, ctx.chain(3)).load(b)
+    for _ in range(2):
+        ev.multiply_inplace(ct, ct if square else other)
+        a = ref.tensor(a, a if square else b, 3)
+        assert np.array_equal(ct.numpy(), a)
+        ev.relinearize_inplace(ct, rk)
+        a = ref.relinearize(a, 3, rkey)
+        assert np.array_equal(ct.numpy(), a)
