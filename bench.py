@@ -20,7 +20,7 @@ over all 768 ciphertexts (96 chunks in one call), end to end (no extrapolation);
 the plain per-ciphertext form (768 sequential single-ciphertext calls, each waited for, the
 reference's loop), ordinary groups of 8, shared-a n = 4 and shared-a n = 8, with decryption
 errors on a sample of outputs. `roofline` is the dominant kernel of a
-shared-a chunk, whichever NTT tile pass takes more time per chunk (the plain forward pass
+shared-a chunk, whichever NTT row pass takes more time per chunk (the plain forward pass
 or the fused last pass with the ModDown combine and rescale; the other one is
 `roofline_other_kernel`), from HIP events around each of its launches in one eager chunk. `cpu_baseline` is the oracle's key-switch
 primitives at the same parameters, weighted by the key-switch work the GPU path counts per
@@ -60,13 +60,13 @@ REF_SHARED_A_N8_S = 193.3      # reference, 768 cts shared-a n = 8, RTX PRO 6000
 
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "contract_int8_192x192_N65536_L24_pmc.txt")
 BOOT_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "ntt_tile_passes_shared_a_n8_c3_pmc.txt")
-# the NTT tile passes as the profiles name them (lazy integer butterflies, 512-thread
-# blocks): the plain forward pass and the fused rescale / ModDown pass
-PLAIN_TILE_KERNEL = "k_ntt_blocks<12,true,0,true,512>"
-RESCALE_TILE_KERNEL = "k_ntt_blocks<12,true,2,true,512>"
-TILE_NOTE = ("12 stages of 64-bit integer Harvey butterflies through LDS per 4096-word tile (4 rounds of radix-8 "
-             "units; the two wave-uniform rounds read their twiddles through scalar loads); bound by VALU issue of "
-             "the 64-bit modular products, not by HBM (the same tile's load and store alone run near peak)")
+# the NTT's row passes as the profiles name them: the plain forward pass (the ModUp digits'
+# form) and the fused rescale / ModDown pass
+PLAIN_TILE_KERNEL = "k_ntt_rows<true,5,true,512>"
+RESCALE_TILE_KERNEL = "k_ntt_rows<true,2,true,512>"
+TILE_NOTE = ("last 9 stages, one wave per row of 512 words: butterflies by split products (6 multiply-adds), three "
+             "rounds of radix-8 units through the wave's LDS, no barriers; the column pass's intermediate is read "
+             "besides the algorithmic operands; bound by memory, with VALU issue next")
 
 
 def measured_traffic(kernel: str, path: str = TRAFFIC_PROFILE):
@@ -672,13 +672,13 @@ def main() -> int:
 
     fused = tile_roofline(pr, RESCALE_TILE_KERNEL, "fused last NTT pass: ModDown combine and rescale",
                           TILE_NOTE)
-    plain = tile_roofline(pp, PLAIN_TILE_KERNEL, "forward NTT tile pass: ModUp digits and other forward transforms",
+    plain = tile_roofline(pp, PLAIN_TILE_KERNEL, "forward NTT row pass: ModUp digits and other forward transforms",
                           TILE_NOTE)
     # the dominant kernel of the chunk (most time) is the roofline object
     roofline, roofline_other = (plain, fused) if pp["ms"] >= pr["ms"] else (fused, plain)
     avg_ms, gbs = fused["kernel_ms_avg"], fused["achieved"]
     log(f"bench: fused NTT pass {pr['launches']} launches, {avg_ms * 1e3:.1f} us avg, {gbs:.0f} GB/s algorithmic; "
-        f"plain forward tile pass {pp['launches']} launches, {plain['kernel_ms_avg'] * 1e3:.1f} us avg, "
+        f"plain forward row pass {pp['launches']} launches, {plain['kernel_ms_avg'] * 1e3:.1f} us avg, "
         f"{plain['achieved']:.0f} GB/s algorithmic")
 
     if not args.quick:

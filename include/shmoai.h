@@ -111,7 +111,7 @@ int shm_galois_elt_from_step(const shm_context *ctx, int step, uint32_t *elt);
 /* ---- raw limb transforms ------------------------------------------------------
  * Replace nwt_2d_radix8_forward_inplace / nwt_2d_radix8_backward_inplace
  * (fntt_2d.cu:620, intt_2d.cu:724): n_polys x n_limbs limbs, limb k uses prime
- * first_prime + k. `data` is a device pointer aligned to 16 bytes (the tile pass
+ * first_prime + k. `data` is a device pointer aligned to 16 bytes (the row pass
  * reads pairs of words; SHM_ERR_INVALID_ARGUMENT otherwise, before any launch). */
 int shm_ntt_forward(shm_context *ctx, uint64_t *data, uint32_t n_polys, uint32_t n_limbs, uint32_t first_prime,
                     shm_stream_t stream);
@@ -561,7 +561,7 @@ int shm_boot_graph_info(const shm_boot_graph *g, uint32_t *chunk, uint64_t *node
 int shm_boot_graph_destroy(shm_boot_graph *g);
 
 /* ---- measurement hooks (no counterpart in the reference, which times no kernel) -------
- * Probe of the fused last NTT pass (the tile pass that writes the ModDown combine
+ * Probe of the fused last NTT pass (the row pass that writes the ModDown combine
  * (cx - NTT(delta)) P^-1 and the rescale (acc - NTT(last)) q_last^-1): between begin and
  * end every eager launch is bracketed by timing events on its stream; end waits for
  * the device and returns the launch count, the summed kernel milliseconds and the
@@ -569,7 +569,7 @@ int shm_boot_graph_destroy(shm_boot_graph *g);
  * combined operand read, plus the output read where it accumulates). */
 int shm_probe_fused_ntt_begin(void);
 int shm_probe_fused_ntt_end(uint64_t *launches, double *ms, double *bytes);
-/* The plain forward NTT tile passes (the ModUp digits' and other forward transforms' last
+/* The plain forward NTT row passes (the ModUp digits' and other forward transforms' last
  * pass) timed in the same window, with 16 N algorithmic bytes per limb (each limb read and
  * written once); valid after shm_probe_fused_ntt_end. */
 int shm_probe_plain_ntt_last(uint64_t *launches, double *ms, double *bytes);

@@ -840,7 +840,7 @@ def probe_fused_ntt_end() -> dict:
 
 
 def probe_plain_ntt_last() -> dict:
-    """The plain forward NTT tile passes of the last probe window: launches, ms, bytes."""
+    """The plain forward NTT row passes of the last probe window: launches, ms, bytes."""
     n, ms, by = C.c_uint64(), C.c_double(), C.c_double()
     check(_lib().shm_probe_plain_ntt_last(C.byref(n), C.byref(ms), C.byref(by)))
     return {"launches": n.value, "ms": ms.value, "bytes": by.value}

@@ -265,7 +265,7 @@ void ntt_forward(const Context &c, uint64_t *data, size_t n_polys, size_t n_limb
 // bit-reversed order (tw[m + i] belongs to group i of the stage with m groups).
 constexpr int kNttCols = 256;  // column entries kept per prime (N / 512 are used)
 void ntt_make_tables(const Context &c, const uint64_t *tw, DevBuf &col, DevBuf &row);
-// Events recorded around the tile pass of every fused-rescale NTT launched while
+// Events recorded around the row pass of every fused-rescale NTT launched while
 // set (nullptr to stop); used to time the matmul's rescale.
 void set_rescale_tile_events(hipEvent_t start, hipEvent_t stop);
 // Timing probe of the fused last NTT pass (ModDown combine and rescale) over eager
@@ -273,7 +273,7 @@ void set_rescale_tile_events(hipEvent_t start, hipEvent_t stop);
 // launch count, the summed kernel time and the algorithmic bytes of those launches.
 void probe_fused_ntt_begin();
 void probe_fused_ntt_end(size_t *launches, double *ms, double *bytes);
-// The same window's plain forward tile passes (the ModUp digits' and other forward
+// The same window's plain forward row passes (the ModUp digits' and other forward
 // NTTs' last pass), with 16 N algorithmic bytes per limb; valid after probe_fused_ntt_end.
 void probe_plain_ntt_last(size_t *launches, double *ms, double *bytes);
 // Key-switch work counters, per level Ql (index < 128): polynomials ModUp'd,

@@ -971,10 +971,10 @@ __global__ __launch_bounds__(256, 3) void k_rows_mac(MacJob job, NttTables tb, i
     }
 }
 
-// optional events around the tile pass of the fused rescale (timing of one launch)
+// optional events around the row pass of the fused rescale (timing of one launch)
 hipEvent_t g_rescale_tile_ev[2] = {nullptr, nullptr};
 
-// Probe of the fused last pass (IO_RESCALE tile pass of forward NTTs: the ModDown
+// Probe of the fused last pass (IO_RESCALE row pass of forward NTTs: the ModDown
 // combine and the rescale): while on, every eager launch is bracketed by a pair of
 // timing events and its algorithmic bytes are recorded.
 struct FusedProbe {
@@ -982,7 +982,7 @@ struct FusedProbe {
     bool on = false;
     std::vector<hipEvent_t> ev;  // start, stop per launch of the fused last pass
     double bytes = 0.0;
-    std::vector<hipEvent_t> ev_plain;  // the same for the plain forward tile pass
+    std::vector<hipEvent_t> ev_plain;  // the same for the plain forward row pass
     double bytes_plain = 0.0;
     size_t last_plain_launches = 0;
     double last_plain_ms = 0.0, last_plain_bytes = 0.0;
