@@ -365,7 +365,8 @@ void ntt_rows_digits(const Context &c, uint64_t *d, size_t Ql, size_t beta, size
 // (primes of positions among QlP limbs), at out + (2 e + o) out_stride.
 //   key != null: operands are key rows (term stride 2 op_stride, output stride op_stride, by
 //     prime); the group's own limbs of digit t come from op.p[e]; with add_on, P add.p[2 e + o]
-//     is added on the data limbs.
+//     is added on the data limbs. With perm, own limbs and addends are read through that
+//     NTT-domain permutation, and only output 0 has an addend.
 //   else: operand (t, o) is op.p[t] + o op_stride, by limb; with accumulate, onto the output.
 struct MacJob {
     const uint64_t *data;
@@ -377,7 +378,7 @@ struct MacJob {
     uint64_t *out;
     size_t out_stride;
     bool accumulate, add_on;
-    const uint32_t *own_perm;  // own limbs are read through this NTT-domain permutation, unless null
+    const uint32_t *perm;
     PolyPack add;
     const uint64_t *pmod, *pmod_s;
 };
@@ -528,15 +529,15 @@ void ks_inner_batch(const Context &c, const uint64_t *d, size_t m, size_t Ql, co
 // exact centred conversion over {q_last, P} in place of ModDown then rescale.
 void keyswitch_rescale_batch(const Context &c, const PolyPack &c2, const PolyPack &d01, size_t m, const uint64_t *key,
                              size_t Ql, const PolyPack &out, hipStream_t s);
+// Key switch of sigma(a_k) for m size-2 ciphertexts (a_k, b_k given unpermuted, sigma the
+// NTT-domain permutation `perm`) into out.p[2k], out.p[2k + 1] = (sigma(b_k) + ks_0, ks_1), no
+// permuted copy written. Outputs may be the buffers of any a and b themselves. Returns false,
+// with nothing done, where the fused key switch does not apply.
+bool keyswitch_galois(const Context &c, const PolyPack &a, const PolyPack &b, size_t m, const uint64_t *key, size_t Ql,
+                      const PolyPack &out, const uint32_t *perm, hipStream_t s);
 // Key switch of m polynomials c2.p[i] with one key; the switched pair of member
 // i goes to (ct01.p[2i], ct01.p[2i + 1]), accumulated where acc_mask has the
 // polynomial's bit. One launch per stage for the whole group.
-// Key switch of sigma(a_k) for m size-2 ciphertexts (a_k, b_k given unpermuted, sigma the
-// NTT-domain permutation `perm`) into out.p[2k], out.p[2k + 1] = (sigma(b_k) + ks_0, ks_1), no
-// permuted copy written; outputs must not overlap a or b. Returns false, with nothing done,
-// where the fused key switch does not apply.
-bool keyswitch_galois(const Context &c, const PolyPack &a, const PolyPack &b, size_t m, const uint64_t *key, size_t Ql,
-                      const PolyPack &out, const uint32_t *perm, hipStream_t s);
 void keyswitch_batch(const Context &c, const PolyPack &c2, size_t m, const uint64_t *key, size_t Ql,
                      const PolyPack &ct01, uint64_t acc_mask, hipStream_t s, bool rounded = false);
 

@@ -913,11 +913,11 @@ __global__ __launch_bounds__(256, 3) void k_rows_mac(MacJob job, NttTables tb, i
                 a[o][j] = *global_ptr(reinterpret_cast<const u64x2 *>(op + o * job.op_stride + pair_of(j)));
         u64x2 y[4];
         if (own(t)) {
-            if (job.own_perm) {
+            if (job.perm) {
                 const auto p = global_ptr(job.op.p[e] + (size_t)limb * N);
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const auto i = global_ptr(job.own_perm + row0 + pair_of(j));
+                    const auto i = global_ptr(job.perm + row0 + pair_of(j));
                     y[j] = u64x2{p[i[0]], p[i[1]]};
                 }
             } else {
@@ -952,8 +952,8 @@ __global__ __launch_bounds__(256, 3) void k_rows_mac(MacJob job, NttTables tb, i
 #pragma unroll
     for (int o = 0; o < 2; o++) {
         uint64_t *out = job.out + (size_t)(2 * e + o) * job.out_stride + at;
-        const bool add_on = KEY && job.add_on && limb < job.Ql;
-        const uint64_t *add = add_on ? job.add.p[2 * e + o] + at : nullptr;
+        const bool add_on = KEY && job.add_on && limb < job.Ql && (o == 0 || !job.perm);
+        const uint64_t *add = add_on ? job.add.p[2 * e + o] + (size_t)limb * N : nullptr;
         const uint64_t pm = add_on ? job.pmod[limb] : 0, pms = add_on ? job.pmod_s[limb] : 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -963,7 +963,13 @@ __global__ __launch_bounds__(256, 3) void k_rows_mac(MacJob job, NttTables tb, i
                 const u64x2 c = *at2;
                 v = u64x2{add_mod(v.x, c.x, m.q), add_mod(v.y, c.y, m.q)};
             } else if (add_on) {
-                const u64x2 c = *global_ptr(reinterpret_cast<const u64x2 *>(add + pair_of(j)));
+                u64x2 c;
+                if (job.perm) {
+                    const auto i = global_ptr(job.perm + row0 + pair_of(j));
+                    c = u64x2{global_ptr(add)[i[0]], global_ptr(add)[i[1]]};
+                } else {
+                    c = *global_ptr(reinterpret_cast<const u64x2 *>(add + row0 + pair_of(j)));
+                }
                 v = u64x2{add_mod(v.x, mul_shoup(c.x, pm, pms, m.q), m.q), add_mod(v.y, mul_shoup(c.y, pm, pms, m.q), m.q)};
             }
             __builtin_nontemporal_store(v, at2);

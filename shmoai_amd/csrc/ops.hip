@@ -91,23 +91,13 @@ void apply_galois(Context &c, Ciphertext &ct, uint32_t elt, const GaloisKeys &gk
         ct = std::move(o);
         return;
     }
-    {
-        // both parts are read through the permutation where the key switch runs fused
-        Ciphertext o;
-        o.ctx = &c;
-        o.resize(2, ct.chain, s, false);  // the fused ModDown writes every word
-        o.scale = ct.scale;
-        o.ntt = true;
-        PolyPack a{}, b{}, op{};
-        a.p[0] = ct.poly(1);
-        b.p[0] = ct.poly(0);
-        op.p[0] = o.poly(0);
-        op.p[1] = o.poly(1);
-        if (keyswitch_galois(c, a, b, 1, it->second->k.as<uint64_t>(), Ql, op, table, s)) {
-            ct = std::move(o);
-            return;
-        }
-    }
+    // In the caller's buffer: its address and capacity stay, and a recorded rotation neither
+    // allocates its result nor gives the block back. Both parts are read through the
+    // permutation where the key switch runs fused.
+    PolyPack a{}, b{}, op{};
+    a.p[0] = op.p[1] = ct.poly(1);
+    b.p[0] = op.p[0] = ct.poly(0);
+    if (keyswitch_galois(c, a, b, 1, it->second->k.as<uint64_t>(), Ql, op, table, s)) return;
     Scratch t0(Ql * N * sizeof(uint64_t), s), t1(Ql * N * sizeof(uint64_t), s);
     launch_permute(c, ct.poly(0), t0.as<uint64_t>(), table, Ql, s);
     launch_permute(c, ct.poly(1), t1.as<uint64_t>(), table, Ql, s);
