@@ -412,7 +412,11 @@ void ctpt_matmul_int8(const Context &c, const std::vector<const Ciphertext *> &X
     };
     Scratch dW(row_w * col_w * sizeof(double), s);
     Scratch dscale(row_w * sizeof(double), s);
-    Scratch frag(frag_count((int)((kc_max + 63) / 64)) * sizeof(i8x16), s);
+    // The chunks hold kc_max or row_w / nch rows, and fewer rows can take more fragments: their
+    // phases stage more row blocks, so the last one pads further (257 rows of 6 digits: 129
+    // rows 36 KB, 128 rows 48 KB).
+    const size_t frag_cap = std::max(frag_count((int)((kc_max + 63) / 64)), frag_count((int)((row_w / nch + 63) / 64)));
+    Scratch frag(frag_cap * sizeof(i8x16), s);
     Scratch corr(Ql * col_w * sizeof(uint64_t), s);
     Scratch mu(Ql * sizeof(uint64_t), s);
     Scratch fc(2 * Ql * sizeof(u32x4), s);
@@ -431,6 +435,7 @@ void ctpt_matmul_int8(const Context &c, const std::vector<const Ciphertext *> &X
         const size_t kc = row_w / nch + (ch < row_w % nch ? 1 : 0);
         const int KS = (int)((kc + 63) / 64), RB = rb_for(KS, DW);
         const size_t nfrag = frag_count(KS);
+        if (nfrag > frag_cap) throw LogicError("weight fragments beyond their workspace");
         const double *Wc = dW.as<double>() + k0 * col_w;
         const double *sc = dscale.as<double>() + k0;
         k_weight_frags<<<grid_for(nfrag), kBlock, 0, s>>>(Wc, sc, frag.as<i8x16>(), kc, col_w, DW, MB, KS, RB);
