@@ -63,8 +63,11 @@ class DevBuf {
         o.ptr_ = nullptr;
         o.bytes_ = 0;
     }
-    DevBuf &operator=(DevBuf &&o) noexcept {
+    // The new words were made from the old ones on o's stream: the old block goes back behind
+    // that work, not on the stream that owned it before.
+    DevBuf &operator=(DevBuf &&o) {
         if (this != &o) {
+            if (o.ptr_ && o.async_) use_on(o.s_);
             release();
             ptr_ = o.ptr_;
             bytes_ = o.bytes_;
