@@ -1,7 +1,8 @@
-"""Key switching over every form of the base conversions, bit-exact against the oracle: 1 to 6
+"""Key switching over the forms of the base conversions, bit-exact against the oracle: 1 to 5
 source limbs fused into the NTT's column stages at every ring degree (column stages of one
 and of two rounds), a last digit shorter than the others, and chains outside the fused form
-(60-bit primes, more than 5 special primes)."""
+(60-bit primes, more than 5 special primes). Conversions of 6 source limbs come from ModDown
+merged with the rescale (test_gpu_merged_rescale.py)."""
 import numpy as np
 import pytest
 
