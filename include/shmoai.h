@@ -584,7 +584,7 @@ int shm_keyswitch_counters_reset(void);
  * ct-pt matmul's contraction and rescale one after the other, or overlaps the contraction
  * (row_W <= 256, in limb windows) with the rescale on a second stream of the context;
  * "ntt_tile_threads" (512, the default, or 256) runs the NTT row pass in blocks of 512 or
- * 256 threads (the same words).
+ * 256 threads (the same words; launches with a prime not just below a power of two take 256).
  * Process-wide. */
 int shm_set_tuning(const char *name, int32_t value);
 int shm_get_tuning(const char *name, int32_t *value);

@@ -294,7 +294,8 @@ struct KsTuning {
     // both kernels fill the GPU, and the overlapped form measured 7% slower)
     int matmul_overlap = 0;
     // threads per block of the NTT row pass, 512 or 256 (one wave per row either way; the
-    // same words and, within 2%, the same times)
+    // same words and, within 2%, the same times); launches with a prime that has no split form
+    // take 256
     int ntt_tile_threads = 512;
 };
 KsTuning &ks_tuning();

@@ -720,12 +720,16 @@ __device__ __forceinline__ void row_pass(const K &k, uint64_t *lds, uint64_t *ba
 // once (round 3 into registers, rounds 1 and 2 into LDS), and the next polynomial's words are
 // requested before the current one's stages. 118 VGPRs, 4 waves per SIMD: the prefetch and
 // the shared twiddles (a row's twiddles are twice its data) gave more than 8 waves did.
+// GENERAL launches hold both kinds of arithmetic and run 3 waves per SIMD, in blocks of 256
+// threads, three of which fill it: held to 4 waves they spilled 36 to 80 registers (64 x 9 limbs
+// of 50 and 60 bits at N = 2^16, forward 415 -> 269 us, inverse 333 -> 266; at N = 2^13 63 -> 38
+// and 67 -> 39), and blocks of 512 leave only 2 waves (283, 275, 43 and 44).
 // Work order: workgroups are dispatched to the 8 XCDs round-robin, so block
 // b runs on XCD b % 8. Each XCD takes a contiguous range of blocks' row indices
 // O = (limb * rows + row) * chunks + chunk: the polynomials that share one prime and row
 // (hence one run of twiddles) run back to back on the same L2.
 template <bool FWD, int IO, bool FAST, int NT>
-__global__ __launch_bounds__(NT, 4) void k_ntt_rows(uint64_t *__restrict__ data, LimbMap mp, NttTables tb, int logN,
+__global__ __launch_bounds__(NT, FAST ? 4 : 3) void k_ntt_rows(uint64_t *__restrict__ data, LimbMap mp, NttTables tb, int logN,
                                                  NttIO io, uint32_t n_polys, uint32_t per_xcd, uint32_t chunk) {
     __shared__ uint64_t lds[NT / 64][kRowLds];
     const size_t N = size_t(1) << logN;
@@ -1044,7 +1048,7 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
             aligned = aligned && (((uintptr_t)io.out_p.p[p] | (io.packed ? (uintptr_t)io.acc_p.p[p] : 0)) & 15) == 0;
     }
     if (!aligned) throw InvalidArgument("NTT operands must be 16-byte aligned");
-    const int row_threads = ks_tuning().ntt_tile_threads;
+    const int row_threads = fast ? ks_tuning().ntt_tile_threads : 256;
     // up to 4 polynomials per wave share a row's twiddles in registers and prefetch each
     // other's words, while 8192 waves (8 per SIMD) remain: the plain forward pass of a
     // shared-a chunk's launches 96 -> 75 us (8 polynomials measured the same)
@@ -1081,8 +1085,6 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
             SHM_ROWS(true, 512);
         else if (fast)
             SHM_ROWS(true, 256);
-        else if (row_threads == 512)
-            SHM_ROWS(false, 512);
         else
             SHM_ROWS(false, 256);
 #undef SHM_ROWS
