@@ -1059,14 +1059,15 @@ void launch_ntt(const Context &c, uint64_t *data, const LimbMap &mp, size_t tota
     const size_t row_waves = (size_t)((n_polys + chunk - 1) / chunk) * mp.n_active * (N / kRow);
     const uint32_t per_xcd = (uint32_t)((row_waves + row_threads / 64 * 8 - 1) / (row_threads / 64 * 8));
     auto cols = [&]() {
-#define SHM_COLS(S, RA, RB)                                                                            \
-    case S: {                                                                                          \
-        const unsigned grid = (unsigned)(total_limbs * (kRow / col_width(RA, RB)));                    \
-        if (fast)                                                                                      \
-            k_ntt_cols<RA, RB, FWD, IOA, true><<<grid, kThreads, 0, s>>>(data, mp, tb, logN, io);      \
-        else                                                                                           \
-            k_ntt_cols<RA, RB, FWD, IOA, false><<<grid, kThreads, 0, s>>>(data, mp, tb, logN, io);     \
-        break;                                                                                         \
+#define SHM_COLS(S, RA, RB)                                                                                 \
+    case S: {                                                                                               \
+        const size_t grid = total_limbs * (kRow / col_width(RA, RB));                                       \
+        if (grid * kThreads >> 32) throw LogicError("NTT beyond the threads of one launch");                \
+        if (fast)                                                                                           \
+            k_ntt_cols<RA, RB, FWD, IOA, true><<<(unsigned)grid, kThreads, 0, s>>>(data, mp, tb, logN, io); \
+        else                                                                                                \
+            k_ntt_cols<RA, RB, FWD, IOA, false><<<(unsigned)grid, kThreads, 0, s>>>(data, mp, tb, logN, io);\
+        break;                                                                                              \
     }
         switch (stages) {
             SHM_COLS(3, 3, 0)
@@ -1173,11 +1174,23 @@ void ntt_make_tables(const Context &c, const uint64_t *tw, DevBuf &col, DevBuf &
     SHM_HIP(hipGetLastError());
 }
 
-void ntt_forward(const Context &c, uint64_t *data, size_t n_polys, size_t n_limbs, size_t first_prime,
-                 hipStream_t s) {
+// Any number of polynomials, in launches of up to 2^33 words (64 GB): the column pass has a
+// thread per 4 words of a ring of 2^13 and per 8 of the others, and of 2^32 threads and more a
+// launch runs the remainder modulo 2^32, with no error.
+template <bool FWD>
+static void ntt_polys(const Context &c, uint64_t *data, size_t n_polys, size_t n_limbs, size_t first_prime,
+                      hipStream_t s) {
+    if (n_limbs == 0) return;
     LimbMap mp{(uint32_t)n_limbs, 0, 0xffffffffu, 0, 0xffffffffu, (uint32_t)c.nQ, (uint32_t)first_prime,
                (uint64_t)n_limbs * c.N};
-    launch_ntt<true, IO_PLAIN, IO_PLAIN>(c, data, mp, n_polys * n_limbs, s);
+    const size_t step = std::max<size_t>(1, (size_t(1) << 33) / (n_limbs * c.N));
+    for (size_t p = 0; p < n_polys; p += step)
+        launch_ntt<FWD, IO_PLAIN, IO_PLAIN>(c, data + p * n_limbs * c.N, mp, std::min(step, n_polys - p) * n_limbs, s);
+}
+
+void ntt_forward(const Context &c, uint64_t *data, size_t n_polys, size_t n_limbs, size_t first_prime,
+                 hipStream_t s) {
+    ntt_polys<true>(c, data, n_polys, n_limbs, first_prime, s);
 }
 
 void probe_fused_ntt_begin() {
@@ -1273,9 +1286,7 @@ void rows_mac(const Context &c, const MacJob &job, hipStream_t s) {
 
 void ntt_inverse(const Context &c, uint64_t *data, size_t n_polys, size_t n_limbs, size_t first_prime,
                  hipStream_t s) {
-    LimbMap mp{(uint32_t)n_limbs, 0, 0xffffffffu, 0, 0xffffffffu, (uint32_t)c.nQ, (uint32_t)first_prime,
-               (uint64_t)n_limbs * c.N};
-    launch_ntt<false, IO_PLAIN, IO_PLAIN>(c, data, mp, n_polys * n_limbs, s);
+    ntt_polys<false>(c, data, n_polys, n_limbs, first_prime, s);
 }
 
 void ntt_inverse_gather(const Context &c, const PolyPack &in, uint64_t *out, size_t n_polys, size_t n_limbs,
