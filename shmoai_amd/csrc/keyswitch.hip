@@ -50,12 +50,13 @@ constexpr int kMaxAlpha = 16;
 // The base conversions unroll their sums over the digit's (or the special primes')
 // limbs to a compile-time bound A >= that count, so the common sizes (5 special primes
 // at the bootstrapping parameters, 1 for the matmul's chain) carry no tests for absent
-// terms: A is 1, 2, 4, 5, 8 or 16.
-template <typename F>
+// terms: A is LO (1 or 2), 2, 4, 5, 8 or 16. With one special prime ModUp and ModDown convert
+// in the column stages (convert_covers), so they start at 2; the merged rescale starts at 1.
+template <int LO, typename F>
 void with_alpha_bound(size_t alpha, F &&f) {
-    if (alpha <= 1)
-        f(std::integral_constant<int, 1>{});
-    else if (alpha <= 2)
+    if constexpr (LO <= 1)
+        if (alpha <= 1) return f(std::integral_constant<int, 1>{});
+    if (alpha <= 2)
         f(std::integral_constant<int, 2>{});
     else if (alpha <= 4)
         f(std::integral_constant<int, 4>{});
@@ -238,7 +239,8 @@ __global__ __launch_bounds__(256) void k_ks_inner_multi(const uint64_t *__restri
 // delta[p][i][j] = fastbconv of the coefficient-form P limbs of polynomial p to
 // q_i, one thread per (p, j). With `rounded`, the conversion is exact and
 // centred: it subtracts round(sum_j y_j / p_j) P, so delta is the representative
-// of cx mod P in (-P/2, P/2] and (cx - delta) / P rounds to nearest.
+// of cx mod P in (-P/2, P/2] and (cx - delta) / P rounds to nearest. Two special primes and
+// more: one converts in the column stages (convert_covers).
 template <bool P52, int A>
 __global__ void k_moddown_bconv(const uint64_t *__restrict__ cx, uint64_t *__restrict__ delta,
                                 const DevMod *__restrict__ mods, const uint64_t *__restrict__ phat_inv,
@@ -257,7 +259,7 @@ __global__ void k_moddown_bconv(const uint64_t *__restrict__ cx, uint64_t *__res
             y[jj] = 0;
             if ((size_t)jj < nP) {
                 const uint64_t pj = mods[nQ + jj].q;
-                y[jj] = nP == 1 ? cxP[0] : mul_shoup(cxP[jj * N], phat_inv[jj], phat_inv_s[jj], pj);
+                y[jj] = mul_shoup(cxP[jj * N], phat_inv[jj], phat_inv_s[jj], pj);
                 if (rounded) v = __dadd_rn(v, __ddiv_rn((double)y[jj], (double)pj));
             }
         }
@@ -268,7 +270,7 @@ __global__ void k_moddown_bconv(const uint64_t *__restrict__ cx, uint64_t *__res
         for (size_t i = 0; i < Ql; i++) {
             const DevMod mq = mods[i];
             uint64_t val;
-            if (P52 && nP > 1) {
+            if (P52) {
                 Acc52 acc{0, 0, 0};
                 if (nP == (size_t)A) {
 #pragma unroll
@@ -280,9 +282,6 @@ __global__ void k_moddown_bconv(const uint64_t *__restrict__ cx, uint64_t *__res
                 }
                 if (rounded) mac52(acc, split26(mq.q - r), pmod[i]);
                 val = reduce52(acc, mq);
-            } else if (nP == 1) {
-                val = reduce64(y[0], mq);
-                if (r) val = sub_mod(val, reduce64(mods[nQ].q, mq), mq.q);
             } else {
                 Acc128 acc{0, 0};
 #pragma unroll
@@ -730,7 +729,7 @@ void ks_modup(const Context &c, const uint64_t *c2, size_t Ql, uint64_t *d, hipS
     in.p[0] = const_cast<uint64_t *>(c2);  // read only
     ntt_inverse_gather(c, in, tcoef.as<uint64_t>(), 1, Ql, 0, s);
     if (alpha > (size_t)kMaxAlpha) throw InvalidArgument("at most 16 special primes");
-    with_alpha_bound(alpha, [&](auto bound) {
+    with_alpha_bound<2>(alpha, [&](auto bound) {
         constexpr int A = decltype(bound)::value;
         (c.primes52 ? k_modup_bconv<true, A> : k_modup_bconv<false, A>)<<<grid_for(beta * N), kBlock, 0, s>>>(
             tcoef.as<uint64_t>(), d, c.mods(), L.hat_inv.as<uint64_t>(), L.hat_inv_s.as<uint64_t>(),
@@ -820,7 +819,7 @@ void ks_moddown_pack(const Context &c, uint64_t *cx, size_t npolys, size_t Ql, c
     }
     ntt_inverse_qlp(c, cx, Ql, Ql, QlP, npolys, QlP * N, s);
     if (nP > (size_t)kMaxAlpha) throw InvalidArgument("at most 16 special primes");
-    with_alpha_bound(nP, [&](auto bound) {
+    with_alpha_bound<2>(nP, [&](auto bound) {
         constexpr int A = decltype(bound)::value;
         (c.primes52 ? k_moddown_bconv<true, A> : k_moddown_bconv<false, A>)<<<grid_for(npolys * N), kBlock, 0, s>>>(
             cx, delta.as<uint64_t>(), c.mods(), c.phat_inv.as<uint64_t>(), c.phat_inv_s.as<uint64_t>(),
@@ -878,7 +877,7 @@ void ks_modup_batch(const Context &c, const PolyPack &c2, size_t m, size_t Ql, u
     // fill the GPU, so the own limbs are written in coefficient form and one launch
     // transforms every limb (back to c2's words for the own ones).
     const bool per_digit = m >= 4;
-    with_alpha_bound(alpha, [&](auto bound) {
+    with_alpha_bound<2>(alpha, [&](auto bound) {
         constexpr int A = decltype(bound)::value;
         (c.primes52 ? k_modup_bconv<true, A> : k_modup_bconv<false, A>)<<<grid_for(m * beta * N), kBlock, 0, s>>>(
             tcoef.as<uint64_t>(), d, c.mods(), L.hat_inv.as<uint64_t>(), L.hat_inv_s.as<uint64_t>(),
@@ -1022,7 +1021,7 @@ void keyswitch_rescale_batch(const Context &c, const PolyPack &c2, const PolyPac
         return;
     }
     ntt_inverse_qlp(c, cx.as<uint64_t>(), Ql, Ql - 1, QlP, 2 * m, QlP * N, s);
-    with_alpha_bound(nP, [&](auto bound) {
+    with_alpha_bound<1>(nP, [&](auto bound) {
         constexpr int A = decltype(bound)::value;
         (c.primes52 ? k_moddown_rescale_bconv<true, A>
                     : k_moddown_rescale_bconv<false, A>)<<<grid_for(2 * m * N), kBlock, 0, s>>>(
