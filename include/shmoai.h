@@ -269,7 +269,8 @@ int shm_rescale_to_next_inplace_noalloc(shm_context *ctx, shm_ciphertext *ct, sh
 int shm_mod_switch_to_next_inplace(shm_context *ctx, shm_ciphertext *ct, shm_stream_t stream);
 int shm_mod_switch_to_inplace(shm_context *ctx, shm_ciphertext *ct, uint32_t chain_index, shm_stream_t stream);
 int shm_plain_mod_switch_to_inplace(shm_context *ctx, shm_plaintext *pt, uint32_t chain_index, shm_stream_t stream);
-/* evaluate.cu:1586-1647 apply_galois_inplace */
+/* evaluate.cu:1586-1647 apply_galois_inplace. Rotations and the conjugation write into the
+ * ciphertext's own buffer: its address (shm_ciphertext_data) and its room stay. */
 int shm_apply_galois_inplace(shm_context *ctx, shm_ciphertext *ct, uint32_t galois_elt, const shm_galois_keys *gk,
                              shm_stream_t stream);
 /* evaluate.cu:1650-1715 rotate_vector_inplace (NAF split when a key is missing) */

@@ -319,14 +319,14 @@ void ntt_forward_qlp(const Context &c, uint64_t *data, size_t Ql, size_t lo, siz
 void ntt_inverse_qlp(const Context &c, uint64_t *data, size_t Ql, size_t lo, size_t hi, size_t n_polys,
                      size_t poly_stride, hipStream_t s);
 
-// Rescale tail fused into one forward NTT: limb k (< L1) of polynomial p is
-// NTT([last_p]_{q_k}); the block pass stores (acc[p][k] - that) * qinv_k to
-// outs[p / ppo] (or out_single) at ((p % ppo) * L1 + k) * N.
-// rounded: divide with rounding to nearest (centred last limb) instead of the floor.
 // rescale_ntt_fused over output limbs lo .. lo + n - 1 of L1 only (outputs keep L1 limbs per polynomial)
 void rescale_ntt_fused_window(const Context &c, const uint64_t *last, const uint64_t *acc, size_t acc_limbs,
                               uint64_t *delta, uint64_t *const *outs, size_t ppo, size_t n_polys, size_t L1,
                               size_t lo, size_t n, const uint64_t *qinv, const uint64_t *qinv_s, hipStream_t s);
+// Rescale tail fused into one forward NTT: limb k (< L1) of polynomial p is
+// NTT([last_p]_{q_k}); the row pass stores (acc[p][k] - that) * qinv_k to
+// outs[p / ppo] (or out_single) at ((p % ppo) * L1 + k) * N.
+// rounded: divide with rounding to nearest (centred last limb) instead of the floor.
 void rescale_ntt_fused(const Context &c, const uint64_t *last, const uint64_t *acc, size_t acc_limbs,
                        uint64_t *delta, uint64_t *const *outs, uint64_t *out_single, size_t ppo, size_t n_polys,
                        size_t L1, const uint64_t *qinv, const uint64_t *qinv_s, hipStream_t s, bool rounded = false);
@@ -344,7 +344,7 @@ struct PolyPack {
 // (prime of position k among QlP limbs) of polynomial m digits + g, at out + that out_stride
 // + k N, gets the column stages of sum_i y_i conv[g][k][i] (minus round(sum_i y_i / q_i) D_g
 // when rounded). With skip_own, the limbs of the digit itself are left out. The row stages
-// follow (ntt_rows_digits, moddown_rows_fused).
+// follow (ntt_rows_digits, rows_mac, moddown_ntt_fused with columns_done).
 struct ConvertJob {
     const uint64_t *src;
     size_t src_stride;
@@ -431,11 +431,11 @@ void launch_tensor(const Context &c, const uint64_t *a, const uint64_t *b, uint6
                    size_t a_limbs = 0, size_t b_limbs = 0, bool accumulate = false);
 void launch_square(const Context &c, const uint64_t *a, uint64_t *out3, size_t Ql, hipStream_t s,
                    size_t a_limbs = 0);
-// (d0, d1, d2) = 2 (a (x) b) - cval (t0, t1, 0), the Chebyshev step T_k = 2 T_a T_b - T_(a-b)
-// before relinearisation (b == a squares; t may be null); operands through their first Ql limbs
 // out3 = sum_i a_i (x) b_i over size-2 operands (sums of up to 15 products per launch)
 void launch_tensor_sum(const Context &c, const std::vector<const uint64_t *> &a, const std::vector<const uint64_t *> &b,
                        uint64_t *out3, size_t Ql, size_t a_limbs, size_t b_limbs, hipStream_t s);
+// (d0, d1, d2) = 2 (a (x) b) - cval (t0, t1, 0), the Chebyshev step T_k = 2 T_a T_b - T_(a-b)
+// before relinearisation (b == a squares; t may be null); operands through their first Ql limbs
 void launch_tensor_cheb(const Context &c, const uint64_t *a, const uint64_t *b, const uint64_t *t, uint64_t cval,
                         uint64_t *out3, size_t Ql, hipStream_t s, size_t a_limbs, size_t b_limbs, size_t t_limbs);
 void launch_rescale(const Context &c, const uint64_t *in, uint64_t *out, size_t Ql, size_t npolys, hipStream_t s,
@@ -515,9 +515,9 @@ void ks_moddown(const Context &c, uint64_t *cx, size_t npolys, size_t Ql, uint64
 void ks_moddown_pack(const Context &c, uint64_t *cx, size_t npolys, size_t Ql, const PolyPack &out,
                      uint64_t acc_mask, hipStream_t s, bool rounded = false, const PolyPack *add_src = nullptr,
                      const uint32_t *perm = nullptr);
-// ModUp of m polynomials c2.p[i] (Ql limbs, NTT) into d [m][beta][QlP][N]; from 4
-// members on the digits' own limbs are not written (they are c2's limbs: pass c2
-// as `own` to ks_inner_batch, which reads them from there in every case)
+// ModUp of m polynomials c2.p[i] (Ql limbs, NTT) into d [m][beta][QlP][N]. The digits' own
+// limbs are c2's and need not be written (the fused form never writes them, the separate
+// kernels below 4 members only): pass c2 as `own` to ks_inner_batch, which reads them from there
 void ks_modup_batch(const Context &c, const PolyPack &c2, size_t m, size_t Ql, uint64_t *d, hipStream_t s,
                     bool rounded = false);
 // cx [m][2][QlP][N] = inner products of the m digit sets of d with one key

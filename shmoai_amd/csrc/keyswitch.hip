@@ -629,8 +629,12 @@ void ks_counters_reset() {
 }
 
 // Rows (of 512 words, over limbs and members) from which the row stages and the products run
-// fused, one wave each for all digits: 2 waves per SIMD. Below, the digits' rows run side by
-// side in the separate kernels instead of one after the other in too few waves.
+// fused, one wave each for all digits. With few rows the digits' rows had better run side by side
+// in the separate kernels than one after the other in too few waves. Rotations of one member,
+// apart and fused in us: 16 digits of one prime 224 / 148 at 2048 rows, 134 / 102 at 1408, 78 /
+// 71 at 640, 63 / 64 at 288 and 67 / 75 at 272; digits of 5 primes 120 / 98 at 2048, 84 / 76 at
+// 1024, 70 / 64 at 640. The line is safe rather than tight: set for 2 waves per SIMD, where the
+// products now run 3, it leaves 600 to 2048 rows to the separate kernels.
 constexpr size_t kFusedRows = 2048;
 
 // ModUp of m members with the conversion fused into the NTT's column stages: the inverse
